@@ -106,18 +106,21 @@ def draw(rng):
 # Inputs
 # ---------------------------------------------------------------------------
 def _positions(N, rho, g, jitter, whole_cells=False):
-    """N positions at density rho: sites of the smallest FCC lattice that has
-    them (N of its sites taken at random, all of them for whole_cells), each
-    moved by a normal jitter, in a cubic box.  -> (N, 3) float32, box length"""
+    """N positions at density rho: sites of the smallest near-cubic FCC lattice
+    that has them (N of its sites taken at random, all of them for
+    whole_cells), each moved by a normal jitter, in a cubic box.
+    -> (N, 3) float32, box length"""
     n = math.ceil((N / 4) ** (1 / 3) - 1e-9)
-    corner = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), axis=-1).reshape(-1, 1, 3)
+    cells = min((a * b * c, (a, b, c)) for a in (n, n - 1) for b in (n, n - 1) for c in (n, n + 1)
+                if 4 * a * b * c >= N)[1]
+    corner = np.stack(np.meshgrid(*[np.arange(k) for k in cells], indexing="ij"), axis=-1).reshape(-1, 1, 3)
     sites = (corner + np.array([[0, 0, 0], [.5, .5, 0], [.5, 0, .5], [0, .5, .5]]) + 0.25).reshape(-1, 3)
     if whole_cells:
         assert len(sites) == N
     else:
         sites = sites[np.sort(g.permutation(len(sites))[:N])]
     L = float(np.float32((N / rho) ** (1 / 3)))
-    r = (sites / n - 0.5) * L + g.normal(0.0, jitter, sites.shape)
+    r = (sites / np.array(cells) - 0.5) * L + g.normal(0.0, jitter, sites.shape)
     r -= L * np.round(r / L)
     return r.astype(np.float32), L
 
@@ -182,15 +185,17 @@ def _prepare_md(case, seed):
     if case["scalars"]:
         actions.append(gp.ScalarSaver(SCALAR_EVERY))
     sim = gp.Simulation(conf, inter, _integrator(case, seed), actions, num_timeblocks=TIMEBLOCKS,
-                        steps_per_timeblock=case["steps"], compute_plan=plan, storage="memory")
+                        steps_per_timeblock=case["steps"], compute_plan=plan, storage="memory", steps_in_kernel_test=0)
     rdf = gp.CalculatorRadialDistribution(conf, bins=case["rdf_bins"]) if case["rdf_bins"] else None
     conf.copy_to_device()   # the start, where the first g(r) is taken
     return {"kind": "md", "conf": conf, "sim": sim, "rdf": rdf, "blocks": sim.run_timeblocks()}
 
 
 def _replica_points(case, seed):
-    g = np.random.default_rng(seed)
-    return [(int(g.integers(case["Nmin"], case["Nmax"] + 1)), float(g.uniform(1.1, 1.25)), float(g.uniform(0.7, 2.0)))
+    """(N, density, temperature) of each replica: sizes spread over the case's
+    range, state points from the seed."""
+    g, n = np.random.default_rng(seed), np.random.default_rng(case["replicas"])
+    return [(int(n.integers(case["Nmin"], case["Nmax"] + 1)), float(g.uniform(1.1, 1.25)), float(g.uniform(0.7, 2.0)))
             for _ in range(case["replicas"])]
 
 
