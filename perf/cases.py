@@ -108,7 +108,7 @@ def draw(rng):
 def _positions(N, rho, g, jitter, whole_cells=False):
     """N positions at density rho: sites of the smallest near-cubic FCC lattice
     that has them (N of its sites taken at random, all of them for
-    whole_cells), each moved by a normal jitter, in a cubic box.
+    whole_cells), each moved by up to jitter per dimension, in a cubic box.
     -> (N, 3) float32, box length"""
     n = math.ceil((N / 4) ** (1 / 3) - 1e-9)
     cells = min((a * b * c, (a, b, c)) for a in (n, n - 1) for b in (n, n - 1) for c in (n, n + 1)
@@ -120,12 +120,12 @@ def _positions(N, rho, g, jitter, whole_cells=False):
     else:
         sites = sites[np.sort(g.permutation(len(sites))[:N])]
     L = float(np.float32((N / rho) ** (1 / 3)))
-    r = (sites / np.array(cells) - 0.5) * L + g.normal(0.0, jitter, sites.shape)
+    r = (sites / np.array(cells) - 0.5) * L + g.uniform(-jitter, jitter, sites.shape)
     r -= L * np.round(r / L)
     return r.astype(np.float32), L
 
 
-def _configuration(system, N, rho, T, seed, lap=False, jitter=0.05):
+def _configuration(system, N, rho, T, seed, lap=False, jitter=0.06):
     g = np.random.default_rng(seed)
     conf = gp.Configuration(D=3, compute_flags={"lapU": True} if lap else None)
     r, L = _positions(N, rho, g, jitter, whole_cells=system == "chains")
@@ -221,7 +221,7 @@ def _prepare_adjoint(case, seed):
 
 
 def _rdf_configuration(case, seed):
-    conf = _configuration("ka", case["N"], case["rho"], 1.0, seed, jitter=0.08)
+    conf = _configuration("ka", case["N"], case["rho"], 1.0, seed, jitter=0.1)
     order = np.random.default_rng(seed + 1).permutation(case["N"])
     conf["r"] = np.ascontiguousarray(conf["r"][order])
     conf.ptype = np.ascontiguousarray(conf.ptype[order])
