@@ -2,6 +2,7 @@
 
     python -m gamdpy_amd._build
 """
+import concurrent.futures
 import os
 import shutil
 import subprocess
@@ -9,14 +10,18 @@ import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(_HERE)
-# gmd_core.hip holds the host code, the base-0 step kernels and every other
-# kernel; each further pair-function base, and the NPT_Atomic kernels of each
-# base, have instance files of their own, so they compile in parallel and are
-# linked into one library
-SOURCES = [os.path.join(_HERE, "csrc", f) for f in ("gmd_core.hip", "gmd_steps_b1.hip", "gmd_steps_b2.hip",
-                                                     "gmd_steps_b3.hip", "gmd_steps_npt_b0.hip",
-                                                     "gmd_steps_npt_b1.hip", "gmd_steps_npt_b2.hip",
-                                                     "gmd_steps_npt_b3.hip")]
+# gmd_core.hip holds the host code and every kernel but the step kernels, which
+# gmd_steps_inst.hip instantiates one (pair-function base, cutoff) group per
+# compilation, and the NPT_Atomic kernels of each base in one more: the groups
+# compile in parallel (the longest first) and are linked into one library
+_CORE = os.path.join(_HERE, "csrc", "gmd_core.hip")
+_INST = os.path.join(_HERE, "csrc", "gmd_steps_inst.hip")
+SOURCES = [(_INST, f"steps_b{b}_c{c}", [f"-DGMD_INST_BASE={b}", f"-DGMD_INST_CUT={c}"])
+           for b in (2, 3, 1) for c in range(3)] + \
+          [(_INST, f"steps_b{b}_npt", [f"-DGMD_INST_BASE={b}", "-DGMD_INST_NPT"]) for b in (2, 3, 1, 0)] + \
+          [(_INST, f"steps_b0_c{c}", ["-DGMD_INST_BASE=0", f"-DGMD_INST_CUT={c}"]) for c in range(3)] + \
+          [(_CORE, "core", [])]
+JOBS = max(1, min(8, os.cpu_count() or 1))   # compilations at a time
 DEPS = [os.path.join(_HERE, "csrc", f) for f in ("gmd_device.h", "gmd_kernels.h", "gmd_steps.h", "gmd_adjoint.h")] + \
        [os.path.join(ROOT, "include", "gamdpy_amd.h")]
 OUT = os.path.join(_HERE, "libgamdpy_amd.so")
@@ -46,27 +51,25 @@ def build(verbose=False):
     (always recompiles)."""
     cc = hipcc()
     inc = ["-I", os.path.join(ROOT, "include")]
-    objs, procs = [], []
-    for src in SOURCES:
-        obj = OUT + "." + os.path.splitext(os.path.basename(src))[0] + ".o"
-        cmd = [cc] + HIPCC_FLAGS + inc + ["-c", src, "-o", obj]
+    jobs = [(src, OUT + "." + name + ".o", HIPCC_FLAGS + inc + defs + ["-c"]) for src, name, defs in SOURCES]
+    jobs.append((REF_SOURCE, REF_OUT + ".tmp", HIPCC_FLAGS + ["-shared"]))
+    failed = []
+
+    def compile_one(job):
+        src, out, flags = job
+        cmd = [cc] + flags + [src, "-o", out]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True), src))
-        objs.append(obj)
-    ref_cmd = [cc] + HIPCC_FLAGS + ["-shared", REF_SOURCE, "-o", REF_OUT + ".tmp"]
-    if verbose:
-        print(" ".join(ref_cmd), flush=True)
-    procs.append((subprocess.Popen(ref_cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True),
-                  REF_SOURCE))
-    failed = []
-    for proc, src in procs:
-        out, _ = proc.communicate()
-        if proc.returncode != 0:
-            sys.stderr.write(out)
-            failed.append(src)
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        if res.returncode != 0:
+            sys.stderr.write(res.stdout)
+            failed.append(os.path.basename(out))
+
+    with concurrent.futures.ThreadPoolExecutor(JOBS) as pool:
+        list(pool.map(compile_one, jobs))
     if failed:
-        raise RuntimeError(f"hipcc failed for {', '.join(os.path.basename(f) for f in failed)}")
+        raise RuntimeError(f"hipcc failed for {', '.join(failed)}")
+    objs = [out for _, out, _ in jobs[:-1]]
     tmp = OUT + ".tmp"
     cmd = [cc, f"--offload-arch={ARCH}", "-shared", "-fPIC"] + objs + ["-o", tmp]
     if verbose:

@@ -16,8 +16,8 @@
 
 #include "gmd_steps.h"
 
-// the instances of the other pair-function bases live in gmd_steps_b{1,2,3}.hip,
-// the NPT_Atomic instances in gmd_steps_npt_b{0,1,2,3}.hip
+// the step kernels are instantiated by gmd_steps_inst.hip, a group per compilation
+GMD_STEP_KERNELS_BASE(extern, 0)
 GMD_STEP_KERNELS_BASE(extern, 1)
 GMD_STEP_KERNELS_BASE(extern, 2)
 GMD_STEP_KERNELS_BASE(extern, 3)
@@ -591,6 +591,7 @@ typedef void (*sfun)(const DP *, int);
 typedef void (*bfun)(const DP *const *, const BatchBlk *);
 
 // the kernel instances of one (pair function, cutoff, integrator) combination
+// and list kind
 struct Kernels {
     kfun pers;
     sfun step;
@@ -598,38 +599,39 @@ struct Kernels {
 };
 
 template <int BASE, int CUT, int INTEG>
-Kernels pick() {
-    return Kernels{k_persistent<BASE, CUT, INTEG>, k_step<BASE, CUT, INTEG>, k_batch_persistent<BASE, CUT, INTEG>,
-                   k_batch_step<BASE, CUT, INTEG>};
+Kernels pick(int kind) {
+    return Kernels{kind == 1 ? k_persistent<BASE, CUT, INTEG, 1> : k_persistent<BASE, CUT, INTEG, 0>,
+                   kind == 1 ? k_step<BASE, CUT, INTEG, 1> : k_step<BASE, CUT, INTEG, 0>,
+                   k_batch_persistent<BASE, CUT, INTEG>, k_batch_step<BASE, CUT, INTEG>};
 }
 
 template <int BASE, int CUT>
-Kernels pick_integ(int integ) {
+Kernels pick_integ(int integ, int kind) {
     switch (integ) {
-        case 0: return pick<BASE, CUT, 0>();
-        case 1: return pick<BASE, CUT, 1>();
-        case 2: return pick<BASE, CUT, 2>();
-        case 3: return pick<BASE, CUT, 3>();
-        default: return pick<BASE, CUT, 4>();
+        case 0: return pick<BASE, CUT, 0>(kind);
+        case 1: return pick<BASE, CUT, 1>(kind);
+        case 2: return pick<BASE, CUT, 2>(kind);
+        case 3: return pick<BASE, CUT, 3>(kind);
+        default: return pick<BASE, CUT, 4>(kind);
     }
 }
 
 template <int BASE>
-Kernels pick_cut(int cut, int integ) {
+Kernels pick_cut(int cut, int integ, int kind) {
     switch (cut) {
-        case 0: return pick_integ<BASE, 0>(integ);
-        case 1: return pick_integ<BASE, 1>(integ);
-        default: return pick_integ<BASE, 2>(integ);
+        case 0: return pick_integ<BASE, 0>(integ, kind);
+        case 1: return pick_integ<BASE, 1>(integ, kind);
+        default: return pick_integ<BASE, 2>(integ, kind);
     }
 }
 
 // pair functions 2..5 share one instance (a uniform switch on the kind
 // inside), and so do 6..7 (parameter rows)
-Kernels pick_kernels(int base, int cut, int integ) {
-    return base == 0   ? pick_cut<0>(cut, integ)
-           : base == 1 ? pick_cut<1>(cut, integ)
-           : base <= 5 ? pick_cut<2>(cut, integ)
-                       : pick_cut<3>(cut, integ);
+Kernels pick_kernels(int base, int cut, int integ, int kind) {
+    return base == 0   ? pick_cut<0>(cut, integ, kind)
+           : base == 1 ? pick_cut<1>(cut, integ, kind)
+           : base <= 5 ? pick_cut<2>(cut, integ, kind)
+                       : pick_cut<3>(cut, integ, kind);
 }
 
 float i2f(int v) {
@@ -943,12 +945,13 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     // dynamic LDS: pair table | reduction scratch (one row of sums per wave) |
     // rebuild scratch; sized so that four blocks of 256 fit in a CU's 160 KB
     const size_t lds_cells = (d.nblist_kind == GMD_NBLIST_LINKED_LISTS) ? (size_t)wpb * LL_WAVE_LDS : 0;
-    // N squared: the tile of positions (16 B each) and 256 accepted slots per wave (8 B per thread)
+    // N squared: two tiles of positions (16 B each) and the accepted slots of a wave's particles
     // (a list step stages each wave's velocities and reference positions in
     // the same region: 2 KB a wave)
     // (and a deferred Nose-Hoover tail stages the previous step's kinetic
     // partials after them: RED_PRE floats a thread)
-    c->lds_build = std::max(std::max(lds_cells, (size_t)block * 24), (size_t)wpb * 2048 + (size_t)RED_PRE * block * 4);
+    const size_t lds_nsq = (size_t)block * 32 + (size_t)wpb * NSQ_PP * NSQ_CAP * 2;
+    c->lds_build = std::max(std::max(lds_cells, lds_nsq), (size_t)wpb * 2048 + (size_t)RED_PRE * block * 4);
     const size_t lds_pp = 0;
     const size_t lds_red = ((size_t)d.ntypes * d.ntypes * sizeof(PairP) + 15) / 16 * 16;
     const size_t lds_b = lds_red + (size_t)wpb * GMD_NRED * sizeof(double);
@@ -1180,7 +1183,7 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     P.perm = (const GMEM int *)c->perm;
 
     TRY(dalloc(&c->d_P, 1));
-    c->kern = pick_kernels(d.pair_base, d.cutoff, d.integrator);
+    c->kern = pick_kernels(d.pair_base, d.cutoff, d.integrator, d.nblist_kind);
 
     // ---- cooperative grid: all blocks must be co-resident ----
     if (d.gridsync) {

@@ -124,6 +124,13 @@ __device__ __forceinline__ void wave_sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A barrier of the block over its LDS only: __syncthreads also waits for the
+// wavefront's global loads and stores, here the next tile's positions and
+// the list entries, which no other wavefront of the block reads
+__device__ __forceinline__ void block_sync_lds() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ---------------------------------------------------------------------------
 // Cell grid: nblist_linked_lists.py:125-131, cell index evaluated in float64
 // (numba promotes r + 0.5*L to float64): floor((r + L/2) n / L) mod n.
@@ -1254,20 +1261,39 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
 }
 
 // ---------------------------------------------------------------------------
-// Rebuild step, N squared (nblist.py:89-143): one wavefront per particle i.
-// The block stages 256 positions at a time in LDS; each wavefront tests them
-// against its particle 64 at a time and compacts the accepted tile slots with
-// a ballot, then appends those j to the list (so it is in ascending j) and
-// adds their pair terms in one pass, every lane busy; lane 0 integrates the
-// particle.  Every wavefront of every block runs the same number of rounds
-// (the tiles are shared).
+// Rebuild step, N squared (nblist.py:89-143): NSQ_PP particles per wavefront
+// at a time.  The block stages tiles of blockDim.x positions in LDS (two
+// buffers, the next tile's load in flight during the current one: one block
+// barrier a tile).  A wavefront reads 64 positions of the tile once and tests
+// them against its particles, compacting each particle's accepted tile slots
+// with a ballot; then every particle's 16 lanes write its list entries
+// (ascending j) and add its pair terms, the particles side by side.  The
+// first lane of each group integrates its particle.
+//
+// The kernel is bound by the latency of each wavefront's chain (tile read,
+// test, ballot, compaction): a system that takes the N-squared list leaves a
+// SIMD one wavefront or less, so the particles of a wavefront are its only
+// independent work, and one at a time left most of the chain exposed.
+// Measured with one and with four at a time (and the rebuild in a kernel
+// without the linked-list walk): a rebuild step of LJ N = 2048 (512
+// wavefronts) 56.5 -> 33.6 us, of KA N = 4000 101 -> 57.6 us.  A wavefront
+// then spends about 5100 cycles a tile on the tests and 2850 on the pairs,
+// an instruction about every 10 cycles.
+//
+// The sums keep the order of a wavefront that gives each accepted pair of a
+// tile the lane of its rank mod 64 and adds the lanes pairwise (32, 16, ...,
+// 1 apart): rank 16 k + l of a particle is added to its sum k in lane l of
+// its group, and sums 0 + 2 and 1 + 3 are those two levels.
 // ---------------------------------------------------------------------------
+#define NSQ_PP 4                 // particles a wavefront takes at a time (16 lanes each in the pair pass)
+#define NSQ_CAP 256              // accepted slots of one particle and tile (a tile holds at most 256 positions)
+
 template <int BASE, int CUT, int INTEG>
 __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B, const StepInfo &I, const PairP *pp,
-                                                 float4 *tile, float acc[GMD_NRED]) {
+                                                 float4 *tiles, float acc[GMD_NRED]) {
     const int bd = blockDim.x;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, wpb = bd >> 6;
-    const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int g = lane >> 4, l16 = lane & 15;
     const int per_round = B.nb * wpb;
     const int rounds = (P.N + per_round - 1) / per_round;
     const float L0 = INTEG == 4 ? I.L0 : P.box0, L1 = INTEG == 4 ? I.L1 : P.box1, L2 = INTEG == 4 ? I.L2 : P.box2;
@@ -1276,83 +1302,199 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
     const int N = P.N, maxnb = P.max_nbs;
     const bool niii = P.niii != 0, has_excl = P.excl != nullptr;
     const float cps2 = P.cps2;
-    // this wave's accepted tile slots (a tile holds bd <= 256 positions)
-    unsigned short *accs = (unsigned short *)(tile + bd) + wid * 256;
-    for (int rd = 0; rd < rounds; ++rd) {
-        const int i = (rd * B.nb + B.bid) * wpb + wid;   // wave-uniform
-        const bool valid = i < P.N;
-        float4 ri = make_float4(0.f, 0.f, 0.f, 0.f), vi = make_float4(0.f, 0.f, 0.f, 1.f);
-        if (valid) {
-            ri = pos[i];
-            vi = P.vel[i];
+    // held in registers (the list stores would otherwise make the compiler
+    // read the descriptor again every tile)
+    const int tp = P.tp, tsh = P.tp_shift;
+    const bool nb16 = P.nb16 != 0;
+    GMEM int *const nbl = P.nbl;
+    const size_t rs = (size_t)N * (size_t)tp;
+    const float iL0 = P.ibox0, iL1 = P.ibox1, iL2 = P.ibox2;
+    // With every position in the box and the list radius below half of it,
+    // the three-instruction image gives the same bits for every pair inside
+    // the radius (mic_list differs from mic1 only where |d| is L/2 to within
+    // a few ulp, and such a pair is outside)
+    const float hmin = 0.5f * fminf(L0, fminf(L1, L2));
+    const bool near = I.wrapped && cps2 < 0.9999f * (hmin * hmin);
+    // this wave's accepted tile slots, NSQ_CAP a particle
+    unsigned short *accs = (unsigned short *)(tiles + 2 * bd) + wid * (NSQ_PP * NSQ_CAP);
+    for (int rd = 0; rd < rounds; rd += NSQ_PP) {
+        // particle k of the wavefront: round rd + k, held by lanes 16k .. 16k + 15
+        const int iq = ((rd + g) * B.nb + B.bid) * wpb + wid;
+        const bool mine = iq < N && rd + g < rounds;
+        float4 rq = make_float4(0.f, 0.f, 0.f, 0.f), vq = make_float4(0.f, 0.f, 0.f, 1.f);
+        if (mine) {
+            rq = pos[iq];
+            vq = P.vel[iq];
         }
-        const PairP *ppi = pp + (valid ? __float_as_int(ri.w) : 0) * P.ntypes;
-        int cnt = 0, nhalf = 0;
-        float fx = 0.f, fy = 0.f, fz = 0.f, uu = 0.f, ww = 0.f, ll = 0.f;
-        for (int t0 = 0; t0 < P.N; t0 += bd) {
-            __syncthreads();
-            const int jl = t0 + (int)threadIdx.x;
-            if (jl < P.N) tile[threadIdx.x] = pos[jl];
-            __syncthreads();
+        int ik[NSQ_PP], cnt[NSQ_PP], nhalf[NSQ_PP];
+        float xk[NSQ_PP], yk[NSQ_PP], zk[NSQ_PP];
+#pragma unroll
+        for (int k = 0; k < NSQ_PP; ++k) {
+            // a round past the last, or an index past N, takes no pair
+            ik[k] = lane_i(mine ? iq : -1, 16 * k);
+            xk[k] = lane_f(rq.x, 16 * k);
+            yk[k] = lane_f(rq.y, 16 * k);
+            zk[k] = lane_f(rq.z, 16 * k);
+            cnt[k] = 0;
+            nhalf[k] = 0;
+        }
+        const PairP *ppi = pp + __float_as_int(rq.w) * P.ntypes;
+        float fx[4], fy[4], fz[4], uu[4], ww[4], ll[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) fx[u] = fy[u] = fz[u] = uu[u] = ww[u] = ll[u] = 0.f;
+        auto rotate = [&]() {
+            auto turn1 = [](float (&v)[4]) {
+                const float t = v[0];
+                v[0] = v[1];
+                v[1] = v[2];
+                v[2] = v[3];
+                v[3] = t;
+            };
+            turn1(fx);
+            turn1(fy);
+            turn1(fz);
+            turn1(uu);
+            turn1(ww);
+            turn1(ll);
+        };
+        int buf = 0;
+        float4 nxt = pos[min((int)threadIdx.x, N - 1)];
+        if (rd > 0) block_sync_lds();   // the last tiles of the previous round have been read
+        for (int t0 = 0; t0 < N; t0 += bd) {
+            float4 *tile = tiles + buf * bd;
+            buf ^= 1;
+            tile[threadIdx.x] = nxt;
+            block_sync_lds();
+            if (t0 + bd < N) nxt = pos[min(t0 + bd + (int)threadIdx.x, N - 1)];
             const int tn = min(bd, N - t0);
-            if (!valid) continue;
-            // the list test only, branch-free (e < bd: inside the tile; lanes
-            // past tn are masked), accepted slots compacted in ballot order
-            int nacc = 0;
-            for (int c0 = 0; c0 < tn; c0 += 64) {
-                const int e = c0 + lane;
-                const float4 rj = tile[e];
-                const int j = t0 + e;
-                float dx, dy, dz;
-                const float d2 = dist_sq_mic(rj.x, rj.y, rj.z, ri.x, ri.y, ri.z, L0, L1, L2, dx, dy, dz);
-                bool ok = (e < tn) & (j != i) & (d2 < cps2);
-                if (has_excl) {
-                    if (ok) ok = !excluded(P, i, j);
-                }
-                const unsigned long long mask = __ballot(ok);
-                if (ok) accs[nacc + __popcll(mask & lt_mask)] = (unsigned short)e;
-                nacc += __popcll(mask);
-                if (niii) nhalf += __popcll(__ballot(ok && niii_owns(i, j, N)));
+            // the list test of 64 positions against each particle.  PLAIN: a
+            // full tile that holds none of the particles themselves, no
+            // exclusions, no half lists
+            int nacc[NSQ_PP];
+            bool plain = tn == bd && !has_excl && !niii;
+#pragma unroll
+            for (int k = 0; k < NSQ_PP; ++k) {
+                nacc[k] = 0;
+                plain = plain && ik[k] >= 0 && (unsigned)(ik[k] - t0) >= (unsigned)bd;
             }
+            float4 cj[4];   // the tile's positions (at most 256), read together
+#pragma unroll
+            for (int u = 0; u < 4; ++u) cj[u] = tile[64 * u < bd ? 64 * u + lane : lane];
+            auto filter = [&](auto img, auto full) {
+                constexpr bool NEAR = decltype(img)::value, PLAIN = decltype(full)::value;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (64 * u >= tn) break;   // the same for every lane
+                    const int c0 = 64 * u, left = tn - c0;
+                    // the distances of all the particles before the first
+                    // compaction: independent chains
+                    float d2[NSQ_PP];
+#pragma unroll
+                    for (int k = 0; k < NSQ_PP; ++k) {
+                        float dx, dy, dz;
+                        d2[k] = NEAR ? dist_sq_list(cj[u].x, cj[u].y, cj[u].z, xk[k], yk[k], zk[k], L0, L1, L2, iL0,
+                                                    iL1, iL2, dx, dy, dz)
+                                     : dist_sq_mic(cj[u].x, cj[u].y, cj[u].z, xk[k], yk[k], zk[k], L0, L1, L2, dx, dy,
+                                                   dz);
+                    }
+#pragma unroll
+                    for (int k = 0; k < NSQ_PP; ++k) {
+                        bool ok = d2[k] < cps2;
+                        unsigned long long mask = __ballot(ok);
+                        if (!PLAIN) {
+                            mask &= left >= 64 ? ~0ull : (1ull << left) - 1ull;
+                            const unsigned self = (unsigned)(ik[k] - (t0 + c0));   // the particle itself
+                            if (self < 64u) mask &= ~(1ull << self);
+                            if (ik[k] < 0) mask = 0ull;
+                            ok = (mask >> lane) & 1ull;
+                            if (has_excl) {
+                                if (ok) ok = !excluded(P, ik[k], t0 + c0 + lane);
+                                mask = __ballot(ok);
+                            }
+                            if (niii) nhalf[k] += __popcll(__ballot(ok && niii_owns(ik[k], t0 + c0 + lane, N)));
+                        }
+                        const int at = nacc[k] + __builtin_amdgcn_mbcnt_hi(
+                                                     (unsigned)(mask >> 32),
+                                                     __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+                        if (ok) accs[k * NSQ_CAP + at] = (unsigned short)(c0 + lane);
+                        nacc[k] += __popcll(mask);
+                    }
+                }
+            };
+            if (near && plain)
+                filter(std::integral_constant<bool, true>{}, std::integral_constant<bool, true>{});
+            else if (near)
+                filter(std::integral_constant<bool, true>{}, std::integral_constant<bool, false>{});
+            else
+                filter(std::integral_constant<bool, false>{}, std::integral_constant<bool, false>{});
             wave_sync_lds();
-            // the accepted pairs of the tile, every lane busy: list entries
-            // (slots cnt + a, tile order) and pair terms
-            for (int a = lane; a < nacc; a += 64) {
-                const int e = accs[a];
+            // the accepted pairs of the tile, each particle on its 16 lanes:
+            // list entries (slots cnt + rank, tile order) and pair terms
+            const int na = g == 0 ? nacc[0] : g == 1 ? nacc[1] : g == 2 ? nacc[2] : nacc[3];
+            const int c_q = g == 0 ? cnt[0] : g == 1 ? cnt[1] : g == 2 ? cnt[2] : cnt[3];
+            const int amax = max(max(nacc[0], nacc[1]), max(nacc[2], nacc[3]));
+            const unsigned short *mya = accs + g * NSQ_CAP;
+            auto pair = [&](const int a, float &ax, float &ay, float &az, float &au, float &aw, float &al) {
+                if (a >= na) return;
+                const int e = mya[a];
                 const float4 rj = tile[e];
-                const int slot = cnt + a;
-                if (slot < maxnb)
-                    nbl_put(P.nbl + (size_t)i * P.tp, slot, t0 + e, P.tp_shift, P.tp, (size_t)P.N * P.tp, P.nb16 != 0);
+                const int slot = c_q + a;
+                if (slot < maxnb) nbl_put(nbl + (size_t)iq * tp, slot, t0 + e, tsh, tp, rs, nb16);
                 float dx, dy, dz;
-                const float d2 = dist_sq_mic(rj.x, rj.y, rj.z, ri.x, ri.y, ri.z, L0, L1, L2, dx, dy, dz);
+                const float d2 = dist_sq_mic(rj.x, rj.y, rj.z, rq.x, rq.y, rq.z, L0, L1, L2, dx, dy, dz);
                 const PairP &q = ppi[__float_as_int(rj.w)];
-                if (d2 < q.cut2) {
-                    if (niii)
-                        pair_accum_w<BASE, CUT>(d2, dx, dy, dz, q, fx, fy, fz, uu, ww, ll, lap,
-                                                niii_owns(i, t0 + e, N) ? 2.0f : 0.0f);
-                    else
-                        pair_accum<BASE, CUT>(d2, dx, dy, dz, q, fx, fy, fz, uu, ww, ll, lap);
-                }
+                if (d2 >= q.cut2) return;
+                if (niii)
+                    pair_accum_w<BASE, CUT>(d2, dx, dy, dz, q, ax, ay, az, au, aw, al, lap,
+                                            niii_owns(iq, t0 + e, N) ? 2.0f : 0.0f);
+                else
+                    pair_accum<BASE, CUT>(d2, dx, dy, dz, q, ax, ay, az, au, aw, al, lap);
+            };
+            // (the sums take turns by rotation, so the pair function is there
+            // once: the families of the later bases are long)
+            int turn = 0;
+#pragma unroll 1
+            for (int a0 = 0; a0 < amax; a0 += 16, ++turn) {
+                pair(a0 + l16, fx[0], fy[0], fz[0], uu[0], ww[0], ll[0]);
+                rotate();
             }
-            cnt += nacc;
+#pragma unroll 1
+            for (; turn & 3; ++turn) rotate();
+#pragma unroll
+            for (int k = 0; k < NSQ_PP; ++k) cnt[k] += nacc[k];
             wave_sync_lds();   // accs is rewritten for the next tile
         }
-        if (valid) {
-            fx = wave_sum_f(fx);
-            fy = wave_sum_f(fy);
-            fz = wave_sum_f(fz);
-            uu = wave_sum_f(uu);
-            ww = wave_sum_f(ww);
-            if (lap) ll = wave_sum_f(ll);
-            if (lane == 0) {
-                P.nbc[i] = cnt;
-                P.rref[i] = ri;
-                list_overflow(P, cnt, nhalf);
+        auto total = [&](const float (&v)[4]) {
+            float t = (v[0] + v[2]) + (v[1] + v[3]);
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+            return t;
+        };
+        float sx = total(fx), sy = total(fy), sz = total(fz), su = total(uu), sw = total(ww);
+        float sl = lap ? total(ll) : 0.f;
+        float part[GMD_NRED];
+#pragma unroll
+        for (int c = 0; c < GMD_NRED; ++c) part[c] = 0.f;
+        if (mine) {
+            const int n = g == 0 ? cnt[0] : g == 1 ? cnt[1] : g == 2 ? cnt[2] : cnt[3];
+            const int nh = g == 0 ? nhalf[0] : g == 1 ? nhalf[1] : g == 2 ? nhalf[2] : nhalf[3];
+            if (l16 == 0) {
+                P.nbc[iq] = n;
+                P.rref[iq] = rq;
+                list_overflow(P, n, nh);
             }
-            if (P.boff) bond_terms(P, pos, i, ri, L0, L1, L2, fx, fy, fz, uu, ww, ll);
-            particle_finish<INTEG>(P, I, i, ri, vi, ri, fx, fy, fz, uu * 0.5f, ww * (0.5f / 3.0f), ll, lane == 0,
-                                   acc);
+            if (P.boff) bond_terms(P, pos, iq, rq, L0, L1, L2, sx, sy, sz, su, sw, sl);
+            particle_finish<INTEG>(P, I, iq, rq, vq, rq, sx, sy, sz, su * 0.5f, sw * (0.5f / 3.0f), sl, l16 == 0,
+                                   part);
         }
+        // the step's sums in lane 0, particle after particle
+#pragma unroll
+        for (int k = 0; k < NSQ_PP; ++k)
+#pragma unroll
+            for (int c = 0; c < GMD_NRED; ++c) {
+                const float v = lane_f(part[c], 16 * k);
+                if (lane == 0) acc[c] += v;
+            }
     }
 }
 
@@ -1364,12 +1506,15 @@ __device__ __forceinline__ void step_cells_clear(const DP &P, const BlockCtx &B,
     }
 }
 
-// One full step body (everything but the cross-block tail)
-template <int BASE, int CUT, int INTEG>
+// One full step body (everything but the cross-block tail).  KIND: the list
+// kind the kernel is for (0 N squared, 1 linked lists), or 2 for a kernel
+// that runs replicas of either: a kernel that holds one rebuild only keeps
+// its registers and its instructions
+template <int BASE, int CUT, int INTEG, int KIND>
 __device__ __forceinline__ void step_body(const DP &P, const BlockCtx &B, const StepInfo &I, const PairP *pp, char *build,
                                  float acc[GMD_NRED]) {
     if (I.rebuild) {
-        if (P.nblist_kind == 1)
+        if (KIND == 1 || (KIND == 2 && P.nblist_kind == 1))
             step_ll_rebuild<BASE, CUT, INTEG>(P, B, I, pp, build, acc);
         else
             step_nsq_rebuild<BASE, CUT, INTEG>(P, B, I, pp, (float4 *)build, acc);

@@ -1,7 +1,7 @@
 // gmd_steps.h -- the step kernels as templates over (pair function, cutoff,
-// integrator): included by gmd_core.hip (which instantiates the LJ
-// sigma/epsilon family and declares the others extern) and by one file per
-// further pair-function base, so the instances compile in parallel.
+// integrator, list kind): included by gmd_core.hip, which declares them
+// extern, and by gmd_steps_inst.hip, which instantiates one group of them per
+// compilation.
 #pragma once
 #include "gmd_kernels.h"
 
@@ -20,7 +20,7 @@ __device__ __forceinline__ T *uniform_ptr(T *p) {
     return (T *)(((unsigned long long)hi << 32) | lo);
 }
 
-template <int BASE, int CUT, int INTEG>
+template <int BASE, int CUT, int INTEG, int KIND>
 __device__ __forceinline__ void persistent_body(const DP *Pp, const BlockCtx &B) {
     extern __shared__ __align__(16) char lds[];
     PairP *pp = (PairP *)(lds + Pp->lds_pp);
@@ -36,7 +36,7 @@ __device__ __forceinline__ void persistent_body(const DP *Pp, const BlockCtx &B)
         float acc[GMD_NRED];
 #pragma unroll
         for (int c = 0; c < GMD_NRED; ++c) acc[c] = 0.f;
-        step_body<BASE, CUT, INTEG>(P, B, I, pp, build, acc);
+        step_body<BASE, CUT, INTEG, KIND>(P, B, I, pp, build, acc);
         const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
         if (mask) block_partials(P, B, acc, red, P.partial, mask);
         grid_barrier(P.ctrl, B.nb, [&]() { step_tail(P, I, red, B.nb); });
@@ -49,7 +49,7 @@ __device__ __forceinline__ void persistent_body(const DP *Pp, const BlockCtx &B)
 // buffers.  Otherwise (replicas of a batch) the step index and the rebuild
 // decision come from the control block that the previous step's k_batch_tail
 // wrote.
-template <int BASE, int CUT, int INTEG, bool FOLD>
+template <int BASE, int CUT, int INTEG, int KIND, bool FOLD>
 __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k) {
     extern __shared__ __align__(16) char lds[];
     const int s = FOLD ? P.ctrl->s_base + k : P.ctrl->step;
@@ -135,7 +135,7 @@ __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k)
     float acc[GMD_NRED];
 #pragma unroll
     for (int c = 0; c < GMD_NRED; ++c) acc[c] = 0.f;
-    step_body<BASE, CUT, INTEG>(P, B, I, pp, build, acc);
+    step_body<BASE, CUT, INTEG, KIND>(P, B, I, pp, build, acc);
     const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
     if (mask) block_partials(P, B, acc, red, FOLD ? P.partial + (size_t)(s & 1) * GMD_NRED * P.pstride : P.partial, mask);
     if (FOLD && rebuild && B.bid == 0 && threadIdx.x == 0) P.ctrl->nbflag[2] += 1;
@@ -150,9 +150,9 @@ __device__ __forceinline__ BlockCtx xcd_block(int b, int nb) {
     return BlockCtx{b, nb};
 }
 
-template <int BASE, int CUT, int INTEG>
+template <int BASE, int CUT, int INTEG, int KIND>
 __global__ void __launch_bounds__(256) k_persistent(const DP *__restrict__ Pp) {
-    persistent_body<BASE, CUT, INTEG>(Pp, xcd_block((int)blockIdx.x, (int)gridDim.x));
+    persistent_body<BASE, CUT, INTEG, KIND>(Pp, xcd_block((int)blockIdx.x, (int)gridDim.x));
 }
 
 // One step per launch (step s_base + k).  The cross-block work of a step
@@ -161,9 +161,9 @@ __global__ void __launch_bounds__(256) k_persistent(const DP *__restrict__ Pp) {
 // between steps, and no last-block-done scheme, which would need an
 // agent-scope release per block (a write-back of the XCD's L2 under the
 // blocks still running).
-template <int BASE, int CUT, int INTEG>
+template <int BASE, int CUT, int INTEG, int KIND>
 __global__ void __launch_bounds__(256, 4) k_step(const DP *__restrict__ Pp, int k) {
-    step_once<BASE, CUT, INTEG, true>(*Pp, xcd_block((int)blockIdx.x, (int)gridDim.x), k);
+    step_once<BASE, CUT, INTEG, KIND, true>(*Pp, xcd_block((int)blockIdx.x, (int)gridDim.x), k);
 }
 
 // Batched replicas: block b of the grid works for replica blk[b].rep as its
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(256) k_batch_persistent(const DP *const *Ps, c
     const int rep = __builtin_amdgcn_readfirstlane(a.rep);
     if (rep < 0) return;
     const BlockCtx B = {__builtin_amdgcn_readfirstlane(a.bid), __builtin_amdgcn_readfirstlane(a.nb)};
-    persistent_body<BASE, CUT, INTEG>(uniform_ptr(Ps[rep]), B);
+    persistent_body<BASE, CUT, INTEG, 2>(uniform_ptr(Ps[rep]), B);
 }
 
 // (at most 168 VGPRs: three wavefronts per SIMD)
@@ -189,15 +189,17 @@ __global__ void __launch_bounds__(256, 3) k_batch_step(const DP *const *Ps, cons
     const int rep = __builtin_amdgcn_readfirstlane(a.rep);
     if (rep < 0) return;
     const BlockCtx B = {__builtin_amdgcn_readfirstlane(a.bid), __builtin_amdgcn_readfirstlane(a.nb)};
-    step_once<BASE, CUT, INTEG, false>(*uniform_ptr(Ps[rep]), B, 0);
+    step_once<BASE, CUT, INTEG, 2, false>(*uniform_ptr(Ps[rep]), B, 0);
 }
 
 
-// explicit instantiation (EXT empty) or declaration (EXT extern) of the four
-// step kernels of one (base, cutoff, integrator)
+// explicit instantiation (EXT empty) or declaration (EXT extern) of the step
+// kernels of one (base, cutoff, integrator)
 #define GMD_STEP_KERNELS(EXT, B, C, I)                                                          \
-    EXT template __global__ void k_persistent<B, C, I>(const DP *);                              \
-    EXT template __global__ void k_step<B, C, I>(const DP *, int);                               \
+    EXT template __global__ void k_persistent<B, C, I, 0>(const DP *);                           \
+    EXT template __global__ void k_persistent<B, C, I, 1>(const DP *);                           \
+    EXT template __global__ void k_step<B, C, I, 0>(const DP *, int);                            \
+    EXT template __global__ void k_step<B, C, I, 1>(const DP *, int);                            \
     EXT template __global__ void k_batch_persistent<B, C, I>(const DP *const *, const BatchBlk *); \
     EXT template __global__ void k_batch_step<B, C, I>(const DP *const *, const BatchBlk *);
 #define GMD_STEP_KERNELS_CUT(EXT, B, C) \
