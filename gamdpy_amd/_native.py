@@ -135,6 +135,7 @@ _SIGNATURES = {
     "gmd_batch_size": (ctypes.c_int, [ctypes.c_void_p, c_int_p, c_int_p]),
     "gmd_batch_context": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_void_p)]),
     "gmd_batch_run": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_float, ctypes.c_int]),
+    "gmd_batch_fetch": (ctypes.c_int, [ctypes.c_void_p]),
     "gmd_batch_last_run_ms": (ctypes.c_int, [ctypes.c_void_p, c_float_p]),
     "gmd_adj_create": (ctypes.c_int, [ctypes.POINTER(GmdAdjDesc), c_int_p, c_float_p, ctypes.POINTER(ctypes.c_void_p)]),
     "gmd_adj_destroy": (ctypes.c_int, [ctypes.c_void_p]),
@@ -289,6 +290,8 @@ class Context:
         self.N = d.N
         self.nscalars = d.nscalars
         self.max_nbs = d.max_nbs
+        self._all_columns = sum(k >= 0 for k in (d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq,
+                                                 d.sid_m)) == d.nscalars
         self.saves_per_block = d.scalar_saves_per_block
         self.conf_saves_per_block = d.conf_saves_per_block
 
@@ -322,14 +325,16 @@ class Context:
         check(self.lib.gmd_upload(self.h, fptr(arrs[0]), fptr(arrs[1]), fptr(arrs[2]), fptr(arrs[3]),
                                   iptr(arrs[4]), iptr(arrs[5])), "gmd_upload")
 
-    def download(self):
+    def download(self, vectors=None):
+        """(r, v, f, scalars, ptype, r_im) on the host; vectors: three
+        C-contiguous (N, 3) float32 arrays to fill with r, v and f instead of
+        new ones."""
         N = self.N
-        r = np.zeros((N, 3), np.float32)
-        v = np.zeros((N, 3), np.float32)
-        f = np.zeros((N, 3), np.float32)
-        sc = np.zeros((N, self.nscalars), np.float32)
-        pt = np.zeros(N, np.int32)
-        im = np.zeros((N, 3), np.int32)
+        r, v, f = vectors if vectors is not None else (np.empty((N, 3), np.float32) for _ in range(3))
+        # (a scalar column without a device array is left as it is: zero)
+        sc = (np.empty if self._all_columns else np.zeros)((N, self.nscalars), np.float32)
+        pt = np.empty(N, np.int32)
+        im = np.empty((N, 3), np.int32)
         check(self.lib.gmd_download(self.h, fptr(r), fptr(v), fptr(f), fptr(sc), iptr(pt), iptr(im)), "gmd_download")
         return r, v, f, sc, pt, im
 
@@ -449,6 +454,11 @@ class Batch:
 
     def run(self, time_zero, steps):
         check(self.lib.gmd_batch_run(self.h, ctypes.c_float(np.float32(time_zero)), int(steps)), "gmd_batch_run")
+
+    def fetch(self):
+        """Bring every replica's state to the host in one go, for the
+        downloads that follow."""
+        check(self.lib.gmd_batch_fetch(self.h), "gmd_batch_fetch")
 
     def last_run_ms(self):
         x = ctypes.c_float()

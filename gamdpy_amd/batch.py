@@ -178,6 +178,7 @@ class BatchedSimulation:
                     ra.initialize_before_timeblock()
             self.integrate_self(np.float32(block * self.steps_per_block * self.dt), self.steps_per_block)
             block_times.append(self.batch.last_run_ms())
+            self.batch.fetch()
             for r in self.replicas:
                 r.configuration.copy_to_host()
                 r.integrator.download_state(r.ctx)

@@ -45,9 +45,21 @@ __global__ void __launch_bounds__(256) k_batch_tail(const DP *const *Ps, int int
 // ---- run set-up: cell grid of the starting positions and the skin test ----
 // Kernel parameters are generic pointers (an address-space qualifier would
 // change the kernel's mangled name between the host and device passes).
-__global__ void k_begin_run(Ctrl *Cp, int nsteps, float t0, int buf0, long long lstep0) {
-    GMEM Ctrl *C = (GMEM Ctrl *)Cp;
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+//
+// What a run starts from, in one launch: the control block, the rebuild flags
+// (that of step 0 set where a rebuild is pending), the saver's rows and the
+// three cell buffers cleared.  For small systems a launch costs more than its
+// work, so the clears share one (before: two memsets, a copy and two
+// kernels); block 0 of the x grid writes the control block.
+struct RunStart {
+    int buf0, need_rebuild;
+    long long lstep;
+};
+
+__device__ __forceinline__ void run_begin(const DP &P, int nsteps, float t0, const RunStart R) {
+    GMEM Ctrl *C = P.ctrl;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+    if (t == 0) {
         // NPT_Atomic: the last run left the state of its final step at
         // npt[nsteps & 1]; this run's step 0 reads npt[0]
         if (C->nsteps & 1)
@@ -55,8 +67,8 @@ __global__ void k_begin_run(Ctrl *Cp, int nsteps, float t0, int buf0, long long 
         C->npt_grid_bad = 0;
         C->nsteps = nsteps;
         C->t0 = t0;
-        C->buf0 = buf0;
-        C->lstep0 = lstep0;
+        C->buf0 = R.buf0;
+        C->lstep0 = R.lstep;
         C->step = 0;
         C->s_base = 0;
         C->red_count = 0;
@@ -64,18 +76,25 @@ __global__ void k_begin_run(Ctrl *Cp, int nsteps, float t0, int buf0, long long 
         C->cell_overflow = 0;
         C->unwrapped = 0;
     }
+    for (int k = t; k < nsteps + 2; k += nt) P.rebuild_flag[k] = k == 0 ? R.need_rebuild : 0;
+    if (P.save_every > 0)
+        for (int k = t; k < P.saves_per_block * 6; k += nt) P.saver_out[k] = 0.f;
+    if (P.nblist_kind == 1)
+        for (int k = t; k < 3 * P.ncells; k += nt) P.ccount[k] = 0;
 }
 
-__global__ void __launch_bounds__(256) k_cells_clear(const DP *__restrict__ Pp) {
-    const DP &P = *Pp;
-    const int n = 3 * P.ncells;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) P.ccount[c] = 0;
+__global__ void __launch_bounds__(256) k_run_begin(const DP *__restrict__ Pp, int nsteps, float t0, RunStart R) {
+    run_begin(*Pp, nsteps, t0, R);
+}
+
+// the same for the replicas of a batch (one per y of the grid)
+__global__ void __launch_bounds__(256) k_batch_begin(const DP *const *Ps, int nsteps, float t0, const RunStart *R) {
+    run_begin(*uniform_ptr(Ps[blockIdx.y]), nsteps, t0, R[blockIdx.y]);
 }
 
 // skin test of the starting positions (nblist.py:58-86 at step 0) and, for
 // linked lists, insertion into cell buffer 0
-__global__ void __launch_bounds__(256) k_run_setup(const DP *__restrict__ Pp) {
-    const DP &P = *Pp;
+__device__ __forceinline__ void run_setup(const DP &P) {
     cpos_t pos = P.ctrl->buf0 ? P.pos1 : P.pos0;
     // the box of step 0 (NPT_Atomic: of its state)
     const float L0 = P.npt ? P.ctrl->npt[0][3] : P.box0, L1 = P.npt ? P.ctrl->npt[0][4] : P.box1,
@@ -94,6 +113,10 @@ __global__ void __launch_bounds__(256) k_run_setup(const DP *__restrict__ Pp) {
     }
 }
 
+__global__ void __launch_bounds__(256) k_run_setup(const DP *__restrict__ Pp) { run_setup(*Pp); }
+
+__global__ void __launch_bounds__(256) k_batch_setup(const DP *const *Ps) { run_setup(*uniform_ptr(Ps[blockIdx.y])); }
+
 // the prepared pair table of the context (once)
 __global__ void k_pair_table(const DP *__restrict__ Pp) {
     const DP &P = *Pp;
@@ -105,9 +128,150 @@ __global__ void k_pair_table(const DP *__restrict__ Pp) {
     }
 }
 
-__global__ void k_setup_finish(const DP *__restrict__ Pp) {
+// replicas read the decision of their next step from the control block
+__global__ void __launch_bounds__(256) k_batch_setup_finish(const DP *const *Ps, int nrep) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < nrep) Ps[r]->ctrl->rebuild_now = Ps[r]->rebuild_flag[0];
+}
+
+// ---- what the host reads after a run, into pinned memory: the control block
+// and the saver's rows (a kernel's stores instead of a copy per read) ----
+__device__ __forceinline__ void run_publish(const DP &P) {
+    const GMEM int *c = (const GMEM int *)P.ctrl;
+    const int nc = (int)(sizeof(Ctrl) / 4);
+    for (int k = threadIdx.x; k < nc; k += blockDim.x) P.pub[k] = c[k];
+    if (P.save_every > 0)
+        for (int k = threadIdx.x; k < P.saves_per_block * 6; k += blockDim.x)
+            P.pub[nc + k] = __float_as_int(P.saver_out[k]);
+}
+
+__global__ void __launch_bounds__(256) k_run_publish(const DP *__restrict__ Pp) { run_publish(*Pp); }
+
+__global__ void __launch_bounds__(256) k_batch_publish(const DP *const *Ps) { run_publish(*uniform_ptr(Ps[blockIdx.x])); }
+
+// ---- the host's arrays to and from the device layout ----
+// One kernel gathers every array into the packed buffer (unpack) or takes it
+// apart (pack), in the caller's numbering, and one copy moves the buffer: a
+// copy and a host loop per array cost about 15 us each of round trips and,
+// at N = 50021, 0.6 ms of host time.  Up to XFER_DIRECT particles the kernels
+// read and write the pinned buffer themselves (one launch less; N = 500: an
+// upload, evaluation and download take 74 us, 203 us with the copies per
+// array); above, where the 12-byte rows would make poor use of the bus, a
+// linear copy kernel moves it, or from XFER_DMA words (1 MB, where its launch
+// no longer matters) the copy engine: 66 us for the 3.4 MB of N = 50021.  The
+// kernels themselves take 6 us there and are bound by latency.
+#define XFER_DIRECT 1024
+#define XFER_DMA (1 << 18)
+#define XFER_CHUNK (640 << 10)   // words of a half of the pinned buffer of a large system
+
+__device__ __forceinline__ void unpack_state(const DP &P, int cur, unsigned what, int *dst_p, int i) {
+    GMEM int *dst = (GMEM int *)dst_p;
+    const XferSeg X((size_t)P.N, (size_t)P.nscal);
+    const size_t N = P.N, o = P.perm[i];
+    auto put3 = [&](size_t at, float x, float y, float z) {
+        dst[at + 3 * o] = __float_as_int(x);
+        dst[at + 3 * o + 1] = __float_as_int(y);
+        dst[at + 3 * o + 2] = __float_as_int(z);
+    };
+    if (what & (XF_R | XF_T)) {
+        const float4 r = cur ? P.pos1[i] : P.pos0[i];
+        if (what & XF_R) put3(X.r, r.x, r.y, r.z);
+        if (what & XF_T) dst[X.t + o] = __float_as_int(r.w);
+    }
+    if (what & (XF_V | XF_S)) {
+        const float4 v = P.vel[i];
+        if (what & XF_V) put3(X.v, v.x, v.y, v.z);
+        if (what & XF_S) {
+            GMEM int *row = dst + X.s + o * P.nscal;
+            if (P.sid_u >= 0) row[P.sid_u] = __float_as_int(P.sc[SC_U * N + i]);
+            if (P.sid_w >= 0) row[P.sid_w] = __float_as_int(P.sc[SC_W * N + i]);
+            if (P.sid_lap >= 0) row[P.sid_lap] = __float_as_int(P.sc[SC_LAP * N + i]);
+            if (P.sid_k >= 0) row[P.sid_k] = __float_as_int(P.sc[SC_K * N + i]);
+            if (P.sid_fsq >= 0) row[P.sid_fsq] = __float_as_int(P.sc[SC_FSQ * N + i]);
+            if (P.sid_m >= 0) row[P.sid_m] = __float_as_int(v.w);
+        }
+    }
+    if (what & XF_F) {
+        const float4 f = P.frc[i];
+        put3(X.f, f.x, f.y, f.z);
+    }
+    if (what & XF_IM)
+        for (int k = 0; k < 3; ++k) dst[X.im + 3 * o + k] = P.rim[(size_t)k * N + i];
+}
+
+__global__ void __launch_bounds__(256) k_unpack(const DP *__restrict__ Pp, int cur, unsigned what, int *dst) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < Pp->N; i += gridDim.x * blockDim.x)
+        unpack_state(*Pp, cur, what, dst, i);
+}
+
+// every replica of a batch into its own packed buffer in device memory
+__global__ void __launch_bounds__(256) k_batch_unpack(const DP *const *Ps, const RunStart *R) {
+    const DP &P = *uniform_ptr(Ps[blockIdx.y]);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < P.N; i += gridDim.x * blockDim.x)
+        unpack_state(P, R[blockIdx.y].buf0, XF_ALL, (int *)P.xdev, i);
+}
+
+__device__ __forceinline__ void copy_words(const int *src_p, int *dst_p, size_t n) {
+    const GMEM int4 *src = (const GMEM int4 *)src_p;
+    GMEM int4 *dst = (GMEM int4 *)dst_p;
+    const size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
+    for (size_t k = t; k < n / 4; k += nt) dst[k] = src[k];
+    for (size_t k = n / 4 * 4 + t; k < n; k += nt) ((GMEM int *)dst_p)[k] = ((const GMEM int *)src_p)[k];
+}
+
+// n words between two 16-byte aligned buffers
+__global__ void __launch_bounds__(256) k_copy_words(const int *src, int *dst, size_t n) { copy_words(src, dst, n); }
+
+__global__ void __launch_bounds__(256) k_batch_fetch(const DP *const *Ps) {
+    const DP &P = *uniform_ptr(Ps[blockIdx.y]);
+    copy_words((const int *)P.xdev, P.xhost, XferSeg((size_t)P.N, (size_t)P.nscal).end);
+}
+
+// the packed arrays named by what, in the identity numbering, into the device
+// layout; positions go to pos0.  Positions and types share pos, velocities
+// and masses share vel: a field that is not given keeps its value
+__global__ void __launch_bounds__(256) k_pack(const DP *__restrict__ Pp, int cur, unsigned what, const int *src_p) {
     const DP &P = *Pp;
-    if (threadIdx.x == 0 && blockIdx.x == 0) P.ctrl->rebuild_now = P.rebuild_flag[0];
+    const GMEM int *src = (const GMEM int *)src_p;
+    const GMEM float *fs = (const GMEM float *)src_p;
+    const size_t N = P.N;
+    const XferSeg X(N, (size_t)P.nscal);
+    const bool new_m = (what & XF_S) && P.sid_m >= 0;
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < N; i += (size_t)gridDim.x * blockDim.x) {
+        const GMEM float *row = fs + X.s + i * P.nscal;
+        if (what & (XF_R | XF_T)) {
+            float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (!(what & XF_R) || !(what & XF_T)) r = cur ? P.pos1[i] : P.pos0[i];
+            if (what & XF_R) {
+                r.x = fs[X.r + 3 * i];
+                r.y = fs[X.r + 3 * i + 1];
+                r.z = fs[X.r + 3 * i + 2];
+            }
+            if (what & XF_T) r.w = __int_as_float(src[X.t + i]);
+            P.pos0[i] = r;
+        }
+        if ((what & XF_V) || new_m) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (!(what & XF_V) || !new_m) v = P.vel[i];
+            if (what & XF_V) {
+                v.x = fs[X.v + 3 * i];
+                v.y = fs[X.v + 3 * i + 1];
+                v.z = fs[X.v + 3 * i + 2];
+            }
+            if (new_m) v.w = row[P.sid_m];
+            P.vel[i] = v;
+        }
+        if (what & XF_F) P.frc[i] = make_float4(fs[X.f + 3 * i], fs[X.f + 3 * i + 1], fs[X.f + 3 * i + 2], 0.f);
+        if (what & XF_S) {
+            P.sc[SC_U * N + i] = P.sid_u >= 0 ? row[P.sid_u] : 0.f;
+            P.sc[SC_W * N + i] = P.sid_w >= 0 ? row[P.sid_w] : 0.f;
+            P.sc[SC_LAP * N + i] = P.sid_lap >= 0 ? row[P.sid_lap] : 0.f;
+            P.sc[SC_K * N + i] = P.sid_k >= 0 ? row[P.sid_k] : 0.f;
+            P.sc[SC_FSQ * N + i] = P.sid_fsq >= 0 ? row[P.sid_fsq] : 0.f;
+        }
+        if (what & XF_IM)
+            for (int k = 0; k < 3; ++k) P.rim[(size_t)k * N + i] = src[X.im + 3 * i + k];
+    }
 }
 
 // ============================================================================
@@ -586,6 +750,41 @@ int dalloc(T **p, size_t n) {
     return 0;
 }
 
+// Device buffers of one owner in one allocation (an allocation costs about as
+// much as a small system's step): pointers are registered with their sizes,
+// those to be cleared first, then allocated together
+struct Arena {
+    struct Want {
+        void **p;
+        size_t bytes;
+    };
+    std::vector<Want> zeroed, plain;
+    char *base = nullptr;
+
+    template <typename T>
+    void add(T **p, size_t n, bool zero = false) {
+        *p = nullptr;
+        (zero ? zeroed : plain).push_back(Want{(void **)p, std::max<size_t>(n, 1) * sizeof(T)});
+    }
+    static size_t padded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+    int allocate() {
+        size_t total = 0, clear = 0;
+        for (const Want &w : zeroed) clear += padded(w.bytes);
+        total = clear;
+        for (const Want &w : plain) total += padded(w.bytes);
+        HIPCHECK(hipMalloc((void **)&base, total));
+        HIPCHECK(hipMemset(base, 0, clear));
+        size_t at = 0;
+        for (const std::vector<Want> *v : {&zeroed, &plain})
+            for (const Want &w : *v) {
+                *w.p = base + at;
+                at += padded(w.bytes);
+            }
+        return 0;
+    }
+};
+
 typedef void (*kfun)(const DP *);
 typedef void (*sfun)(const DP *, int);
 typedef void (*bfun)(const DP *const *, const BatchBlk *);
@@ -646,6 +845,24 @@ int f2i(float v) {
     return i;
 }
 
+// One host array's place in the packed buffer: words [at, at + n)
+struct HostSeg {
+    void *host;
+    size_t at, n;
+};
+
+// Words [lo, hi) of the packed buffer, held at buf, to or from the host
+// arrays they belong to (one thread: a core copies tens of GB/s here, and
+// starting another costs 25 us)
+void host_move(int *buf, size_t lo, size_t hi, const std::vector<HostSeg> &segs, bool into) {
+    for (const HostSeg &s : segs) {
+        const size_t b = std::max(lo, s.at), e = std::min(hi, s.at + s.n);
+        if (b >= e) continue;
+        char *h = (char *)s.host + (b - s.at) * 4, *p = (char *)(buf + (b - lo));
+        memcpy(into ? p : h, into ? h : p, (e - b) * 4);
+    }
+}
+
 bool is_pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
 
 int ilog2(int x) {
@@ -666,8 +883,15 @@ struct gmd_ctx {
     std::vector<int> boff;       // bonds per particle (CSR offsets, N + 1; empty: no bonds)
     std::vector<int2> bnd;       // (partner, bond type) per entry
     std::vector<float2> bpar;    // (r0, k) per bond type
-    std::vector<float4> h_pos, h_vel;
-    std::vector<int> h_rim;
+    char *arena = nullptr;       // every device buffer but rebuild_flag
+    hipEvent_t xev[2] = {nullptr, nullptr};   // a half of xhost is free again / has arrived
+    size_t xcap = 0;             // words of xhost
+    int *pinned = nullptr;       // pinned host memory: the published control block and saver rows, then xhost
+    int *xhost = nullptr, *xdev = nullptr;   // packed host arrays (XferSeg), in pinned and in device memory
+    Ctrl *pub = nullptr;         // the control block as of the end of the last run
+    bool pub_valid = false;      // nothing has changed the device's control block since pub was written
+    bool fetched = false;        // xhost holds the current state (gmd_batch_fetch)
+    bool all_cols = true;        // every column of the host's scalar rows has a device array
     hipStream_t stream = nullptr;
     bool own_stream = true;   // false: a replica of a gmd_batch (the batch owns the stream and the context)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -761,13 +985,11 @@ static int ctx_free(gmd_ctx *c) {
     if (!c) return 0;
     if (c->gexec) hipGraphExecDestroy(c->gexec);
     if (c->graph) hipGraphDestroy(c->graph);
-    void *ptrs[] = {c->pos0, c->pos1, c->vel, c->frc, c->rref, c->obeta, c->sc, c->rim, c->nbl, c->nbc,
-                    c->ccount, c->cmem, c->d_excl, c->d_boff, c->d_bnd, c->d_bpar,
-                    c->d_params, c->ctrl, c->partial, c->rebuild_flag, c->saver_out, c->conf_out, c->ptab, c->d_P,
-                    c->perm, c->skey, c->sorder, c->scnt, c->scur, c->tb.vel, c->tb.frc, c->tb.rref, c->tb.obeta,
-                    c->tb.sc, c->tb.rim, c->tb.perm};
-    for (void *p : ptrs)
-        if (p) hipFree(p);
+    if (c->arena) hipFree(c->arena);
+    if (c->rebuild_flag) hipFree(c->rebuild_flag);
+    for (hipEvent_t e : c->xev)
+        if (e) hipEventDestroy(e);
+    if (c->pinned) hipHostFree(c->pinned);
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->stream && c->own_stream) hipStreamDestroy(c->stream);
@@ -898,9 +1120,7 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
 
     int dev = 0;
     HTRY(hipGetDevice(&dev));
-    hipDeviceProp_t prop;
-    HTRY(hipGetDeviceProperties(&prop, dev));
-    c->cus = prop.multiProcessorCount;
+    HTRY(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, dev));
     if (shared_stream) {
         c->stream = shared_stream;
         c->own_stream = false;
@@ -978,34 +1198,27 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     size_t rows = std::max((size_t)(slots_nb + tp - 1) / tp, (size_t)8);
     if (c->nb16) rows = (rows + 1) & ~(size_t)1;
     c->nbl_len = (c->nb16 ? rows / 2 : rows) * (size_t)N * tp;
-    TRY(dalloc(&c->pos0, N));
-    TRY(dalloc(&c->pos1, N));
-    TRY(dalloc(&c->vel, N));
-    TRY(dalloc(&c->frc, N));
-    TRY(dalloc(&c->rref, N));
-    TRY(dalloc(&c->obeta, N));
-    TRY(dalloc(&c->sc, (size_t)5 * N));
-    TRY(dalloc(&c->rim, (size_t)3 * N));
-    TRY(dalloc(&c->nbl, c->nbl_len));
-    TRY(dalloc(&c->nbc, N));
-    TRY(dalloc(&c->ccount, (size_t)3 * ncells));
-    TRY(dalloc(&c->cmem, (size_t)3 * ncells * ccap));
-    TRY(dalloc(&c->d_params, c->params.size()));
-    TRY(dalloc(&c->ptab, (size_t)d.ntypes * d.ntypes));
-    TRY(dalloc(&c->ctrl, 1));
+    Arena A;
+    A.add(&c->pos0, N);
+    A.add(&c->pos1, N);
+    A.add(&c->vel, N);
+    A.add(&c->frc, N, true);
+    A.add(&c->rref, N, true);
+    A.add(&c->obeta, N, true);
+    A.add(&c->sc, (size_t)5 * N, true);
+    A.add(&c->rim, (size_t)3 * N, true);
+    A.add(&c->nbl, c->nbl_len, true);   // entries past a count stay valid indices
+    A.add(&c->nbc, N, true);
+    A.add(&c->ccount, (size_t)3 * ncells, true);
+    A.add(&c->cmem, (size_t)3 * ncells * ccap, true);
+    A.add(&c->d_params, c->params.size());
+    A.add(&c->ptab, (size_t)d.ntypes * d.ntypes);
+    A.add(&c->ctrl, 1);
     const int max_grid = std::max(c->grid_step, c->cus * 32);
-    TRY(dalloc(&c->partial, (size_t)2 * max_grid * GMD_NRED));   // two buffers: steps alternate (folded tail)
-    TRY(dalloc(&c->saver_out, (size_t)std::max(1, d.scalar_saves_per_block) * 6));
-    if (d.conf_saves_per_block > 0) {
-        TRY(dalloc(&c->conf_out, (size_t)d.conf_saves_per_block * 6 * N));
-        HTRY(hipMemset(c->conf_out, 0, (size_t)d.conf_saves_per_block * 6 * N * sizeof(float)));
-    }
-    TRY(dalloc(&c->perm, N));
-    {
-        std::vector<int> iota(N);
-        for (int i = 0; i < N; ++i) iota[i] = i;
-        HTRY(hipMemcpy(c->perm, iota.data(), (size_t)N * sizeof(int), hipMemcpyHostToDevice));
-    }
+    A.add(&c->partial, (size_t)2 * max_grid * GMD_NRED);   // two buffers: steps alternate (folded tail)
+    A.add(&c->saver_out, (size_t)std::max(1, d.scalar_saves_per_block) * 6, true);
+    if (d.conf_saves_per_block > 0) A.add(&c->conf_out, (size_t)d.conf_saves_per_block * 6 * N, true);
+    A.add(&c->perm, N);
     int side = 1;
     while (side < std::max(ncx, std::max(ncy, ncz))) side *= 2;
     if (d.nblist_kind == GMD_NBLIST_LINKED_LISTS && c->excl.empty() && c->boff.empty() && !d.utilize_niii &&
@@ -1014,44 +1227,46 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
         // particle, and the NIII half-list rule by the caller's index, so
         // systems with exclusions, bonds or UtilizeNIII keep the caller's
         // numbering)
-        TRY(dalloc(&c->skey, N));
-        TRY(dalloc(&c->sorder, N));
+        A.add(&c->skey, N);
+        A.add(&c->sorder, N);
         c->nkeys = side * side * side;
-        TRY(dalloc(&c->scnt, (size_t)c->nkeys));
-        TRY(dalloc(&c->scur, (size_t)c->nkeys));
-        TRY(dalloc(&c->tb.vel, N));
-        TRY(dalloc(&c->tb.frc, N));
-        TRY(dalloc(&c->tb.rref, N));
-        TRY(dalloc(&c->tb.obeta, N));
-        TRY(dalloc(&c->tb.sc, (size_t)5 * N));
-        TRY(dalloc(&c->tb.rim, (size_t)3 * N));
-        TRY(dalloc(&c->tb.perm, N));
+        A.add(&c->scnt, (size_t)c->nkeys);
+        A.add(&c->scur, (size_t)c->nkeys);
+        A.add(&c->tb.vel, N);
+        A.add(&c->tb.frc, N);
+        A.add(&c->tb.rref, N);
+        A.add(&c->tb.obeta, N);
+        A.add(&c->tb.sc, (size_t)5 * N);
+        A.add(&c->tb.rim, (size_t)3 * N);
+        A.add(&c->tb.perm, N);
         c->reorder_every = 400;
         c->since_reorder = 1LL << 40;
     }
-    if (!c->excl.empty()) {
-        TRY(dalloc(&c->d_excl, c->excl.size()));
-        HTRY(hipMemcpy(c->d_excl, c->excl.data(), c->excl.size() * sizeof(int), hipMemcpyHostToDevice));
-    }
+    if (!c->excl.empty()) A.add(&c->d_excl, c->excl.size());
     if (!c->boff.empty()) {
-        TRY(dalloc(&c->d_boff, c->boff.size()));
-        TRY(dalloc(&c->d_bnd, c->bnd.size()));
-        TRY(dalloc(&c->d_bpar, c->bpar.size()));
+        A.add(&c->d_boff, c->boff.size());
+        A.add(&c->d_bnd, c->bnd.size());
+        A.add(&c->d_bpar, c->bpar.size());
+    }
+    const XferSeg X((size_t)N, (size_t)std::max(0, d.nscalars));
+    A.add(&c->xdev, X.end);
+    A.add(&c->d_P, 1);
+    rc = A.allocate();
+    c->arena = A.base;
+    TRY(rc);
+    {
+        std::vector<int> iota(N);
+        for (int i = 0; i < N; ++i) iota[i] = i;
+        HTRY(hipMemcpy(c->perm, iota.data(), (size_t)N * sizeof(int), hipMemcpyHostToDevice));
+    }
+    if (!c->excl.empty())
+        HTRY(hipMemcpy(c->d_excl, c->excl.data(), c->excl.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (!c->boff.empty()) {
         HTRY(hipMemcpy(c->d_boff, c->boff.data(), c->boff.size() * sizeof(int), hipMemcpyHostToDevice));
         HTRY(hipMemcpy(c->d_bnd, c->bnd.data(), c->bnd.size() * sizeof(int2), hipMemcpyHostToDevice));
         HTRY(hipMemcpy(c->d_bpar, c->bpar.data(), c->bpar.size() * sizeof(float2), hipMemcpyHostToDevice));
     }
     HTRY(hipMemcpy(c->d_params, c->params.data(), c->params.size() * sizeof(float), hipMemcpyHostToDevice));
-    HTRY(hipMemset(c->ccount, 0, (size_t)3 * ncells * sizeof(int)));
-    HTRY(hipMemset(c->sc, 0, (size_t)5 * N * sizeof(float)));
-    HTRY(hipMemset(c->rim, 0, (size_t)3 * N * sizeof(int)));
-    HTRY(hipMemset(c->nbc, 0, (size_t)N * sizeof(int)));
-    HTRY(hipMemset(c->nbl, 0, c->nbl_len * sizeof(int)));   // entries past a count stay valid indices
-    HTRY(hipMemset(c->cmem, 0, (size_t)3 * ncells * ccap * sizeof(int)));
-    HTRY(hipMemset(c->obeta, 0, (size_t)N * sizeof(float4)));
-    HTRY(hipMemset(c->frc, 0, (size_t)N * sizeof(float4)));
-    HTRY(hipMemset(c->rref, 0, (size_t)N * sizeof(float4)));
-    HTRY(hipMemset(c->saver_out, 0, (size_t)std::max(1, d.scalar_saves_per_block) * 6 * sizeof(float)));
     Ctrl h_ctrl;
     memset(&h_ctrl, 0, sizeof h_ctrl);
     h_ctrl.shift_step = -1;
@@ -1061,9 +1276,20 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     }
     HTRY(hipMemcpy(c->ctrl, &h_ctrl, sizeof h_ctrl, hipMemcpyHostToDevice));
     for (int k = 0; k < 3; ++k) c->cur_box[k] = d.box[k];
-    c->h_pos.assign(N, make_float4(0.f, 0.f, 0.f, 0.f));
-    c->h_vel.assign(N, make_float4(0.f, 0.f, 0.f, 1.f));
-    c->h_rim.assign((size_t)3 * N, 0);
+    {
+        // the whole of a small system's arrays; a large one's go through it in
+        // two halves by turns (pinning costs about 0.25 ms a MB)
+        c->xcap = std::min(X.end, (size_t)2 * XFER_CHUNK);
+        if (c->xcap < X.end)
+            for (hipEvent_t &e : c->xev) HTRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        const size_t pub_words = (sizeof(Ctrl) / 4 + (size_t)std::max(1, d.scalar_saves_per_block) * 6 + 63) / 64 * 64;
+        HTRY(hipHostMalloc((void **)&c->pinned, (pub_words + c->xcap) * 4, hipHostMallocDefault));
+        c->pub = (Ctrl *)c->pinned;
+        c->xhost = c->pinned + pub_words;
+        int used = 0;
+        for (int sid : {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq, d.sid_m}) used += sid >= 0;
+        c->all_cols = used == d.nscalars;
+    }
 
     // ---- device parameter block ----
     DP &P = c->P;
@@ -1181,8 +1407,18 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     P.lds_build = (int)lds_b;
     P.step_grid = c->grid_step;
     P.perm = (const GMEM int *)c->perm;
+    P.xdev = (GMEM int *)c->xdev;
+    P.xhost = c->xhost;
+    P.pub = c->pinned;
+    P.nscal = d.nscalars;
+    P.sid_u = d.sid_u;
+    P.sid_w = d.sid_w;
+    P.sid_lap = d.sid_lap;
+    P.sid_k = d.sid_k;
+    P.sid_fsq = d.sid_fsq;
+    P.sid_m = d.sid_m;
 
-    TRY(dalloc(&c->d_P, 1));
+    HTRY(hipMemcpy(c->d_P, &P, sizeof(DP), hipMemcpyHostToDevice));
     c->kern = pick_kernels(d.pair_base, d.cutoff, d.integrator, d.nblist_kind);
 
     // ---- cooperative grid: all blocks must be co-resident ----
@@ -1206,129 +1442,149 @@ int gmd_destroy(gmd_ctx *ctx) {
     return ctx_free(ctx);
 }
 
+// blocks of a packing kernel
+static dim3 xfer_grid(const gmd_ctx *c, size_t n) {
+    return dim3((unsigned)std::max<size_t>(1, std::min<size_t>((n + 255) / 256, (size_t)c->cus * 8)));
+}
+
+// words of a packed buffer between host and device, on the context's stream
+static int xfer_copy(gmd_ctx *c, const int *src, int *dst, size_t n, hipMemcpyKind kind) {
+    if (n >= XFER_DMA)
+        HIPCHECK(hipMemcpyAsync(dst, src, n * 4, kind, c->stream));
+    else
+        hipLaunchKernelGGL(k_copy_words, xfer_grid(c, n / 4), dim3(256), 0, c->stream, src, dst, n);
+    return 0;
+}
+
 int gmd_upload(gmd_ctx *c, const float *r, const float *v, const float *f, const float *scalars, const int *ptype,
                const int *r_im) {
     if (!c) return fail("gmd_upload: null context");
     // work queued on the context's stream (a run, an RDF snapshot of the
     // positions) finishes before any of its buffers is overwritten
     HIPCHECK(hipStreamSynchronize(c->stream));
-    if (unpermute(c)) return -1;   // host arrays come in the caller's numbering
-    const int N = c->d.N;
+    const size_t N = c->d.N;
     const gmd_desc &d = c->d;
-    // A field merged into a packed device array whose other fields are not
-    // given keeps their current device values: positions and types share pos,
-    // velocities and masses share vel.
-    const bool new_m = scalars && d.sid_m >= 0;
-    if ((r == nullptr) != (ptype == nullptr))
-        HIPCHECK(hipMemcpy(c->h_pos.data(), c->buf0 ? c->pos1 : c->pos0, (size_t)N * sizeof(float4),
-                           hipMemcpyDeviceToHost));
-    if ((v == nullptr) != !new_m)
-        HIPCHECK(hipMemcpy(c->h_vel.data(), c->vel, (size_t)N * sizeof(float4), hipMemcpyDeviceToHost));
     if (ptype)
-        for (int i = 0; i < N; ++i) {
+        for (size_t i = 0; i < N; ++i)
             if (ptype[i] < 0 || ptype[i] >= d.ntypes)
-                return fail("gmd_upload: particle %d has type %d outside [0,%d)", i, ptype[i], d.ntypes);
-            c->h_pos[i].w = i2f(ptype[i]);
+                return fail("gmd_upload: particle %d has type %d outside [0,%d)", (int)i, ptype[i], d.ntypes);
+    if (unpermute(c)) return -1;   // host arrays come in the caller's numbering
+    c->fetched = false;
+    const XferSeg X(N, (size_t)std::max(0, d.nscalars));
+    unsigned what = 0;
+    size_t lo = X.end, hi = 0;
+    std::vector<HostSeg> segs;
+    auto take = [&](unsigned bit, const void *src, size_t at, size_t n) {
+        if (!src || n == 0) return;
+        what |= bit;
+        lo = std::min(lo, at);
+        hi = std::max(hi, at + n);
+        segs.push_back(HostSeg{const_cast<void *>(src), at, n});
+    };
+    take(XF_R, r, X.r, 3 * N);
+    take(XF_V, v, X.v, 3 * N);
+    take(XF_F, f, X.f, 3 * N);
+    take(XF_S, scalars, X.s, N * (size_t)std::max(0, d.nscalars));
+    take(XF_T, ptype, X.t, N);
+    take(XF_IM, r_im, X.im, 3 * N);
+    if (!what) return 0;
+    const int *src = c->xhost;
+    if (c->xcap >= X.end) {
+        host_move(c->xhost, 0, X.end, segs, true);
+        if (N > XFER_DIRECT) {
+            lo = lo / 4 * 4;   // (16-byte aligned in both buffers)
+            if (xfer_copy(c, c->xhost + lo, c->xdev + lo, hi - lo, hipMemcpyHostToDevice)) return -1;
+            src = c->xdev;
         }
-    if (r)
-        for (int i = 0; i < N; ++i) {
-            c->h_pos[i].x = r[3 * i];
-            c->h_pos[i].y = r[3 * i + 1];
-            c->h_pos[i].z = r[3 * i + 2];
+    } else {
+        // by halves: the host fills one while the other is on its way
+        int half = 0, turn = 0;
+        for (size_t at = lo; at < hi; at += XFER_CHUNK, half ^= 1, ++turn) {
+            const size_t n = std::min((size_t)XFER_CHUNK, hi - at);
+            int *buf = c->xhost + (size_t)half * XFER_CHUNK;
+            if (turn >= 2) HIPCHECK(hipEventSynchronize(c->xev[half]));
+            host_move(buf, at, at + n, segs, true);
+            HIPCHECK(hipMemcpyAsync(c->xdev + at, buf, n * 4, hipMemcpyHostToDevice, c->stream));
+            HIPCHECK(hipEventRecord(c->xev[half], c->stream));
         }
-    if (v)
-        for (int i = 0; i < N; ++i) {
-            c->h_vel[i].x = v[3 * i];
-            c->h_vel[i].y = v[3 * i + 1];
-            c->h_vel[i].z = v[3 * i + 2];
-        }
-    if (new_m)
-        for (int i = 0; i < N; ++i) c->h_vel[i].w = scalars[(size_t)i * d.nscalars + d.sid_m];
-    if (r || ptype) {
-        // the current buffer becomes pos0; whether the list is still valid is
-        // decided by the skin test at the start of the next run
-        c->buf0 = 0;
-        HIPCHECK(hipMemcpy(c->pos0, c->h_pos.data(), (size_t)N * sizeof(float4), hipMemcpyHostToDevice));
+        src = c->xdev;
     }
-    if (v || new_m)
-        HIPCHECK(hipMemcpy(c->vel, c->h_vel.data(), (size_t)N * sizeof(float4), hipMemcpyHostToDevice));
-    if (f) {
-        std::vector<float4> h(N);
-        for (int i = 0; i < N; ++i) h[i] = make_float4(f[3 * i], f[3 * i + 1], f[3 * i + 2], 0.f);
-        HIPCHECK(hipMemcpy(c->frc, h.data(), (size_t)N * sizeof(float4), hipMemcpyHostToDevice));
-    }
-    if (scalars) {
-        std::vector<float> h((size_t)5 * N, 0.f);
-        const int sids[5] = {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq};
-        for (int col = 0; col < 5; ++col)
-            if (sids[col] >= 0)
-                for (int i = 0; i < N; ++i) h[(size_t)col * N + i] = scalars[(size_t)i * d.nscalars + sids[col]];
-        HIPCHECK(hipMemcpy(c->sc, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice));
-    }
-    if (r_im) {
-        for (int i = 0; i < N; ++i)
-            for (int k = 0; k < 3; ++k) c->h_rim[(size_t)k * N + i] = r_im[3 * i + k];
-        HIPCHECK(hipMemcpy(c->rim, c->h_rim.data(), c->h_rim.size() * sizeof(int), hipMemcpyHostToDevice));
-    }
+    hipLaunchKernelGGL(k_pack, xfer_grid(c, N), dim3(256), 0, c->stream, (const DP *)c->d_P, c->buf0, what, src);
+    HIPCHECK(hipGetLastError());
+    // the current buffer becomes pos0; whether the list is still valid is
+    // decided by the skin test at the start of the next run
+    if (r || ptype) c->buf0 = 0;
     return 0;
 }
 
 int gmd_download(gmd_ctx *c, float *r, float *v, float *f, float *scalars, int *ptype, int *r_im) {
     if (!c) return fail("gmd_download: null context");
-    const int N = c->d.N;
+    const size_t N = c->d.N;
     const gmd_desc &d = c->d;
-    HIPCHECK(hipStreamSynchronize(c->stream));
-    std::vector<int> perm;   // internal index -> caller's index (empty: identity)
-    if (host_perm(c, perm)) return -1;
-    auto at = [&](int i) { return perm.empty() ? i : perm[i]; };
-    if (r || ptype) {
-        HIPCHECK(hipMemcpy(c->h_pos.data(), c->buf0 ? c->pos1 : c->pos0, (size_t)N * sizeof(float4),
-                           hipMemcpyDeviceToHost));
-        for (int i = 0; i < N; ++i) {
-            const int o = at(i);
-            if (r) {
-                r[3 * o] = c->h_pos[i].x;
-                r[3 * o + 1] = c->h_pos[i].y;
-                r[3 * o + 2] = c->h_pos[i].z;
-            }
-            if (ptype) ptype[o] = f2i(c->h_pos[i].w);
+    const size_t ns = (size_t)std::max(0, d.nscalars);
+    const XferSeg X(N, ns);
+    unsigned what = 0;
+    size_t lo = X.end, hi = 0;
+    auto want = [&](unsigned bit, const void *dst, size_t at, size_t n) {
+        if (!dst || n == 0) return;
+        what |= bit;
+        lo = std::min(lo, at);
+        hi = std::max(hi, at + n);
+    };
+    want(XF_R, r, X.r, 3 * N);
+    want(XF_V, v, X.v, 3 * N);
+    want(XF_F, f, X.f, 3 * N);
+    want(XF_S, scalars, X.s, N * ns);
+    want(XF_T, ptype, X.t, N);
+    want(XF_IM, r_im, X.im, 3 * N);
+    const bool whole = c->xcap >= X.end;
+    if (!c->fetched && what) {
+        const bool direct = whole && N <= XFER_DIRECT && !c->permuted;
+        hipLaunchKernelGGL(k_unpack, xfer_grid(c, N), dim3(256), 0, c->stream, (const DP *)c->d_P, c->buf0, what,
+                           direct ? c->xhost : c->xdev);
+        HIPCHECK(hipGetLastError());
+        if (whole && !direct) {
+            const size_t at = lo / 4 * 4;
+            if (xfer_copy(c, c->xdev + at, c->xhost + at, hi - at, hipMemcpyDeviceToHost)) return -1;
         }
     }
-    if (v || scalars) {
-        HIPCHECK(hipMemcpy(c->h_vel.data(), c->vel, (size_t)N * sizeof(float4), hipMemcpyDeviceToHost));
-        if (v)
-            for (int i = 0; i < N; ++i) {
-                const int o = at(i);
-                v[3 * o] = c->h_vel[i].x;
-                v[3 * o + 1] = c->h_vel[i].y;
-                v[3 * o + 2] = c->h_vel[i].z;
-            }
-    }
-    if (f) {
-        std::vector<float4> h(N);
-        HIPCHECK(hipMemcpy(h.data(), c->frc, (size_t)N * sizeof(float4), hipMemcpyDeviceToHost));
-        for (int i = 0; i < N; ++i) {
-            const int o = at(i);
-            f[3 * o] = h[i].x;
-            f[3 * o + 1] = h[i].y;
-            f[3 * o + 2] = h[i].z;
+    c->fetched = false;
+    std::vector<HostSeg> segs;
+    auto put = [&](void *dst, size_t at, size_t n) {
+        if (dst && n) segs.push_back(HostSeg{dst, at, n});
+    };
+    put(r, X.r, 3 * N);
+    put(v, X.v, 3 * N);
+    put(f, X.f, 3 * N);
+    put(ptype, X.t, N);
+    put(r_im, X.im, 3 * N);
+    std::vector<float> rows;   // columns without a device array stay as the caller has them
+    if (scalars && !c->all_cols) rows.resize(N * ns);
+    put(c->all_cols ? (void *)scalars : (void *)rows.data(), X.s, scalars ? N * ns : 0);
+    if (whole) {
+        HIPCHECK(hipStreamSynchronize(c->stream));
+        host_move(c->xhost, 0, X.end, segs, false);
+    } else if (what) {
+        // by halves: the host empties one while the other is on its way
+        auto start = [&](size_t at, int half) {
+            const size_t n = std::min((size_t)XFER_CHUNK, hi - at);
+            HIPCHECK(hipMemcpyAsync(c->xhost + (size_t)half * XFER_CHUNK, c->xdev + at, n * 4, hipMemcpyDeviceToHost,
+                                    c->stream));
+            HIPCHECK(hipEventRecord(c->xev[half], c->stream));
+            return 0;
+        };
+        if (start(lo, 0)) return -1;
+        int half = 0;
+        for (size_t at = lo; at < hi; at += XFER_CHUNK, half ^= 1) {
+            if (at + XFER_CHUNK < hi && start(at + XFER_CHUNK, half ^ 1)) return -1;
+            HIPCHECK(hipEventSynchronize(c->xev[half]));
+            host_move(c->xhost + (size_t)half * XFER_CHUNK, at, std::min(at + XFER_CHUNK, hi), segs, false);
         }
     }
-    if (scalars) {
-        std::vector<float> h((size_t)5 * N);
-        HIPCHECK(hipMemcpy(h.data(), c->sc, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-        const int sids[5] = {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq};
-        for (int col = 0; col < 5; ++col)
-            if (sids[col] >= 0)
-                for (int i = 0; i < N; ++i) scalars[(size_t)at(i) * d.nscalars + sids[col]] = h[(size_t)col * N + i];
-        if (d.sid_m >= 0)
-            for (int i = 0; i < N; ++i) scalars[(size_t)at(i) * d.nscalars + d.sid_m] = c->h_vel[i].w;
-    }
-    if (r_im) {
-        HIPCHECK(hipMemcpy(c->h_rim.data(), c->rim, c->h_rim.size() * sizeof(int), hipMemcpyDeviceToHost));
-        for (int i = 0; i < N; ++i)
-            for (int k = 0; k < 3; ++k) r_im[3 * at(i) + k] = c->h_rim[(size_t)k * N + i];
-    }
+    if (!rows.empty())
+        for (int sid : {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq, d.sid_m})
+            if (sid >= 0)
+                for (size_t i = 0; i < N; ++i) scalars[i * ns + sid] = rows[i * ns + sid];
     return 0;
 }
 
@@ -1420,30 +1676,33 @@ static int host_perm(gmd_ctx *c, std::vector<int> &perm) {
 
 // per-run set-up of one system on its stream: control block, rebuild flags,
 // saver rows, the cell grid of the starting positions and the skin test
-static int run_prepare(gmd_ctx *c, float t0, int steps) {
+// (launch = false: the caller launches that for all its replicas)
+static RunStart run_start(const gmd_ctx *c) { return RunStart{c->buf0, c->need_rebuild ? 1 : 0, c->lstep}; }
+
+// blocks of the clears at the start of a run
+static unsigned run_begin_blocks(const gmd_ctx *c, int steps) {
+    const int cells = c->d.nblist_kind == GMD_NBLIST_LINKED_LISTS ? 3 * c->P.ncells : 0;
+    const int rows = c->d.scalar_save_every > 0 ? c->d.scalar_saves_per_block * 6 : 0;
+    return (unsigned)std::max(1, std::min((std::max(steps + 2, std::max(cells, rows)) + 255) / 256, c->cus * 8));
+}
+
+static int run_prepare(gmd_ctx *c, float t0, int steps, bool launch = true) {
     if (steps < 0) return fail("gmd_run: steps must be non-negative");
     if (ensure_flags(c, steps)) return -1;
     if (c->reorder_every > 0 && steps > 0 && c->since_reorder >= c->reorder_every)
         if (reorder(c)) return -1;
-    hipStream_t st = c->stream;
-    const DP *dP = c->d_P;
-    HIPCHECK(hipMemsetAsync(c->rebuild_flag, 0, (size_t)(steps + 2) * sizeof(int), st));
-    if (c->need_rebuild) {
-        int one = 1;
-        HIPCHECK(hipMemcpyAsync(c->rebuild_flag, &one, sizeof(int), hipMemcpyHostToDevice, st));
-    }
-    if (c->d.scalar_save_every > 0)
-        HIPCHECK(hipMemsetAsync(c->saver_out, 0, (size_t)c->d.scalar_saves_per_block * 6 * sizeof(float), st));
+    c->pub_valid = false;
+    c->fetched = false;
     if (!c->ptab_ready) {
-        hipLaunchKernelGGL(k_pair_table, dim3(1), dim3(64), 0, st, dP);
+        hipLaunchKernelGGL(k_pair_table, dim3(1), dim3(64), 0, c->stream, (const DP *)c->d_P);
         c->ptab_ready = true;
     }
-    hipLaunchKernelGGL(k_begin_run, dim3(1), dim3(64), 0, st, c->ctrl, steps, t0, c->buf0, c->lstep);
-    if (c->d.nblist_kind == GMD_NBLIST_LINKED_LISTS)
-        hipLaunchKernelGGL(k_cells_clear, dim3(std::max(1, std::min((3 * c->P.ncells + 255) / 256, c->cus * 8))),
-                           dim3(256), 0, st, dP);
+    if (!launch) return 0;
+    hipStream_t st = c->stream;
+    const DP *dP = c->d_P;
+    hipLaunchKernelGGL(k_run_begin, dim3(run_begin_blocks(c, steps)), dim3(256), 0, st, dP, steps, t0,
+                       run_start(c));
     hipLaunchKernelGGL(k_run_setup, dim3(c->grid_aux), dim3(c->block), 0, st, dP);
-    hipLaunchKernelGGL(k_setup_finish, dim3(1), dim3(64), 0, st, dP);
     HIPCHECK(hipGetLastError());
     return 0;
 }
@@ -1454,8 +1713,8 @@ static int run_complete(gmd_ctx *c, int steps) {
     c->lstep += steps;
     c->since_reorder += steps;
     c->need_rebuild = false;
-    Ctrl h;
-    HIPCHECK(hipMemcpy(&h, c->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    const Ctrl &h = *c->pub;   // published by the run (k_run_publish), on the host since the stream drained
+    c->pub_valid = true;
     if (c->P.npt)
         for (int k = 0; k < 3; ++k) c->cur_box[k] = h.npt[h.nsteps & 1][3 + k];
     if (h.cell_overflow > 0)
@@ -1499,8 +1758,9 @@ static int run_impl(gmd_ctx *c, float t0, int steps) {
         HIPCHECK(hipGetLastError());
     }
     HIPCHECK(hipEventRecord(c->ev1, st));
-    HIPCHECK(hipEventSynchronize(c->ev1));
+    hipLaunchKernelGGL(k_run_publish, dim3(1), dim3(256), 0, st, dP);
     HIPCHECK(hipGetLastError());
+    HIPCHECK(hipStreamSynchronize(st));
     HIPCHECK(hipEventElapsedTime(&c->last_ms, c->ev0, c->ev1));
     return run_complete(c, steps);
 }
@@ -1542,6 +1802,7 @@ int gmd_profile_steps(gmd_ctx *c, float time_zero, int steps, float *step_ms, fl
         for (int s = 0; s < n; ++s)
             hipLaunchKernelGGL(c->kern.step, dim3(c->grid_step), dim3(c->block), c->lds_step, st, dP, s);
         hipEventRecord(ev[1], st);
+        hipLaunchKernelGGL(k_run_publish, dim3(1), dim3(256), 0, st, dP);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
             rc = fail("gmd_profile_steps: launch failed");
     }
@@ -1563,10 +1824,21 @@ int gmd_last_run_ms(gmd_ctx *c, float *ms) {
     return 0;
 }
 
+// the control block: as the last run published it, or from the device
+static int read_ctrl(gmd_ctx *c, Ctrl &h) {
+    if (c->pub_valid) {
+        h = *c->pub;
+        return 0;
+    }
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    HIPCHECK(hipMemcpy(&h, c->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    return 0;
+}
+
 int gmd_read_nbflag(gmd_ctx *c, int nbflag[3]) {
     if (!c || !nbflag) return fail("gmd_read_nbflag: null argument");
     Ctrl h;
-    HIPCHECK(hipMemcpy(&h, c->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (read_ctrl(c, h)) return -1;
     for (int k = 0; k < 3; ++k) nbflag[k] = h.nbflag[k];
     return 0;
 }
@@ -1697,9 +1969,8 @@ int gmd_force_rebuild(gmd_ctx *c) {
 
 int gmd_get_thermostat(gmd_ctx *c, float state[2]) {
     if (!c || !state) return fail("gmd_get_thermostat: null argument");
-    HIPCHECK(hipStreamSynchronize(c->stream));
     Ctrl h;
-    HIPCHECK(hipMemcpy(&h, c->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (read_ctrl(c, h)) return -1;
     state[0] = h.xi;
     state[1] = h.ksum;
     return 0;
@@ -1709,15 +1980,15 @@ int gmd_set_thermostat(gmd_ctx *c, const float state[2]) {
     if (!c || !state) return fail("gmd_set_thermostat: null argument");
     HIPCHECK(hipStreamSynchronize(c->stream));
     HIPCHECK(hipMemcpy(&c->ctrl->xi, state, 2 * sizeof(float), hipMemcpyHostToDevice));
+    c->pub_valid = false;
     return 0;
 }
 
 int gmd_get_npt_state(gmd_ctx *c, float state[6]) {
     if (!c || !state) return fail("gmd_get_npt_state: null argument");
     if (!c->P.npt) return fail("gmd_get_npt_state: the context does not run NPT_Atomic");
-    HIPCHECK(hipStreamSynchronize(c->stream));
     Ctrl h;
-    HIPCHECK(hipMemcpy(&h, c->ctrl, sizeof h, hipMemcpyDeviceToHost));
+    if (read_ctrl(c, h)) return -1;
     for (int k = 0; k < 6; ++k) state[k] = h.npt[h.nsteps & 1][k];
     return 0;
 }
@@ -1733,6 +2004,7 @@ int gmd_set_npt_state(gmd_ctx *c, const float state[6]) {
     for (int b = 0; b < 2; ++b)
         for (int k = 0; k < 6; ++k) both[b][k] = state[k];
     HIPCHECK(hipMemcpy(&c->ctrl->npt[0][0], both, sizeof both, hipMemcpyHostToDevice));
+    c->pub_valid = false;
     for (int k = 0; k < 3; ++k) c->cur_box[k] = state[3 + k];
     return 0;
 }
@@ -1740,8 +2012,11 @@ int gmd_set_npt_state(gmd_ctx *c, const float state[6]) {
 int gmd_read_scalar_output(gmd_ctx *c, float *out) {
     if (!c || !out) return fail("gmd_read_scalar_output: null argument");
     if (c->d.scalar_save_every <= 0) return fail("gmd_read_scalar_output: no scalar saver configured");
-    HIPCHECK(hipMemcpy(out, c->saver_out, (size_t)c->d.scalar_saves_per_block * 6 * sizeof(float),
-                       hipMemcpyDeviceToHost));
+    const size_t bytes = (size_t)c->d.scalar_saves_per_block * 6 * sizeof(float);
+    if (c->pub_valid)
+        memcpy(out, c->pub + 1, bytes);   // published after the control block
+    else
+        HIPCHECK(hipMemcpy(out, c->saver_out, bytes, hipMemcpyDeviceToHost));
     return 0;
 }
 
@@ -2105,6 +2380,7 @@ struct gmd_batch {
     size_t lds = 0;
     Kernels kern = {nullptr, nullptr, nullptr, nullptr};
     std::vector<BatchBlk> h_blk;
+    RunStart *h_start = nullptr;   // pinned: what each replica's run starts from (read by the kernels)
     BatchBlk *d_blk = nullptr;
     const DP **d_Ps = nullptr;
     hipGraph_t graph = nullptr;
@@ -2118,6 +2394,7 @@ static int batch_free(gmd_batch *b) {
     if (b->gexec) hipGraphExecDestroy(b->gexec);
     if (b->graph) hipGraphDestroy(b->graph);
     for (gmd_ctx *c : b->reps) ctx_free(c);
+    if (b->h_start) hipHostFree(b->h_start);
     if (b->d_blk) hipFree(b->d_blk);
     if (b->d_Ps) hipFree(b->d_Ps);
     if (b->ev0) hipEventDestroy(b->ev0);
@@ -2235,6 +2512,7 @@ int gmd_batch_create(const gmd_desc *descs, int nrep, const int *blocks, int dri
     BTRY(hipMemcpy(b->d_blk, b->h_blk.data(), b->h_blk.size() * sizeof(BatchBlk), hipMemcpyHostToDevice));
     std::vector<const DP *> ps(nrep);
     for (int r = 0; r < nrep; ++r) ps[r] = b->reps[r]->d_P;
+    BTRY(hipHostMalloc((void **)&b->h_start, (size_t)nrep * sizeof(RunStart), hipHostMallocDefault));
     BTRY(hipMalloc((void **)&b->d_Ps, nrep * sizeof(DP *)));
     BTRY(hipMemcpy(b->d_Ps, ps.data(), nrep * sizeof(DP *), hipMemcpyHostToDevice));
 #undef BTRY
@@ -2260,16 +2538,29 @@ int gmd_batch_context(gmd_batch *b, int rep, gmd_ctx **out) {
 
 int gmd_batch_run(gmd_batch *b, float time_zero, int steps) {
     if (!b) return fail("gmd_batch_run: null batch");
-    for (size_t r = 0; r < b->reps.size(); ++r)
-        if (run_prepare(b->reps[r], time_zero, steps)) {
+    const unsigned nrep = (unsigned)b->reps.size();
+    unsigned gx = 1, gs = 1;
+    for (size_t r = 0; r < b->reps.size(); ++r) {
+        gmd_ctx *c = b->reps[r];
+        if (run_prepare(c, time_zero, steps, false)) {
             std::string msg = g_err;
             return fail("gmd_batch_run: replica %d: %s", (int)r, msg.c_str());
         }
-    // the rebuild-flag arrays may have been reallocated by the preparation
+        b->h_start[r] = run_start(c);
+        gx = std::max(gx, run_begin_blocks(c, steps));
+        gs = std::max(gs, (unsigned)c->grid_aux);
+    }
+    // the rebuild-flag arrays may have been reallocated by the preparation;
+    // the set-up of all replicas in three launches
     hipStream_t st = b->stream;
-    HIPCHECK(hipEventRecord(b->ev0, st));
     const DP *const *Ps = b->d_Ps;
     const BatchBlk *blk = b->d_blk;
+    hipLaunchKernelGGL(k_batch_begin, dim3(gx, nrep), dim3(256), 0, st, Ps, steps, time_zero,
+                       (const RunStart *)b->h_start);
+    hipLaunchKernelGGL(k_batch_setup, dim3(gs, nrep), dim3(256), 0, st, Ps);
+    hipLaunchKernelGGL(k_batch_setup_finish, dim3((nrep + 255) / 256), dim3(256), 0, st, Ps, (int)nrep);
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipEventRecord(b->ev0, st));
     if (b->driver == GMD_BATCH_PERSISTENT) {
         void *args[] = {(void *)&Ps, (void *)&blk};
         HIPCHECK(hipLaunchCooperativeKernel((const void *)b->kern.bpers, dim3(b->grid), dim3(b->block), args,
@@ -2288,14 +2579,37 @@ int gmd_batch_run(gmd_batch *b, float time_zero, int steps) {
         for (int k = 0; k < launches; ++k) HIPCHECK(hipGraphLaunch(b->gexec, st));
     }
     HIPCHECK(hipEventRecord(b->ev1, st));
-    HIPCHECK(hipEventSynchronize(b->ev1));
+    hipLaunchKernelGGL(k_batch_publish, dim3(nrep), dim3(256), 0, st, Ps);
     HIPCHECK(hipGetLastError());
+    HIPCHECK(hipStreamSynchronize(st));
     HIPCHECK(hipEventElapsedTime(&b->last_ms, b->ev0, b->ev1));
     for (size_t r = 0; r < b->reps.size(); ++r)
         if (run_complete(b->reps[r], steps)) {
             std::string msg = g_err;
             return fail("gmd_batch_run: replica %d: %s", (int)r, msg.c_str());
         }
+    return 0;
+}
+
+int gmd_batch_fetch(gmd_batch *b) {
+    if (!b) return fail("gmd_batch_fetch: null batch");
+    // (replicas on one stream: earlier work is done when these run)
+    HIPCHECK(hipStreamSynchronize(b->stream));
+    const unsigned nrep = (unsigned)b->reps.size();
+    unsigned gx = 1;
+    for (size_t r = 0; r < b->reps.size(); ++r) {
+        b->h_start[r].buf0 = b->reps[r]->buf0;   // the buffer that holds the positions
+        gx = std::max(gx, xfer_grid(b->reps[r], b->reps[r]->d.N).x);
+    }
+    for (const gmd_ctx *c : b->reps)
+        if (c->xcap < XferSeg((size_t)c->d.N, (size_t)std::max(0, c->d.nscalars)).end)
+            return 0;   // a large replica: each is brought by its own gmd_download
+    hipLaunchKernelGGL(k_batch_unpack, dim3(gx, nrep), dim3(256), 0, b->stream, (const DP *const *)b->d_Ps,
+                       (const RunStart *)b->h_start);
+    hipLaunchKernelGGL(k_batch_fetch, dim3(gx, nrep), dim3(256), 0, b->stream, (const DP *const *)b->d_Ps);
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipStreamSynchronize(b->stream));
+    for (gmd_ctx *c : b->reps) c->fetched = true;
     return 0;
 }
 

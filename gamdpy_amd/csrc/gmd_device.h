@@ -163,6 +163,22 @@ struct DP {
     int lds_pp, lds_red, lds_build;   // byte offsets into dynamic LDS
     int step_grid;             // blocks of the step kernel (partial sums to reduce)
     const GMEM int *perm;      // internal index -> index in the caller's order (particles are kept in cell order)
+    // the host's arrays: a packed copy of them in device memory (xdev) and in
+    // pinned host memory (xhost), the words of each array one after another
+    // (XferSeg), and the run's control block and saver rows as the host reads
+    // them (pub, pinned)
+    GMEM int *xdev;
+    int *xhost, *pub;
+    int nscal, sid_u, sid_w, sid_lap, sid_k, sid_fsq, sid_m;   // scalar columns of the host's rows (-1: none)
+};
+
+// The host arrays as segments of a packed buffer of 4-byte words: r, v, f
+// (N, 3), scalars (N, nscal), types (N), images (N, 3)
+enum { XF_R = 1, XF_V = 2, XF_F = 4, XF_S = 8, XF_T = 16, XF_IM = 32, XF_ALL = 63 };
+struct XferSeg {
+    size_t r, v, f, s, t, im, end;
+    __host__ __device__ XferSeg(size_t N, size_t ns)
+        : r(0), v(3 * N), f(6 * N), s(9 * N), t((9 + ns) * N), im((10 + ns) * N), end((13 + ns) * N) {}
 };
 
 // ---------------------------------------------------------------------------

@@ -282,6 +282,10 @@ int gmd_batch_size(gmd_batch *batch, int *nrep, int *grid);
 int gmd_batch_context(gmd_batch *batch, int rep, gmd_ctx **out);
 /* 'steps' steps of every replica (Simulation.integrate_self per replica) */
 int gmd_batch_run(gmd_batch *batch, float time_zero, int steps);
+/* Bring the state of every replica to the host in one go: the next
+ * gmd_download of each replica (before it is run or uploaded again) only
+ * copies it. */
+int gmd_batch_fetch(gmd_batch *b);
 int gmd_batch_last_run_ms(gmd_batch *batch, float *ms);
 
 /* Differentiable NVE trajectory (no counterpart in the reference; it adds
