@@ -109,7 +109,7 @@ __device__ __forceinline__ void run_setup(const DP &P) {
         // each particle into [-L/2, L/2], where it then stays)
         if (fabsf(r.x) * 2.0f > L0 || fabsf(r.y) * 2.0f > L1 || fabsf(r.z) * 2.0f > L2)
             P.ctrl->unwrapped = 1;
-        if (P.nblist_kind == 1) cell_insert(P, 0, i, r.x, r.y, r.z, L0, L1, L2);
+        if (P.nblist_kind == 1) cell_insert(P, 0, i, r.x, r.y, r.z, L0, L1, L2, 1.0f / L0, 1.0f / L1, 1.0f / L2);
     }
 }
 
