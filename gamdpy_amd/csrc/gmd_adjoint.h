@@ -326,11 +326,9 @@ __global__ void __launch_bounds__(256) k_adj_rdf_grad_list(AdjK K, const float4 
             az += sc * dz;
         }
     }
-    for (int mm = 1; mm < K.tp; mm <<= 1) {
-        ax += __shfl_xor(ax, mm, 64);
-        ay += __shfl_xor(ay, mm, 64);
-        az += __shfl_xor(az, mm, 64);
-    }
+    ax = group_sum(ax, K.tp);
+    ay = group_sum(ay, K.tp);
+    az = group_sum(az, K.tp);
     if (i < K.N && tl == 0) out[i] = make_float4(ax, ay, az, 0.f);
 }
 

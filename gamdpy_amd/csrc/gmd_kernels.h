@@ -755,15 +755,13 @@ __device__ __forceinline__ void particle_forces(const DP &P, const StepInfo &I, 
             }
         }
     }
-    for (int mm = 1; mm < tp; mm <<= 1) {
-        fx += __shfl_xor(fx, mm, 64);
-        fy += __shfl_xor(fy, mm, 64);
-        fz += __shfl_xor(fz, mm, 64);
-        if (SCAL) {
-            uu += __shfl_xor(uu, mm, 64);
-            ww += __shfl_xor(ww, mm, 64);
-            if (LAP) ll += __shfl_xor(ll, mm, 64);
-        }
+    fx = group_sum(fx, tp);
+    fy = group_sum(fy, tp);
+    fz = group_sum(fz, tp);
+    if (SCAL) {
+        uu = group_sum(uu, tp);
+        ww = group_sum(ww, tp);
+        if (LAP) ll = group_sum(ll, tp);
     }
     if (P.boff) bond_terms(P, pos, i, ri, L0, L1, L2, fx, fy, fz, uu, ww, ll);
     f6[0] = fx;
@@ -882,25 +880,30 @@ __device__ __forceinline__ float lane_f(float v, int l) {
 // levels halve the set of values a lane carries (eight slots, the last two
 // zero): after them lane l holds a partial of slot l >> 3 over the eight
 // lanes that differ from it in bits 3-5, and three more levels complete it.
-// The total of slot c is then in lanes 8c .. 8c + 7 (10 shuffles instead of
-// 36 for six separate reductions).
+// The total of slot c is then in lanes 8c .. 8c + 7 (10 exchanges instead of
+// 36 for six separate reductions; the swaps across halves and rows are a
+// level's exchange and selection in one).
 __device__ __forceinline__ float wave_sum6(float a0, float a1, float a2, float a3, float a4, float a5) {
-    const int lane = threadIdx.x & 63;
-    const bool h5 = (lane & 32) != 0, h4 = (lane & 16) != 0, h3 = (lane & 8) != 0;
+    const bool h3 = (threadIdx.x & 8) != 0;
+    // sum of x in the lower half or even rows, of y in the others
+    auto halve = [](auto m, float x, float y) {
+        int a = __float_as_int(x), b = __float_as_int(y);
+        lane_swap<decltype(m)::value>(a, b);
+        return __int_as_float(a) + __int_as_float(b);
+    };
+    constexpr std::integral_constant<int, 32> half{};
+    constexpr std::integral_constant<int, 16> row{};
     // level 32: lanes below 32 keep slots 0-3, the others slots 4-7
-    const float y0 = (h5 ? a4 : a0) + __shfl_xor(h5 ? a0 : a4, 32, 64);
-    const float y1 = (h5 ? a5 : a1) + __shfl_xor(h5 ? a1 : a5, 32, 64);
-    const float y2 = (h5 ? 0.f : a2) + __shfl_xor(h5 ? a2 : 0.f, 32, 64);
-    const float y3 = (h5 ? 0.f : a3) + __shfl_xor(h5 ? a3 : 0.f, 32, 64);
+    const float y0 = halve(half, a0, a4), y1 = halve(half, a1, a5);
+    const float y2 = halve(half, a2, 0.f), y3 = halve(half, a3, 0.f);
     // level 16: keep two of the four
-    const float z0 = (h4 ? y2 : y0) + __shfl_xor(h4 ? y0 : y2, 16, 64);
-    const float z1 = (h4 ? y3 : y1) + __shfl_xor(h4 ? y1 : y3, 16, 64);
+    const float z0 = halve(row, y0, y2), z1 = halve(row, y1, y3);
     // level 8: keep one
-    float w = (h3 ? z1 : z0) + __shfl_xor(h3 ? z0 : z1, 8, 64);
-    w += __shfl_xor(w, 4, 64);
-    w += __shfl_xor(w, 2, 64);
-    w += __shfl_xor(w, 1, 64);
-    return w;
+    const int give = __float_as_int(h3 ? z0 : z1);
+    float w = (h3 ? z1 : z0) + __int_as_float(row_xor_i<8>(give));
+    w = xor_sum<4>(w);
+    w = xor_sum<2>(w);
+    return xor_sum<1>(w);
 }
 
 // Test the staged candidates cand[0, ce) against each particle of the cell:
@@ -1223,15 +1226,8 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
             myv = P.vel[myi];
         }
         // stencil-order offsets of every cell's members
-        int ia = na, ib = nb;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int ta = __shfl_up(ia, o, 64), tb = __shfl_up(ib, o, 64);
-            if (lane >= o) {
-                ia += ta;
-                ib += tb;
-            }
-        }
+        const int ia = wave_prefix(na);
+        int ib = wave_prefix(nb);
         const int totA = lane_i(ia, 63);
         ib += totA;
         const int M = lane_i(ib, 63);
@@ -1243,9 +1239,14 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
         for (int done = 0; done < M;) {
             const bool ina = offa >= done && ia - done <= LL_IDXCAP;
             const bool inb = sb < 125 && offb >= done && ib - done <= LL_IDXCAP;
-            int pe = max(ina ? ia : done, inb ? ib : done);
+            // the members up to the last cell of the pass: all of them as a
+            // rule, else the largest prefix sum of its cells
+            int pe = M;
+            if (M - done > LL_IDXCAP) {
+                pe = max(ina ? ia : done, inb ? ib : done);
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) pe = max(pe, __shfl_xor(pe, o, 64));
+                for (int o = 32; o > 0; o >>= 1) pe = max(pe, __shfl_xor(pe, o, 64));
+            }
             const int ce = pe - done;
             wave_sync_lds();
             if (ina && na > 0) stage_cell_members(cmem + (size_t)nca * P.ccap, na, idx + (offa - done));
@@ -1501,9 +1502,10 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
         }
         auto total = [&](const float (&v)[4]) {
             float t = (v[0] + v[2]) + (v[1] + v[3]);
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-            return t;
+            t = xor_sum<8>(t);
+            t = xor_sum<4>(t);
+            t = xor_sum<2>(t);
+            return xor_sum<1>(t);
         };
         float sx = total(fx), sy = total(fy), sz = total(fz), su = total(uu), sw = total(ww);
         float sl = lap ? total(ll) : 0.f;
