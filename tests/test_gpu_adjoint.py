@@ -148,3 +148,28 @@ def test_differentiable_md_workload_vs_finite_differences():
             ad = g[a, b] + (g[b, a] if a != b else 0.0)
             print(which, a, b, ad, fd)
             assert abs(ad - fd) <= 5e-2 * abs(fd) + 1e-12
+
+
+@pytest.mark.parametrize("N,shuffled", [(257, False), (300, True), (1023, True), (1025, False)])
+def test_forward_histogram_at_list_tile_edges(N, shuffled):
+    """Sizes around the list builds' tiles (256 and 1024 positions), with and
+    without a numbering that follows space, hot enough that lists are rebuilt
+    between the checkpoints; float32 against float64 over 30 steps as above."""
+    rng = np.random.default_rng(N)
+    n = int(np.ceil((N / 4) ** (1 / 3)))
+    r, box = gp.make_lattice(gp.unit_cells.FCC, [n, n, n], rho=1.0 * 4 * n ** 3 / N)
+    keep = rng.permutation(len(r))[:N]
+    r = r[keep if shuffled else np.sort(keep)] + rng.uniform(-0.03, 0.03, (N, 3))
+    conf = gp.Configuration(D=3)
+    conf['r'] = r.astype(np.float32)
+    conf.simbox = gp.Orthorhombic(3, np.float32(box))
+    conf['m'] = 1.0
+    conf.ptype[rng.permutation(N)[:N // 5]] = 1
+    conf.randomize_velocities(temperature=3.0, seed=1)
+    traj = dict(dt=0.004, nsteps=30, ckpt_every=15, rdf_every=10, bins=50, rmax=2.5, width=0.03)
+    m, cut = _model(conf, traj)
+    H = m.histogram(torch.tensor(conf['r']), torch.tensor(KA_SIG, dtype=torch.float64),
+                    torch.tensor(KA_EPS, dtype=torch.float64)).numpy()
+    Hc = _c_hist(conf, np.array(KA_SIG), np.array(KA_EPS), cut, traj)
+    print(N, np.abs(H - Hc).max(), Hc.max())
+    assert np.abs(H - Hc).max() <= 1e-3 * Hc.max()
