@@ -277,28 +277,195 @@ __global__ void __launch_bounds__(256) k_pack(const DP *__restrict__ Pp, int cur
 // ============================================================================
 // Radial distribution (calculator_radial_distribution.py:76-109)
 // ============================================================================
-#define RDF_TILE 256     // particles per tile (one block of threads; one staged LDS tile)
-#define RDF_CHUNK 64     // particles per chunk (one wavefront)
+#define RDF_CHUNK 64     // particles per chunk: the i of a wavefront, one a lane
+#define RDF_GROUP 16     // particles per group: the j a chunk is tested and counted against at a time
+#define RDF_PAD 1e30f    // coordinate of the places past the last particle (-: in the role of i)
+#define RDF_LDS_SPARE (4096 + 64)   // of 64 KB a block: beyond the histogram and thresholds
+#define RDF_MAX_CELL 32  // sorting cells per dimension
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+// constant for the kernel, so that an address the same in every lane becomes
+// a scalar load
+typedef const __attribute__((address_space(4))) f32x16 *rdf_quad_t;
 
 struct RdfP {
-    int N, nt, bins, nchunks, ntiles;
-    long long npairs;          // tile pairs I <= J
-    float L0, L1, L2, inv_bw;
-    // per chunk c: [4c] centre and [4c+1] half extents of its box in the
-    // minimum-image frame of its first particle, [4c+2] / [4c+3] lower and
-    // upper corners of its raw coordinates
-    const GMEM float4 *cbox;
-    float skip2;               // chunk pairs whose distance lower bound exceeds this are skipped
-    cpos_t pos;
-    const GMEM int *ptype;     // nullptr: type from pos.w
+    int N, nt, bins, nchunks;
+    int unit, nrow, nper;      // groups a wavefront tests at a time; row pairs; units a row pair
+    float L0, L1, L2, rL0, rL1, rL2;   // box and 1 / box
+    float inv_bw, edge;        // bin estimate and the fraction from which it is settled by the threshold
+    // per group g: [4g] centre and [4g+1] half extents of its box in the
+    // minimum-image frame of its first particle, [4g+2] / [4g+3] lower and
+    // upper corners of its raw coordinates; per chunk the same in cbox
+    const GMEM float4 *gbox, *cbox;
+    float skip2;               // chunk-group pairs whose distance lower bound exceeds this are skipped
+    cpos_t pos;                // sorted and padded to whole chunks; w: byte offset of the type's histogram
     const GMEM float *thr;     // thr[k] k = 0..bins: smallest d^2 of bin >= k (thr[bins]: first excluded)
     GMEM unsigned *part;       // [gridDim][nt][nt][bins]
 };
 
-// Image of every pair of two chunks in one dimension.  fl(xj - xi) lies in
-// [fl(jlo - ihi), fl(jhi - ilo)] because rounding is monotone, so the
+// ---- sorting -----------------------------------------------------------------
+// The histogram does not depend on the numbering, its cost does: particles
+// sorted along a Hilbert curve through coarse cells (Skilling's transform, AIP
+// Conf. Proc. 707, 381 (2004)) make chunks and groups compact,
+// so that more of their pairs are skipped whole and few need the per-pair
+// minimum image.  k_rdf_count gives each particle its cell and its place among
+// the cell's particles (in any order), k_rdf_starts the cells' first places,
+// k_rdf_place writes the sorted positions.
+struct RdfSort {
+    int N, ncell, npad, nt_bytes;   // npad: N up to whole chunks; nt_bytes: histogram bytes a type
+    float rL0, rL1, rL2;
+    const float4 *pos;              // x, y, z, type bits; or null:
+    const float *r;                 // (N, 3) as the host gave them, with
+    const int *ptype;               // their types (also instead of pos.w if given)
+    int *count;                     // [ncell^3], zero on entry
+    int2 *key;                      // [N] cell and place
+    float4 *out;                    // [npad]
+};
+
+__device__ __forceinline__ float4 rdf_read(const RdfSort &S, int i) {
+    if (!S.pos) {
+        const GMEM float *r = (const GMEM float *)S.r;
+        return make_float4(r[3 * i], r[3 * i + 1], r[3 * i + 2], __int_as_float(((const GMEM int *)S.ptype)[i]));
+    }
+    float4 p = ((cpos_t)S.pos)[i];
+    if (S.ptype) p.w = __int_as_float(((const GMEM int *)S.ptype)[i]);
+    return p;
+}
+
+// bits of v (up to five) three apart
+__device__ __forceinline__ int rdf_spread(int v) {
+    v = (v | (v << 8)) & 0x100f;
+    v = (v | (v << 4)) & 0x10c3;
+    return (v | (v << 2)) & 0x1249;
+}
+
+__global__ void __launch_bounds__(256) k_rdf_count(RdfSort S) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= S.N) return;
+    const float4 p = rdf_read(S, i);
+    // any position gets some cell: not a number and infinities the first
+    auto cell = [&](float x, float rL) {
+        float u = x * rL;
+        u = (u - floorf(u)) * (float)S.ncell;
+        return u > 0.f ? min((int)fminf(u, 1e6f), S.ncell - 1) : 0;
+    };
+    int c[3] = {cell(p.x, S.rL0), cell(p.y, S.rL1), cell(p.z, S.rL2)};
+    // transpose of the Hilbert index, from the most significant bit down:
+    // each bit of a coordinate reflects or exchanges the lower bits of the first
+    for (int b = S.ncell >> 1; b > 1; b >>= 1) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const int t = c[d] & b ? b - 1 : (c[0] ^ c[d]) & (b - 1);
+            if (!(c[d] & b)) c[d] ^= t;
+            c[0] ^= t;
+        }
+    }
+    c[1] ^= c[0];
+    c[2] ^= c[1];
+    int t = 0;
+    for (int b = S.ncell >> 1; b > 1; b >>= 1)
+        if (c[2] & b) t ^= b - 1;
+    const int k = rdf_spread(c[0] ^ t) << 2 | rdf_spread(c[1] ^ t) << 1 | rdf_spread(c[2] ^ t);
+    ((GMEM int2 *)S.key)[i] = make_int2(k, atomicAdd(S.count + k, 1));
+}
+
+// exclusive prefix sum of n counts in place, one block of 1024
+__global__ void __launch_bounds__(1024) k_rdf_starts(int *count_p, int n) {
+    GMEM int *count = (GMEM int *)count_p;
+    __shared__ int wsum[16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int per = (n + 1023) / 1024, k0 = threadIdx.x * per;
+    int s = 0;
+    for (int k = k0; k < min(n, k0 + per); ++k) s += count[k];
+    int inc = s;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    if (lane == 63) wsum[wid] = inc;
+    __syncthreads();
+    int base = inc - s;
+    for (int x = 0; x < wid; ++x) base += wsum[x];
+    for (int k = k0; k < min(n, k0 + per); ++k) {
+        const int c = count[k];
+        count[k] = base;
+        base += c;
+    }
+}
+
+// the position and histogram offset of particle i, or what fills a last chunk
+__device__ __forceinline__ float4 rdf_entry(const RdfSort &S, int i) {
+    float4 p = make_float4(RDF_PAD, RDF_PAD, RDF_PAD, 0.f);
+    if (i < S.N) {
+        p = rdf_read(S, i);
+        p.w = __int_as_float(__float_as_int(p.w) * S.nt_bytes);
+    }
+    return p;
+}
+
+__global__ void __launch_bounds__(256) k_rdf_place(RdfSort S) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= S.npad) return;
+    const float4 p = rdf_entry(S, i);
+    int to = i;
+    if (i < S.N) {
+        const int2 k = ((const GMEM int2 *)S.key)[i];
+        to = ((const GMEM int *)S.count)[k.x] + k.y;
+    }
+    ((GMEM float4 *)S.out)[to] = p;
+}
+
+// Boxes of each group and chunk (a wavefront a chunk): centre and half
+// extents in the minimum-image frame of its first particle (tight for one
+// that straddles the periodic boundary), with a rounding margin, and the raw
+// coordinate bounds.  A group without particles gets a negative extent.
+// place: not sorted, so the positions are laid out here.
+__global__ void __launch_bounds__(256) k_rdf_boxes(RdfSort S, int place, float L0, float L1, float L2,
+                                                   float4 *gbox_p, float4 *cbox_p) {
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, N = S.N;
+    const int i0 = c * RDF_CHUNK, i = i0 + lane;
+    if (i >= S.npad) return;
+    GMEM float4 *pos = (GMEM float4 *)S.out;
+    const float4 own = place ? rdf_entry(S, i) : pos[i];
+    if (place) pos[i] = own;
+    for (int level = 0; level < 2; ++level) {
+        const int w = level ? RDF_CHUNK : RDF_GROUP;
+        const int b0 = i0 + (lane & ~(w - 1)), l0 = min(b0, N - 1) - i0;   // (a chunk has a particle)
+        const float4 r0 = make_float4(__shfl(own.x, l0, 64), __shfl(own.y, l0, 64), __shfl(own.z, l0, 64), 0.f);
+        const float4 r = i < N ? own : r0;
+        float lo[3] = {mic1(r.x - r0.x, L0), mic1(r.y - r0.y, L1), mic1(r.z - r0.z, L2)};
+        float hi[3] = {lo[0], lo[1], lo[2]};
+        float rlo[3] = {r.x, r.y, r.z};
+        float rhi[3] = {r.x, r.y, r.z};
+        for (int k = 0; k < 3; ++k) {
+            for (int o = w / 2; o > 0; o >>= 1) {
+                lo[k] = fminf(lo[k], __shfl_xor(lo[k], o, 64));
+                hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], o, 64));
+                rlo[k] = fminf(rlo[k], __shfl_xor(rlo[k], o, 64));
+                rhi[k] = fmaxf(rhi[k], __shfl_xor(rhi[k], o, 64));
+            }
+        }
+        if ((lane & (w - 1)) == 0) {
+            float cc[3], h[3];
+            for (int k = 0; k < 3; ++k) {
+                h[k] = 0.5f * (hi[k] - lo[k]) * 1.0001f + 1e-4f;   // rounding margin
+                cc[k] = 0.5f * (lo[k] + hi[k]);
+            }
+            GMEM float4 *box = level ? (GMEM float4 *)cbox_p + 4 * c : (GMEM float4 *)gbox_p + 4 * (b0 / RDF_GROUP);
+            box[0] = make_float4(r0.x + cc[0], r0.y + cc[1], r0.z + cc[2], 0.f);
+            box[1] = b0 < N ? make_float4(h[0], h[1], h[2], 0.f) : make_float4(-1.f, -1.f, -1.f, 0.f);
+            box[2] = make_float4(rlo[0], rlo[1], rlo[2], 0.f);
+            box[3] = make_float4(rhi[0], rhi[1], rhi[2], 0.f);
+        }
+    }
+}
+
+// ---- counting ----------------------------------------------------------------
+// Image of every pair of a chunk and a group in one dimension.  fl(xj - xi)
+// lies in [fl(jlo - ihi), fl(jhi - ilo)] because rounding is monotone, so the
 // minimum-image rule |d| > L/2 -> d - copysign(L, d) takes one branch for
-// all of them, or the chunks are mixed: 0 = no wrap, 1 = d - L, 2 = d + L,
+// all of them, or they are mixed: 0 = no wrap, 1 = d - L, 2 = d + L,
 // 3 = mixed.
 __device__ __forceinline__ int rdf_dim_code(float ilo, float ihi, float jlo, float jhi, float L) {
 #pragma clang fp contract(off)
@@ -309,210 +476,171 @@ __device__ __forceinline__ int rdf_dim_code(float ilo, float ihi, float jlo, flo
     return 3;
 }
 
-// Pairs of lane i with j = js..je-1 of one staged chunk.  MX bits 0..2 mark
-// mixed dimensions, which take the per-pair minimum image; every other
-// dimension takes the image its code fixes for the whole chunk pair,
-// fl(fl(xj - xi) - s) with s = L, -L or 0, which is what mic1 returns, bit
-// for bit (MX = 8: no dimension wraps, s = 0 dropped).  The bin: the
-// estimate k0 = floor(sqrt(d2) * inv_bw) with inv_bw scaled by (1 - 2^-20),
-// which outweighs the rounding of v_sqrt_f32 and of the product, so k0 is
-// the exact bin or one below it; one comparison with the exact threshold
-// thr[k0 + 1] settles it.  Excluded pairs (d2 >= thr[bins], i.e. d >= L/2)
-// are masked off: an atomic of theirs would land on one word per type pair.
-template <int MX>
-__device__ __forceinline__ void rdf_chunk(const float4 *tj, int js, int je, float xi, float yi, float zi, float sx,
-                                          float sy, float sz, float L0, float L1, float L2, float inv_bw,
-                                          float kmax, float out_thr, const float *thr, char *hist_i) {
+// lower bound of the minimum-image distance between two boxes in a dimension
+__device__ __forceinline__ float rdf_gap(float ci, float hi, float cj, float hj, float L, float rL) {
+    const float d = ci - cj;
+    return fmaxf(0.f, fabsf(d - L * __builtin_rintf(d * rL)) - (hi + hj) - 4e-7f * L);
+}
+
+// Pairs of lane i with the RDF_GROUP particles of one group, read as scalars.
+// CX, CY, CZ: 0 no image, 1 the one the shift s = L or -L gives for the whole
+// group, fl(fl(xj - xi) - s), which is what mic1 returns, bit for bit, 2 the
+// per-pair minimum image.  after: only the j past this one (of the lane's own
+// chunk; -1: all).  The bin: the estimate b = sqrt(d2) * inv_bw with inv_bw
+// scaled down by more than the rounding of v_sqrt_f32, of the product and of
+// the exact rule can raise it, so floor(b) is the exact bin or one below it,
+// and one below only if the fraction of b is past R.edge; those few are settled
+// by the exact threshold thr[k + 1].  Excluded pairs (d2 >= thr[bins], i.e.
+// d >= L/2) are masked off: an atomic of theirs would land on one word per
+// type pair.
+template <int CX, int CY, int CZ>
+__device__ __forceinline__ void rdf_group(const RdfP &R, rdf_quad_t pj, int after, float xi, float yi, float zi,
+                                          float sx, float sy, float sz, float out_thr, const float *thr,
+                                          char *hist_i) {
 #pragma clang fp contract(off)
-    auto dist2 = [&](const float4 rj) {
-        float dx = rj.x - xi, dy = rj.y - yi, dz = rj.z - zi;
-        if (MX != 8) {
-            dx = (MX & 1) ? mic1(dx, L0) : dx - sx;
-            dy = (MX & 2) ? mic1(dy, L1) : dy - sy;
-            dz = (MX & 4) ? mic1(dz, L2) : dz - sz;
+    f32x16 q = pj[0];
+#pragma unroll
+    for (int u0 = 0; u0 < RDF_GROUP; u0 += 4) {
+        f32x16 nxt = q;
+        if (u0 + 4 < RDF_GROUP) nxt = pj[u0 / 4 + 1];
+        float d2[4], b[4], f = 0.f;
+        bool ok[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float dx = q[4 * u] - xi, dy = q[4 * u + 1] - yi, dz = q[4 * u + 2] - zi;
+            if (CX == 1) dx = dx - sx;
+            if (CX == 2) dx = mic1(dx, R.L0);
+            if (CY == 1) dy = dy - sy;
+            if (CY == 2) dy = mic1(dy, R.L1);
+            if (CZ == 1) dz = dz - sz;
+            if (CZ == 2) dz = mic1(dz, R.L2);
+            d2[u] = dx * dx;
+            d2[u] = d2[u] + dy * dy;
+            d2[u] = d2[u] + dz * dz;
+            ok[u] = d2[u] < out_thr;
+            if (CX + CY + CZ == 6) ok[u] &= u0 + u > after;
         }
-        float d2 = dx * dx;
-        d2 = d2 + dy * dy;
-        d2 = d2 + dz * dz;
-        return d2;
-    };
-    int jj = js;
-    // four pairs at a time: the threshold reads of all four are issued before
-    // the first histogram atomic (LDS reads do not pass an LDS atomic)
-    for (; jj + 4 <= je; jj += 4) {
-        float4 rj[4];
-        float d2[4], th[4];
-        int k0[4];
+        // four excluded in every lane skip the binning
+        if (ok[0] | ok[1] | ok[2] | ok[3]) {
+            int k[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) rj[u] = tj[jj + u];
+            for (int u = 0; u < 4; ++u) {
+                b[u] = __builtin_amdgcn_sqrtf(d2[u]) * R.inv_bw;
+                k[u] = (int)b[u];
+                f = fmaxf(f, __builtin_amdgcn_fractf(b[u]));
+            }
+            if (f >= R.edge) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) d2[u] = dist2(rj[u]);
-        // a group of four excluded in every lane skips the binning
-        if (d2[0] < out_thr || d2[1] < out_thr || d2[2] < out_thr || d2[3] < out_thr) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) k0[u] = (int)fminf(__builtin_amdgcn_sqrtf(d2[u]) * inv_bw, kmax);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) th[u] = thr[k0[u] + 1];
+                for (int u = 0; u < 4; ++u)
+                    if (ok[u] && d2[u] >= thr[k[u] + 1]) ++k[u];
+            }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                if (d2[u] < out_thr)
-                    atomicAdd((unsigned *)(hist_i + __float_as_int(rj[u].w) + 4 * k0[u] + (d2[u] >= th[u] ? 4 : 0)),
-                              1u);
+                if (ok[u]) atomicAdd((unsigned *)(hist_i + __float_as_int(q[4 * u + 3]) + 4 * k[u]), 1u);
         }
-    }
-    for (; jj < je; ++jj) {
-        const float4 rj = tj[jj];
-        const float d2 = dist2(rj);
-        const int k0 = (int)fminf(__builtin_amdgcn_sqrtf(d2) * inv_bw, kmax);
-        if (d2 < out_thr)
-            atomicAdd((unsigned *)(hist_i + __float_as_int(rj.w) + 4 * k0 + (d2 >= thr[k0 + 1] ? 4 : 0)), 1u);
+        q = nxt;
     }
 }
 
 // Unordered pairs i < j are visited once and counted in the slot of the
 // ordered type pair (type of the row particle i, type of j); the host adds
-// the (a, b) and (b, a) slots.  A block takes tile pairs (I, J), I <= J;
-// its wavefront w takes the chunk I*4 + w against the four chunks of J,
-// each chunk pair skipped when no pair can be closer than L/2, and handled
-// by the cheapest exact distance form its image code allows.
+// the (a, b) and (b, a) slots.  Chunk I meets the groups of the chunks J >= I;
+// rows I and nchunks-1-I together hold nchunks + 1 chunks, so the work is cut
+// into units of R.unit <= 64 groups of such a row pair, taken by turns by the
+// wavefronts of the grid.  Each lane tests one group of the unit (skipped when
+// no pair can be closer than L/2) and finds its image codes; the groups left
+// are counted one after the other, their positions in scalar registers.
+// Bound by the issue of VALU instructions, about 19 a visited pair and lane,
+// one of them a square root at a quarter of the rate (five cycles an
+// instruction and SIMD measured; LDS is busy a quarter of the time).  N = 65536,
+// 1000 bins, 2 types, in random order: 1.16 ms, against 1.76 for blocks that
+// staged tiles of 256 j in LDS, read the threshold of every pair and took the
+// particles in the caller's order (sorting adds 0.02; along a Morton curve
+// instead 1.22, counting excluded pairs in a spare word instead of masking
+// them off 1.18).
 __global__ void __launch_bounds__(256) k_rdf(RdfP R) {
     extern __shared__ __align__(16) char lds[];
-    const int nb1 = R.bins + 1;   // thresholds
     const int nh = R.nt * R.nt * R.bins;
     unsigned *hist = (unsigned *)lds;
     float *thr = (float *)(lds + (((size_t)nh * 4 + 15) & ~(size_t)15));
-    float4 *tj = (float4 *)((char *)thr + (((size_t)nb1 * 4 + 15) & ~(size_t)15));
-    int *codes = (int *)(tj + RDF_TILE);   // [16]: chunk pair (w, c) -> -1 skip, else 2-bit image codes x|y<<2|z<<4
     for (int x = threadIdx.x; x < nh; x += blockDim.x) hist[x] = 0u;
-    for (int x = threadIdx.x; x < nb1; x += blockDim.x) thr[x] = R.thr[x];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long long T = R.ntiles;
-    const float kmax = (float)(R.bins - 1), out_thr = R.thr[R.bins];
-    for (long long p = blockIdx.x; p < R.npairs; p += gridDim.x) {
-        // decode p -> (I, J), J >= I, rows of length T - I
-        double a = (double)(2 * T + 1);
-        long long I = (long long)((a - sqrt(a * a - 8.0 * (double)p)) * 0.5);
-        if (I < 0) I = 0;
-        if (I > T - 1) I = T - 1;
-        while (I > 0 && I * T - (I * (I - 1)) / 2 > p) --I;
-        while (I + 1 < T && (I + 1) * T - ((I + 1) * I) / 2 <= p) ++I;
-        const long long J = I + (p - (I * T - (I * (I - 1)) / 2));
-        __syncthreads();   // the previous tile pair's chunk and codes are read
-        if (threadIdx.x < 16) {
-            const int cw = threadIdx.x >> 2, cc = threadIdx.x & 3;
-            const long long ci = I * 4 + cw, cj = J * 4 + cc;
-            int code = -1;
-            if (ci < R.nchunks && cj < R.nchunks && !(I == J && cc < cw)) {
-                const float4 bi = R.cbox[4 * ci], hi = R.cbox[4 * ci + 1], bj = R.cbox[4 * cj],
-                             hj = R.cbox[4 * cj + 1];
-                // lower bound of the minimum-image distance between the chunks
-                const float gx = fmaxf(0.f, fabsf(mic1(bi.x - bj.x, R.L0)) - (hi.x + hj.x));
-                const float gy = fmaxf(0.f, fabsf(mic1(bi.y - bj.y, R.L1)) - (hi.y + hj.y));
-                const float gz = fmaxf(0.f, fabsf(mic1(bi.z - bj.z, R.L2)) - (hi.z + hj.z));
-                if (gx * gx + gy * gy + gz * gz <= R.skip2) {
-                    const float4 li = R.cbox[4 * ci + 2], ui = R.cbox[4 * ci + 3], lj = R.cbox[4 * cj + 2],
-                                 uj = R.cbox[4 * cj + 3];
-                    code = rdf_dim_code(li.x, ui.x, lj.x, uj.x, R.L0) |
-                           (rdf_dim_code(li.y, ui.y, lj.y, uj.y, R.L1) << 2) |
-                           (rdf_dim_code(li.z, ui.z, lj.z, uj.z, R.L2) << 4);
-                }
-            }
-            codes[threadIdx.x] = code;
+    for (int x = threadIdx.x; x <= R.bins; x += blockDim.x) thr[x] = R.thr[x];
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
+    const int waves = (int)(gridDim.x * (blockDim.x >> 6));
+    const float out_thr = R.thr[R.bins];
+    const int n = R.nchunks;
+    // unit u of row pair q, advanced by 'waves' units without a division a turn
+    int q = wave / R.nper, u = wave - q * R.nper;
+    const int dq = waves / R.nper, du = waves - dq * R.nper;
+    float xi = 0.f, yi = 0.f, zi = 0.f;
+    char *hist_i = nullptr;
+    int Icur = -1;
+    while (q < R.nrow) {
+        // group x of the row pair: chunk J and row I
+        const int first = (n - q) * (RDF_CHUNK / RDF_GROUP);
+        const int rows = (2 * q == n - 1) ? first : (n + 1) * (RDF_CHUNK / RDF_GROUP);
+        const int x = u * R.unit + lane;
+        int code = -1, I = 0, g = 0;
+        if (lane < R.unit && x < rows) {
+            I = x < first ? q : n - 1 - q;
+            g = x < first ? q * (RDF_CHUNK / RDF_GROUP) + x : I * (RDF_CHUNK / RDF_GROUP) + x - first;
+            const float4 bi = R.cbox[4 * I], hi = R.cbox[4 * I + 1], bj = R.gbox[4 * (size_t)g],
+                         hj = R.gbox[4 * (size_t)g + 1];
+            const float4 li = R.cbox[4 * I + 2], ui = R.cbox[4 * I + 3], lj = R.gbox[4 * (size_t)g + 2],
+                         uj = R.gbox[4 * (size_t)g + 3];
+            const float gx = rdf_gap(bi.x, hi.x, bj.x, hj.x, R.L0, R.rL0);
+            const float gy = rdf_gap(bi.y, hi.y, bj.y, hj.y, R.L1, R.rL1);
+            const float gz = rdf_gap(bi.z, hi.z, bj.z, hj.z, R.L2, R.rL2);
+            if (hj.x >= 0.f && !(gx * gx + gy * gy + gz * gz > R.skip2))
+                code = rdf_dim_code(li.x, ui.x, lj.x, uj.x, R.L0) | (rdf_dim_code(li.y, ui.y, lj.y, uj.y, R.L1) << 2) |
+                       (rdf_dim_code(li.z, ui.z, lj.z, uj.z, R.L2) << 4);
+            if (code >= 0 && g / (RDF_CHUNK / RDF_GROUP) == I) code = 0x3f;   // its own chunk: the form with 'after'
         }
-        __syncthreads();
-        int live = 0;   // the same for every thread of the block
-#pragma unroll
-        for (int x = 0; x < 16; ++x) live |= codes[x] >= 0;
-        if (!live) continue;
-        const int j0 = (int)(J * RDF_TILE);
-        {
-            const int j = j0 + threadIdx.x;
-            if (j < R.N) {
-                float4 rj = R.pos[j];
-                const int t = R.ptype ? R.ptype[j] : __float_as_int(rj.w);
-                rj.w = __int_as_float(t * R.bins * 4);
-                tj[threadIdx.x] = rj;
+        unsigned long long live = __ballot(code >= 0);
+        while (live) {
+            const int l = __builtin_ctzll(live);
+            live &= live - 1;
+            const int cd = __builtin_amdgcn_readlane(code, l), gj = __builtin_amdgcn_readlane(g, l),
+                      Ij = __builtin_amdgcn_readlane(I, l);
+            if (Ij != Icur) {
+                Icur = Ij;
+                float4 ri = R.pos[(size_t)Ij * RDF_CHUNK + lane];
+                if (Ij * RDF_CHUNK + lane >= R.N) ri.x = -RDF_PAD;
+                xi = ri.x;
+                yi = ri.y;
+                zi = ri.z;
+                hist_i = (char *)hist + (size_t)__float_as_int(ri.w) * R.nt;
             }
-        }
-        __syncthreads();
-        const int i = (int)(I * RDF_TILE) + threadIdx.x;
-        if (i < R.N) {
-            const float4 ri = R.pos[i];
-            const int ti = R.ptype ? R.ptype[i] : __float_as_int(ri.w);
-            char *hist_i = (char *)hist + (size_t)ti * R.nt * R.bins * 4;
-            for (int c = 0; c < 4; ++c) {
-                const int code = __builtin_amdgcn_readfirstlane(codes[w * 4 + c]);
-                if (code < 0) continue;
-                const int jb = j0 + c * RDF_CHUNK;
-                const int je = min(RDF_CHUNK, R.N - jb);
-                const int js = (I == J && c == w) ? lane + 1 : 0;
-                const float4 *tjc = tj + c * RDF_CHUNK;
-                const int cx = code & 3, cy = (code >> 2) & 3, cz = (code >> 4) & 3;
-                const float sx = cx == 1 ? R.L0 : (cx == 2 ? -R.L0 : 0.f);
-                const float sy = cy == 1 ? R.L1 : (cy == 2 ? -R.L1 : 0.f);
-                const float sz = cz == 1 ? R.L2 : (cz == 2 ? -R.L2 : 0.f);
-                const int mx = (cx == 3 ? 1 : 0) | (cy == 3 ? 2 : 0) | (cz == 3 ? 4 : 0);
-#define GMD_RDF_CHUNK(M)                                                                                        \
-    case M:                                                                                                     \
-        rdf_chunk<M>(tjc, js, je, ri.x, ri.y, ri.z, sx, sy, sz, R.L0, R.L1, R.L2, R.inv_bw, kmax, out_thr, thr, hist_i); \
+            const int own = gj - Ij * (RDF_CHUNK / RDF_GROUP);   // below 4: a group of the chunk itself
+            const int after = own < RDF_CHUNK / RDF_GROUP ? lane - own * RDF_GROUP : -1;
+            const int cx = cd & 3, cy = (cd >> 2) & 3, cz = (cd >> 4) & 3;
+            const float sx = cx == 2 ? -R.L0 : R.L0, sy = cy == 2 ? -R.L1 : R.L1, sz = cz == 2 ? -R.L2 : R.L2;
+            const rdf_quad_t pj = (rdf_quad_t)(size_t)(R.pos + (size_t)gj * RDF_GROUP);
+            const int form = (cx == 0 ? 0 : cx == 3 ? 2 : 1) * 9 + (cy == 0 ? 0 : cy == 3 ? 2 : 1) * 3 +
+                             (cz == 0 ? 0 : cz == 3 ? 2 : 1);
+#define RDF_FORM(F)                                                                                              \
+    case F:                                                                                                      \
+        rdf_group<(F) / 9, (F) / 3 % 3, (F) % 3>(R, pj, after, xi, yi, zi, sx, sy, sz, out_thr, thr, hist_i);          \
         break;
-                switch (code == 0 ? 8 : mx) {
-                    GMD_RDF_CHUNK(8)
-                    GMD_RDF_CHUNK(0)
-                    GMD_RDF_CHUNK(1)
-                    GMD_RDF_CHUNK(2)
-                    GMD_RDF_CHUNK(3)
-                    GMD_RDF_CHUNK(4)
-                    GMD_RDF_CHUNK(5)
-                    GMD_RDF_CHUNK(6)
-                    default:
-                        GMD_RDF_CHUNK(7)
-                }
-#undef GMD_RDF_CHUNK
-            }
+#define RDF_FORMS3(F) RDF_FORM(F) RDF_FORM(F + 1) RDF_FORM(F + 2)
+#define RDF_FORMS9(F) RDF_FORMS3(F) RDF_FORMS3(F + 3) RDF_FORMS3(F + 6)
+            switch (form) { RDF_FORMS9(0) RDF_FORMS9(9) RDF_FORMS9(18) }
+#undef RDF_FORMS9
+#undef RDF_FORMS3
+#undef RDF_FORM
+        }
+        q += dq;
+        u += du;
+        if (u >= R.nper) {
+            u -= R.nper;
+            ++q;
         }
     }
     __syncthreads();
     GMEM unsigned *dst = R.part + (size_t)blockIdx.x * nh;
     for (int x = threadIdx.x; x < nh; x += blockDim.x) dst[x] = hist[x];
-}
-
-// Boxes of each chunk of 64 consecutive particles (one wavefront per chunk):
-// centre and half extents in the minimum-image frame of the chunk's first
-// particle (tight for a chunk that straddles the periodic boundary), with a
-// rounding margin, and the raw coordinate bounds.
-__global__ void __launch_bounds__(256) k_rdf_boxes(const float4 *pos_p, int N, int nchunks, float L0, float L1,
-                                                   float L2, float4 *box_p) {
-    const GMEM float4 *pos = (const GMEM float4 *)pos_p;
-    GMEM float4 *box = (GMEM float4 *)box_p;
-    const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (c >= nchunks) return;
-    const int i0 = c * RDF_CHUNK, i = i0 + lane;
-    const float4 r0 = pos[i0];
-    const float4 r = i < N ? pos[i] : r0;
-    float lo[3] = {mic1(r.x - r0.x, L0), mic1(r.y - r0.y, L1), mic1(r.z - r0.z, L2)};
-    float hi[3] = {lo[0], lo[1], lo[2]};
-    float rlo[3] = {r.x, r.y, r.z};
-    float rhi[3] = {r.x, r.y, r.z};
-    for (int k = 0; k < 3; ++k) {
-        for (int o = 32; o > 0; o >>= 1) {
-            lo[k] = fminf(lo[k], __shfl_xor(lo[k], o, 64));
-            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], o, 64));
-            rlo[k] = fminf(rlo[k], __shfl_xor(rlo[k], o, 64));
-            rhi[k] = fmaxf(rhi[k], __shfl_xor(rhi[k], o, 64));
-        }
-    }
-    if (lane == 0) {
-        float cc[3], h[3];
-        for (int k = 0; k < 3; ++k) {
-            h[k] = 0.5f * (hi[k] - lo[k]) * 1.0001f + 1e-4f;   // rounding margin
-            cc[k] = 0.5f * (lo[k] + hi[k]);
-        }
-        box[4 * c] = make_float4(r0.x + cc[0], r0.y + cc[1], r0.z + cc[2], 0.f);
-        box[4 * c + 1] = make_float4(h[0], h[1], h[2], 0.f);
-        box[4 * c + 2] = make_float4(rlo[0], rlo[1], rlo[2], 0.f);
-        box[4 * c + 3] = make_float4(rhi[0], rhi[1], rhi[2], 0.f);
-    }
 }
 
 // Independent FMA chains (8 per lane) for gmd_fma_probe: 16 flop per lane and
@@ -572,22 +700,16 @@ __global__ void __launch_bounds__(256) k_copy(const float4 *src_p, float4 *dst_p
 #define NOALLOC_OFF_R 0                                                           // float [3 N]
 #define NOALLOC_OFF_T (NOALLOC_OFF_R + 3 * 4 * NOALLOC_RDF_MAX_N)                // int [N]
 #define NOALLOC_OFF_POS (NOALLOC_OFF_T + 4 * NOALLOC_RDF_MAX_N)                  // float4 [N]
-#define NOALLOC_OFF_BOX (NOALLOC_OFF_POS + 16 * NOALLOC_RDF_MAX_N)               // float4 [4 chunks]
-#define NOALLOC_OFF_THR (NOALLOC_OFF_BOX + 16 * 4 * (NOALLOC_RDF_MAX_N / RDF_CHUNK))   // float [bins + 1]
+#define NOALLOC_OFF_GBOX (NOALLOC_OFF_POS + 16 * NOALLOC_RDF_MAX_N)              // float4 [4 groups]
+#define NOALLOC_OFF_CBOX (NOALLOC_OFF_GBOX + 16 * 4 * (NOALLOC_RDF_MAX_N / RDF_GROUP))   // float4 [4 chunks]
+#define NOALLOC_OFF_KEY (NOALLOC_OFF_CBOX + 16 * 4 * (NOALLOC_RDF_MAX_N / RDF_CHUNK))    // int2 [N]
+#define NOALLOC_OFF_CELL (NOALLOC_OFF_KEY + 8 * NOALLOC_RDF_MAX_N)               // int [cells]
+#define NOALLOC_OFF_THR (NOALLOC_OFF_CELL + 4 * RDF_MAX_CELL * RDF_MAX_CELL * RDF_MAX_CELL)   // float [bins + 1]
 #define NOALLOC_OFF_PART (NOALLOC_OFF_THR + ((4 * (NOALLOC_RDF_MAX_HIST + 1) + 255) / 256) * 256)   // u32 [grid][hist]
 #define NOALLOC_OFF_OUT (NOALLOC_OFF_PART + 4 * NOALLOC_RDF_GRID * NOALLOC_RDF_MAX_HIST)   // u64 [hist]
 #define NOALLOC_BYTES (NOALLOC_OFF_OUT + 8 * NOALLOC_RDF_MAX_HIST)
 
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
-
-// (x, y, z) of host layout (N, 3) and the type -> float4 with the type bits in w
-__global__ void __launch_bounds__(256) k_rdf_pack(const float *r_p, const int *t_p, int N, float4 *pos_p) {
-    const GMEM float *r = (const GMEM float *)r_p;
-    const GMEM int *t = (const GMEM int *)t_p;
-    GMEM float4 *pos = (GMEM float4 *)pos_p;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x)
-        pos[i] = make_float4(r[3 * i], r[3 * i + 1], r[3 * i + 2], __int_as_float(t[i]));
-}
 
 // a fill kernel instead of a memset, so the clear can sit in a captured graph
 __global__ void __launch_bounds__(256) k_fill_u64(unsigned long long *p_p, int n) {
@@ -942,12 +1064,14 @@ struct gmd_ctx {
 
 struct gmd_rdf {
     int N, nt, bins, nchunks;
-    float4 *pos = nullptr;
-    float4 *tbox = nullptr;   // chunk boxes, 4 per chunk
+    float4 *pos = nullptr;    // snapshot of a context's positions; (N, 3) positions of the host
+    float4 *sorted = nullptr; // what the kernels read: cell order, whole chunks
+    float4 *gbox = nullptr, *cbox = nullptr;   // group and chunk boxes, 4 each
+    int2 *key = nullptr;
     int *ptype = nullptr;
     float *d_thr = nullptr;
     unsigned *part = nullptr;
-    unsigned long long *d_out = nullptr;
+    unsigned long long *d_out = nullptr;   // the counts, and after them the sorting cells (cleared together)
     int grid = 0;      // histogram blocks of a launch whose result is awaited at once
     int grid_bg = 0;   // fewer blocks for a launch that runs beside the simulation's steps
     float box[3] = {0, 0, 0};
@@ -2081,7 +2205,62 @@ static size_t rdf_hist_size(int nt, int bins) { return (size_t)nt * nt * bins; }
 
 static size_t rdf_lds_bytes(int nt, int bins) {
     const size_t nh = rdf_hist_size(nt, bins);
-    return ((nh * 4 + 15) & ~(size_t)15) + (((size_t)(bins + 1) * 4 + 15) & ~(size_t)15) + RDF_TILE * 16 + 16 * 4;
+    return ((nh * 4 + 15) & ~(size_t)15) + (((size_t)(bins + 1) * 4 + 15) & ~(size_t)15);
+}
+
+// Sorting cells per dimension: some 16 particles a cell; 1 (none) where the
+// sort's three launches (20 us with their gaps) are what it saves: N = 8000 in
+// random order 165 us a call sorted, 164 not; N = 20000 351 against 394.
+static int rdf_cells(int N) { return N < 8192 ? 1 : N < 32768 ? 8 : N < 262144 ? 16 : RDF_MAX_CELL; }
+
+// The launches of one histogram on a stream: sort, boxes, counts, sum over
+// blocks.  S.pos (or S.r) / S.ptype: the input; out and the cell counts are
+// zero; grid: blocks of k_rdf, at most what R.part holds.
+static int rdf_kernels(RdfP R, RdfSort S, const float box[3], int grid, float4 *gbox, float4 *cbox,
+                       unsigned long long *out, hipStream_t st) {
+    const int N = R.N;
+    R.L0 = box[0];
+    R.L1 = box[1];
+    R.L2 = box[2];
+    R.rL0 = S.rL0 = 1.0f / box[0];
+    R.rL1 = S.rL1 = 1.0f / box[1];
+    R.rL2 = S.rL2 = 1.0f / box[2];
+    const float mn = std::min(box[0], std::min(box[1], box[2]));
+    const double bw = ((double)mn / 2.0) / R.bins;
+    // relative errors of the estimate against the exact rule: square root
+    // 2^-23 here and 2^-24 there, product and constant 2^-24 each, 0.625 2^-21
+    // in all; so scaled by 1 - 0.75 2^-21 it is never above, and below by less
+    // than 1.375 2^-21 of at most 'bins'
+    R.inv_bw = (float)((1.0 / bw) * (1.0 - 0.75 / 2097152.0));
+    R.edge = (float)(1.0 - 1.5 / 2097152.0 * R.bins);
+    R.nchunks = (N + RDF_CHUNK - 1) / RDF_CHUNK;
+    R.nrow = (R.nchunks + 1) / 2;
+    const long long row = (long long)(R.nchunks + 1) * (RDF_CHUNK / RDF_GROUP);
+    // as many groups a unit as leave a wavefront some eight units
+    R.unit = (int)std::max(1LL, std::min(64LL, R.nrow * row / (8LL * 4 * grid)));
+    R.nper = (int)((row + R.unit - 1) / R.unit);
+    R.cbox = (const GMEM float4 *)cbox;
+    R.gbox = (const GMEM float4 *)gbox;
+    R.pos = (cpos_t)S.out;
+    S.N = N;
+    S.npad = R.nchunks * RDF_CHUNK;
+    S.nt_bytes = R.bins * 4;
+    S.ncell = rdf_cells(N);
+    const unsigned nb = (unsigned)((N + 255) / 256);
+    if (S.ncell > 1) {
+        hipLaunchKernelGGL(k_rdf_count, dim3(nb), dim3(256), 0, st, S);
+        hipLaunchKernelGGL(k_rdf_starts, dim3(1), dim3(1024), 0, st, S.count, S.ncell * S.ncell * S.ncell);
+        hipLaunchKernelGGL(k_rdf_place, dim3((unsigned)((S.npad + 255) / 256)), dim3(256), 0, st, S);
+    }
+    hipLaunchKernelGGL(k_rdf_boxes, dim3((unsigned)((R.nchunks + 3) / 4)), dim3(256), 0, st, S, S.ncell > 1 ? 0 : 1,
+                       box[0], box[1], box[2], gbox, cbox);
+    hipLaunchKernelGGL(k_rdf, dim3(grid), dim3(256), rdf_lds_bytes(R.nt, R.bins), st, R);
+    HIPCHECK(hipGetLastError());
+    const int nh = (int)rdf_hist_size(R.nt, R.bins), per = 16;
+    hipLaunchKernelGGL(k_rdf_reduce, dim3((unsigned)((nh + 255) / 256), (unsigned)((grid + per - 1) / per)),
+                       dim3(256), 0, st, (const unsigned *)R.part, grid, nh, per, out);
+    HIPCHECK(hipGetLastError());
+    return 0;
 }
 
 int gmd_rdf_create(int N, int ntypes, int bins, gmd_rdf **out) {
@@ -2094,7 +2273,7 @@ int gmd_rdf_create(int N, int ntypes, int bins, gmd_rdf **out) {
     r->bins = bins;
     r->nchunks = (N + RDF_CHUNK - 1) / RDF_CHUNK;
     const size_t nh = rdf_hist_size(ntypes, bins);
-    if (rdf_lds_bytes(ntypes, bins) > 64 * 1024) {
+    if (rdf_lds_bytes(ntypes, bins) > 64 * 1024 - RDF_LDS_SPARE) {
         delete r;
         return fail("gmd_rdf_create: %d x %d type pairs x %d bins do not fit the LDS histogram", ntypes, ntypes,
                     bins);
@@ -2102,20 +2281,24 @@ int gmd_rdf_create(int N, int ntypes, int bins, gmd_rdf **out) {
     int dev = 0, cus = 0;
     HIPCHECK(hipGetDevice(&dev));
     HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const long long T = (N + RDF_TILE - 1) / RDF_TILE;
-    const long long npairs = T * (T + 1) / 2;
+    // blocks of four wavefronts that have a group each
+    const long long npairs = ((long long)r->nchunks * (r->nchunks + 1) / 2 * (RDF_CHUNK / RDF_GROUP) + 3) / 4;
     // a block's 32-bit counters see at most 2^31 pairs
     const long long need = (long long)(((double)N * (double)N / 2.0) / 2147483648.0) + 1;
     r->grid = (int)std::max(1LL, std::min(npairs, std::max((long long)cus * 4, need)));
     // beside the step kernels, 2 blocks per CU take fewer of their slots and
     // still finish within a block of steps
     r->grid_bg = (int)std::max(1LL, std::min(npairs, std::max((long long)cus * 2, need)));
+    const size_t ng = (size_t)r->nchunks * (RDF_CHUNK / RDF_GROUP), cells = rdf_cells(N);
     if (hipMalloc(&r->pos, (size_t)N * sizeof(float4)) != hipSuccess ||
-        hipMalloc(&r->tbox, (size_t)4 * r->nchunks * sizeof(float4)) != hipSuccess ||
+        hipMalloc(&r->sorted, (size_t)r->nchunks * RDF_CHUNK * sizeof(float4)) != hipSuccess ||
+        hipMalloc(&r->cbox, (size_t)4 * r->nchunks * sizeof(float4)) != hipSuccess ||
+        hipMalloc(&r->gbox, 4 * ng * sizeof(float4)) != hipSuccess ||
+        hipMalloc(&r->key, (size_t)N * sizeof(int2)) != hipSuccess ||
         hipMalloc(&r->ptype, (size_t)N * sizeof(int)) != hipSuccess ||
         hipMalloc(&r->d_thr, (size_t)(bins + 1) * sizeof(float)) != hipSuccess ||
         hipMalloc(&r->part, (size_t)r->grid * nh * sizeof(unsigned)) != hipSuccess ||
-        hipMalloc(&r->d_out, nh * sizeof(unsigned long long)) != hipSuccess) {
+        hipMalloc(&r->d_out, nh * sizeof(unsigned long long) + cells * cells * cells * sizeof(int)) != hipSuccess) {
         gmd_rdf_destroy(r);
         return fail("gmd_rdf_create: out of device memory");
     }
@@ -2136,7 +2319,7 @@ int gmd_rdf_create(int N, int ntypes, int bins, gmd_rdf **out) {
 
 int gmd_rdf_destroy(gmd_rdf *r) {
     if (!r) return 0;
-    void *ptrs[] = {r->pos, r->tbox, r->ptype, r->d_thr, r->part, r->d_out};
+    void *ptrs[] = {r->pos, r->sorted, r->cbox, r->gbox, r->key, r->ptype, r->d_thr, r->part, r->d_out};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (r->pending && r->done) hipEventSynchronize(r->done);
@@ -2148,45 +2331,33 @@ int gmd_rdf_destroy(gmd_rdf *r) {
     return 0;
 }
 
-// Enqueue one histogram of the positions at pos on the calculator's stream,
-// ending in an asynchronous copy of the counts to pinned host memory.
+// Enqueue one histogram on the calculator's stream (pos: positions with types,
+// or null: the host's in r->pos; d_ptype: their types, with pos instead of its
+// own), ending in an asynchronous copy of the counts to pinned host memory.
 static int rdf_launch(gmd_rdf *r, const float4 *pos, const int *d_ptype, const float box[3], int grid) {
     if (box[0] != r->box[0] || box[1] != r->box[1] || box[2] != r->box[2] || r->thr.empty()) {
         rdf_thresholds(box, r->bins, r->thr);
         HIPCHECK(hipMemcpy(r->d_thr, r->thr.data(), (size_t)(r->bins + 1) * sizeof(float), hipMemcpyHostToDevice));
         memcpy(r->box, box, sizeof r->box);
     }
-    RdfP R;
+    const size_t nh = rdf_hist_size(r->nt, r->bins), cells = rdf_cells(r->N);
+    RdfP R = {};
     R.N = r->N;
     R.nt = r->nt;
     R.bins = r->bins;
-    R.nchunks = r->nchunks;
-    R.ntiles = (r->N + RDF_TILE - 1) / RDF_TILE;
-    R.npairs = (long long)R.ntiles * (R.ntiles + 1) / 2;
-    R.L0 = box[0];
-    R.L1 = box[1];
-    R.L2 = box[2];
-    {
-        float mn = std::min(box[0], std::min(box[1], box[2]));
-        double bw = ((double)mn / 2.0) / r->bins;
-        R.inv_bw = (float)((1.0 / bw) * (1.0 - 1.0 / 1048576.0));   // estimate never above the exact bin
-    }
-    R.pos = (cpos_t)pos;
-    R.ptype = (const GMEM int *)d_ptype;
     R.thr = (const GMEM float *)r->d_thr;
     R.part = (GMEM unsigned *)r->part;
-    R.cbox = (const GMEM float4 *)r->tbox;
     R.skip2 = r->thr[r->bins];
-    const size_t nh = rdf_hist_size(r->nt, r->bins);
-    HIPCHECK(hipMemsetAsync(r->d_out, 0, nh * sizeof(unsigned long long), r->stream));
-    hipLaunchKernelGGL(k_rdf_boxes, dim3((unsigned)((r->nchunks + 3) / 4)), dim3(256), 0, r->stream, pos, r->N,
-                       r->nchunks, box[0], box[1], box[2], r->tbox);
-    hipLaunchKernelGGL(k_rdf, dim3(grid), dim3(256), rdf_lds_bytes(r->nt, r->bins), r->stream, R);
-    HIPCHECK(hipGetLastError());
-    const int per = 16;
-    hipLaunchKernelGGL(k_rdf_reduce, dim3((unsigned)((nh + 255) / 256), (unsigned)((grid + per - 1) / per)),
-                       dim3(256), 0, r->stream, (const unsigned *)r->part, grid, (int)nh, per, r->d_out);
-    HIPCHECK(hipGetLastError());
+    RdfSort S = {};
+    S.pos = pos;
+    S.r = (const float *)r->pos;
+    S.ptype = d_ptype;
+    S.count = (int *)(r->d_out + nh);
+    S.key = r->key;
+    S.out = r->sorted;
+    HIPCHECK(hipMemsetAsync(r->d_out, 0, nh * sizeof(unsigned long long) + cells * cells * cells * sizeof(int),
+                            r->stream));
+    if (rdf_kernels(R, S, box, grid, r->gbox, r->cbox, r->d_out, r->stream)) return -1;
     HIPCHECK(hipMemcpyAsync(r->h_out, r->d_out, nh * sizeof(unsigned long long), hipMemcpyDeviceToHost, r->stream));
     HIPCHECK(hipEventRecord(r->done, r->stream));
     r->pending = true;
@@ -2258,11 +2429,10 @@ int gmd_rdf_compute_host(gmd_rdf *r, const float *pos, const int *ptype, const f
     if (!r || !pos || !ptype || !box || !counts) return fail("gmd_rdf_compute_host: null argument");
     for (int i = 0; i < r->N; ++i)
         if (ptype[i] < 0 || ptype[i] >= r->nt) return fail("gmd_rdf_compute_host: type out of range");
-    std::vector<float4> h(r->N);
-    for (int i = 0; i < r->N; ++i) h[i] = make_float4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], i2f(ptype[i]));
     if (r->pending) return fail("gmd_rdf_compute_host: a launched update is not collected");
-    HIPCHECK(hipMemcpy(r->pos, h.data(), h.size() * sizeof(float4), hipMemcpyHostToDevice));
-    if (rdf_launch(r, r->pos, nullptr, box, r->grid)) return -1;
+    HIPCHECK(hipMemcpy(r->pos, pos, (size_t)r->N * 3 * sizeof(float), hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(r->ptype, ptype, (size_t)r->N * sizeof(int), hipMemcpyHostToDevice));
+    if (rdf_launch(r, nullptr, r->ptype, box, r->grid)) return -1;
     return rdf_collect(r, counts);
 }
 
@@ -2310,7 +2480,6 @@ int gmd_rdf_compute_host_noalloc(int N, int ntypes, int bins, const float *pos, 
     float *d_r = (float *)(base + NOALLOC_OFF_R);
     int *d_t = (int *)(base + NOALLOC_OFF_T);
     float4 *d_pos = (float4 *)(base + NOALLOC_OFF_POS);
-    float4 *d_box = (float4 *)(base + NOALLOC_OFF_BOX);
     float *d_thr = (float *)(base + NOALLOC_OFF_THR);
     unsigned *d_part = (unsigned *)(base + NOALLOC_OFF_PART);
     unsigned long long *d_out = (unsigned long long *)(base + NOALLOC_OFF_OUT);
@@ -2322,41 +2491,30 @@ int gmd_rdf_compute_host_noalloc(int N, int ntypes, int bins, const float *pos, 
     HIPCHECK(hipMemcpy(d_r, pos, (size_t)N * 3 * sizeof(float), hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(d_t, ptype, (size_t)N * sizeof(int), hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(d_thr, thr, (size_t)(bins + 1) * sizeof(float), hipMemcpyHostToDevice));
-    RdfP R;
+    RdfP R = {};
     R.N = N;
     R.nt = ntypes;
     R.bins = bins;
-    R.nchunks = (N + RDF_CHUNK - 1) / RDF_CHUNK;
-    R.ntiles = (N + RDF_TILE - 1) / RDF_TILE;
-    R.npairs = (long long)R.ntiles * (R.ntiles + 1) / 2;
-    R.L0 = box[0];
-    R.L1 = box[1];
-    R.L2 = box[2];
-    {
-        float mn = std::min(box[0], std::min(box[1], box[2]));
-        double bw = ((double)mn / 2.0) / bins;
-        R.inv_bw = (float)((1.0 / bw) * (1.0 - 1.0 / 1048576.0));   // estimate never above the exact bin
-    }
-    R.pos = (cpos_t)d_pos;
-    R.ptype = nullptr;   // types ride in pos.w
     R.thr = (const GMEM float *)d_thr;
     R.part = (GMEM unsigned *)d_part;
-    R.cbox = (const GMEM float4 *)d_box;
     R.skip2 = thr[bins];
+    RdfSort S = {};
+    S.r = d_r;
+    S.ptype = d_t;
+    S.count = (int *)(base + NOALLOC_OFF_CELL);
+    S.key = (int2 *)(base + NOALLOC_OFF_KEY);
+    S.out = d_pos;
     // at most NOALLOC_RDF_MAX_N^2 / 2 = 2^31 pairs in total, so even a single
     // block's 32-bit counters cannot overflow
-    const int grid = (int)std::max(1LL, std::min(R.npairs, (long long)NOALLOC_RDF_GRID));
-    hipLaunchKernelGGL(k_rdf_pack, dim3((unsigned)std::min((N + 255) / 256, 1024)), dim3(256), 0, st,
-                       (const float *)d_r, (const int *)d_t, N, d_pos);
+    const long long nc = (N + RDF_CHUNK - 1) / RDF_CHUNK;
+    const int grid = (int)std::min(nc * (nc + 1) / 2, (long long)NOALLOC_RDF_GRID);
     hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, d_out, (int)nh);
-    hipLaunchKernelGGL(k_rdf_boxes, dim3((unsigned)((R.nchunks + 3) / 4)), dim3(256), 0, st, (const float4 *)d_pos, N,
-                       R.nchunks, box[0], box[1], box[2], d_box);
-    hipLaunchKernelGGL(k_rdf, dim3(grid), dim3(256), rdf_lds_bytes(ntypes, bins), st, R);
-    HIPCHECK(hipGetLastError());
-    const int per = 16;
-    hipLaunchKernelGGL(k_rdf_reduce, dim3((unsigned)((nh + 255) / 256), (unsigned)((grid + per - 1) / per)),
-                       dim3(256), 0, st, (const unsigned *)d_part, grid, (int)nh, per, d_out);
-    HIPCHECK(hipGetLastError());
+    const int cells = rdf_cells(N) * rdf_cells(N) * rdf_cells(N);
+    hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)(((cells + 1) / 2 + 255) / 256)), dim3(256), 0, st,
+                       (unsigned long long *)S.count, (cells + 1) / 2);
+    if (rdf_kernels(R, S, box, grid, (float4 *)(base + NOALLOC_OFF_GBOX), (float4 *)(base + NOALLOC_OFF_CBOX), d_out,
+                    st))
+        return -1;
     HIPCHECK(hipMemcpy(raw, d_out, nh * sizeof(unsigned long long), hipMemcpyDeviceToHost));
     // unordered pair counts in ordered-type slots -> ordered pair counts
     for (int a = 0; a < ntypes; ++a)

@@ -254,7 +254,7 @@ int gmd_rdf_compute_host(gmd_rdf *rdf, const float *r, const int *ptype, const f
  * allocation: no counterpart in the reference.  For callers that cannot
  * allocate device memory (code under graph capture, tight serving loops).
  * Every device buffer (staged positions and types, chunk boxes, thresholds,
- * per-block histograms, counts) lives in one static array of about 10.6 MB
+ * per-block histograms, counts) lives in one static array of about 11.5 MB
  * per device, held until the process ends.  Limits: N <= 65536,
  * ntypes * ntypes * bins <= 4096; larger sizes are refused with an error.
  * Runs on the null stream and returns when the counts are on the host.  All
