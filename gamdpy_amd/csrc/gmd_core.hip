@@ -32,14 +32,10 @@ __global__ void k_advance(Ctrl *Cp, int n) {
     if (threadIdx.x == 0 && blockIdx.x == 0) C->s_base += n;
 }
 
-// the tails of all replicas of a batch: block r finishes replica r's step
-__global__ void __launch_bounds__(256) k_batch_tail(const DP *const *Ps, int integrator) {
-    const DP &P = *uniform_ptr(Ps[blockIdx.x]);
-    __shared__ double red[4 * GMD_NRED];
-    const int s = P.ctrl->step;
-    if (s > P.ctrl->nsteps) return;
-    const StepInfo I = step_info(P, s, integrator, P.ctrl->rebuild_now != 0);
-    step_tail(P, I, red, P.step_grid);
+// the same for every replica of a batch
+__global__ void __launch_bounds__(256) k_batch_advance(const DP *__restrict__ Ps, int nrep, int n) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < nrep) Ps[r].ctrl->s_base += n;
 }
 
 // ---- run set-up: cell grid of the starting positions and the skin test ----
@@ -69,7 +65,6 @@ __device__ __forceinline__ void run_begin(const DP &P, int nsteps, float t0, con
         C->t0 = t0;
         C->buf0 = R.buf0;
         C->lstep0 = R.lstep;
-        C->step = 0;
         C->s_base = 0;
         C->red_count = 0;
         C->bar_count = 0;
@@ -88,8 +83,8 @@ __global__ void __launch_bounds__(256) k_run_begin(const DP *__restrict__ Pp, in
 }
 
 // the same for the replicas of a batch (one per y of the grid)
-__global__ void __launch_bounds__(256) k_batch_begin(const DP *const *Ps, int nsteps, float t0, const RunStart *R) {
-    run_begin(*uniform_ptr(Ps[blockIdx.y]), nsteps, t0, R[blockIdx.y]);
+__global__ void __launch_bounds__(256) k_batch_begin(const DP *__restrict__ Ps, int nsteps, float t0, const RunStart *R) {
+    run_begin(Ps[blockIdx.y], nsteps, t0, R[blockIdx.y]);
 }
 
 // skin test of the starting positions (nblist.py:58-86 at step 0) and, for
@@ -115,7 +110,7 @@ __device__ __forceinline__ void run_setup(const DP &P) {
 
 __global__ void __launch_bounds__(256) k_run_setup(const DP *__restrict__ Pp) { run_setup(*Pp); }
 
-__global__ void __launch_bounds__(256) k_batch_setup(const DP *const *Ps) { run_setup(*uniform_ptr(Ps[blockIdx.y])); }
+__global__ void __launch_bounds__(256) k_batch_setup(const DP *__restrict__ Ps) { run_setup(Ps[blockIdx.y]); }
 
 // the prepared pair table of the context (once)
 __global__ void k_pair_table(const DP *__restrict__ Pp) {
@@ -126,12 +121,6 @@ __global__ void k_pair_table(const DP *__restrict__ Pp) {
         prepare_pair(P, t, q);
         P.ptab[t] = q;
     }
-}
-
-// replicas read the decision of their next step from the control block
-__global__ void __launch_bounds__(256) k_batch_setup_finish(const DP *const *Ps, int nrep) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nrep) Ps[r]->ctrl->rebuild_now = Ps[r]->rebuild_flag[0];
 }
 
 // ---- what the host reads after a run, into pinned memory: the control block
@@ -147,7 +136,7 @@ __device__ __forceinline__ void run_publish(const DP &P) {
 
 __global__ void __launch_bounds__(256) k_run_publish(const DP *__restrict__ Pp) { run_publish(*Pp); }
 
-__global__ void __launch_bounds__(256) k_batch_publish(const DP *const *Ps) { run_publish(*uniform_ptr(Ps[blockIdx.x])); }
+__global__ void __launch_bounds__(256) k_batch_publish(const DP *__restrict__ Ps) { run_publish(Ps[blockIdx.x]); }
 
 // ---- the host's arrays to and from the device layout ----
 // One kernel gathers every array into the packed buffer (unpack) or takes it
@@ -205,8 +194,8 @@ __global__ void __launch_bounds__(256) k_unpack(const DP *__restrict__ Pp, int c
 }
 
 // every replica of a batch into its own packed buffer in device memory
-__global__ void __launch_bounds__(256) k_batch_unpack(const DP *const *Ps, const RunStart *R) {
-    const DP &P = *uniform_ptr(Ps[blockIdx.y]);
+__global__ void __launch_bounds__(256) k_batch_unpack(const DP *__restrict__ Ps, const RunStart *R) {
+    const DP &P = Ps[blockIdx.y];
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < P.N; i += gridDim.x * blockDim.x)
         unpack_state(P, R[blockIdx.y].buf0, XF_ALL, (int *)P.xdev, i);
 }
@@ -222,8 +211,8 @@ __device__ __forceinline__ void copy_words(const int *src_p, int *dst_p, size_t 
 // n words between two 16-byte aligned buffers
 __global__ void __launch_bounds__(256) k_copy_words(const int *src, int *dst, size_t n) { copy_words(src, dst, n); }
 
-__global__ void __launch_bounds__(256) k_batch_fetch(const DP *const *Ps) {
-    const DP &P = *uniform_ptr(Ps[blockIdx.y]);
+__global__ void __launch_bounds__(256) k_batch_fetch(const DP *__restrict__ Ps) {
+    const DP &P = Ps[blockIdx.y];
     copy_words((const int *)P.xdev, P.xhost, XferSeg((size_t)P.N, (size_t)P.nscal).end);
 }
 
@@ -909,14 +898,16 @@ struct Arena {
 
 typedef void (*kfun)(const DP *);
 typedef void (*sfun)(const DP *, int);
-typedef void (*bfun)(const DP *const *, const BatchBlk *);
+typedef void (*bfun)(const DP *, const BatchBlk *);
+typedef void (*bsfun)(const DP *, const BatchBlk *, int);
 
 // the kernel instances of one (pair function, cutoff, integrator) combination
 // and list kind
 struct Kernels {
     kfun pers;
     sfun step;
-    bfun bpers, bstep;
+    bfun bpers;
+    bsfun bstep;
 };
 
 template <int BASE, int CUT, int INTEG>
@@ -2540,7 +2531,7 @@ struct gmd_batch {
     std::vector<BatchBlk> h_blk;
     RunStart *h_start = nullptr;   // pinned: what each replica's run starts from (read by the kernels)
     BatchBlk *d_blk = nullptr;
-    const DP **d_Ps = nullptr;
+    DP *d_Ps = nullptr;            // the replicas' DP, one after another (each context's d_P points here)
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     float last_ms = 0.f;
@@ -2629,6 +2620,7 @@ int gmd_batch_create(const gmd_desc *descs, int nrep, const int *blocks, int dri
     BTRY(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
     BTRY(hipEventCreate(&b->ev0));
     BTRY(hipEventCreate(&b->ev1));
+    BTRY(hipMalloc((void **)&b->d_Ps, nrep * sizeof(DP)));
     std::vector<int> nb(nrep);
     for (int r = 0; r < nrep; ++r) {
         gmd_desc d = descs[r];
@@ -2648,6 +2640,7 @@ int gmd_batch_create(const gmd_desc *descs, int nrep, const int *blocks, int dri
             return fail("gmd_batch_create: replica %d: %d blocks requested, allowed 1..%d", r, nb[r], cap);
         }
         c->P.step_grid = nb[r];
+        c->d_P = b->d_Ps + r;
         BTRY(hipMemcpy(c->d_P, &c->P, sizeof(DP), hipMemcpyHostToDevice));
         b->lds = std::max(b->lds, c->lds_step);
         b->block = c->block;
@@ -2668,11 +2661,7 @@ int gmd_batch_create(const gmd_desc *descs, int nrep, const int *blocks, int dri
     }
     BTRY(hipMalloc((void **)&b->d_blk, b->h_blk.size() * sizeof(BatchBlk)));
     BTRY(hipMemcpy(b->d_blk, b->h_blk.data(), b->h_blk.size() * sizeof(BatchBlk), hipMemcpyHostToDevice));
-    std::vector<const DP *> ps(nrep);
-    for (int r = 0; r < nrep; ++r) ps[r] = b->reps[r]->d_P;
     BTRY(hipHostMalloc((void **)&b->h_start, (size_t)nrep * sizeof(RunStart), hipHostMallocDefault));
-    BTRY(hipMalloc((void **)&b->d_Ps, nrep * sizeof(DP *)));
-    BTRY(hipMemcpy(b->d_Ps, ps.data(), nrep * sizeof(DP *), hipMemcpyHostToDevice));
 #undef BTRY
     *out = b;
     return 0;
@@ -2709,14 +2698,13 @@ int gmd_batch_run(gmd_batch *b, float time_zero, int steps) {
         gs = std::max(gs, (unsigned)c->grid_aux);
     }
     // the rebuild-flag arrays may have been reallocated by the preparation;
-    // the set-up of all replicas in three launches
+    // the set-up of all replicas in two launches
     hipStream_t st = b->stream;
-    const DP *const *Ps = b->d_Ps;
+    const DP *Ps = b->d_Ps;
     const BatchBlk *blk = b->d_blk;
     hipLaunchKernelGGL(k_batch_begin, dim3(gx, nrep), dim3(256), 0, st, Ps, steps, time_zero,
                        (const RunStart *)b->h_start);
     hipLaunchKernelGGL(k_batch_setup, dim3(gs, nrep), dim3(256), 0, st, Ps);
-    hipLaunchKernelGGL(k_batch_setup_finish, dim3((nrep + 255) / 256), dim3(256), 0, st, Ps, (int)nrep);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(b->ev0, st));
     if (b->driver == GMD_BATCH_PERSISTENT) {
@@ -2726,15 +2714,18 @@ int gmd_batch_run(gmd_batch *b, float time_zero, int steps) {
     } else {
         if (!b->gexec) {
             HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            for (int k = 0; k < GRAPH_STEPS; ++k) {
-                hipLaunchKernelGGL(b->kern.bstep, dim3(b->grid), dim3(b->block), b->lds, st, Ps, blk);
-                hipLaunchKernelGGL(k_batch_tail, dim3((unsigned)b->reps.size()), dim3(256), 0, st, Ps, b->integrator);
-            }
+            for (int k = 0; k < GRAPH_STEPS; ++k)
+                hipLaunchKernelGGL(b->kern.bstep, dim3(b->grid), dim3(b->block), b->lds, st, Ps, blk, k);
+            hipLaunchKernelGGL(k_batch_advance, dim3((nrep + 255) / 256), dim3(256), 0, st, Ps, (int)nrep, GRAPH_STEPS);
             HIPCHECK(hipStreamEndCapture(st, &b->graph));
             HIPCHECK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
         }
-        const int launches = (steps + 1 + GRAPH_STEPS - 1) / GRAPH_STEPS;
-        for (int k = 0; k < launches; ++k) HIPCHECK(hipGraphLaunch(b->gexec, st));
+        // as in run_impl: whole groups of steps, then the rest
+        const int groups = (steps + 1) / GRAPH_STEPS, rest = (steps + 1) % GRAPH_STEPS;
+        for (int g = 0; g < groups; ++g) HIPCHECK(hipGraphLaunch(b->gexec, st));
+        for (int k = 0; k < rest; ++k)
+            hipLaunchKernelGGL(b->kern.bstep, dim3(b->grid), dim3(b->block), b->lds, st, Ps, blk, k);
+        HIPCHECK(hipGetLastError());
     }
     HIPCHECK(hipEventRecord(b->ev1, st));
     hipLaunchKernelGGL(k_batch_publish, dim3(nrep), dim3(256), 0, st, Ps);
@@ -2762,9 +2753,9 @@ int gmd_batch_fetch(gmd_batch *b) {
     for (const gmd_ctx *c : b->reps)
         if (c->xcap < XferSeg((size_t)c->d.N, (size_t)std::max(0, c->d.nscalars)).end)
             return 0;   // a large replica: each is brought by its own gmd_download
-    hipLaunchKernelGGL(k_batch_unpack, dim3(gx, nrep), dim3(256), 0, b->stream, (const DP *const *)b->d_Ps,
+    hipLaunchKernelGGL(k_batch_unpack, dim3(gx, nrep), dim3(256), 0, b->stream, (const DP *)b->d_Ps,
                        (const RunStart *)b->h_start);
-    hipLaunchKernelGGL(k_batch_fetch, dim3(gx, nrep), dim3(256), 0, b->stream, (const DP *const *)b->d_Ps);
+    hipLaunchKernelGGL(k_batch_fetch, dim3(gx, nrep), dim3(256), 0, b->stream, (const DP *)b->d_Ps);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(b->stream));
     for (gmd_ctx *c : b->reps) c->fetched = true;

@@ -54,10 +54,8 @@ struct Ctrl {
     unsigned red_count;        // last-block counter (kernel-per-phase path)
     unsigned bar_count;        // grid barrier arrival counter
     unsigned bar_gen;          // grid barrier generation
-    int step;                  // current step (kernel-per-phase path)
     int nsteps;
     int buf0;                  // position buffer holding r at step 0 of the run
-    int rebuild_now;           // rebuild before the interactions of 'step'
     float t0;
     int cell_overflow;         // largest cell occupancy seen beyond the cell capacity
     long long lstep0;          // Langevin counter of step 0 of the run

@@ -1701,10 +1701,6 @@ __device__ __forceinline__ void npt_publish(const DP &P, const StepInfo &J, int 
 
 __device__ inline void step_tail(const DP &P, const StepInfo &I, double *red, const int nblocks) {
     GMEM Ctrl *C = P.ctrl;
-    // the rebuild flag thread 0 publishes at the end is loaded first, so the
-    // load overlaps with the reduction (rebuild_flag holds nsteps+2 entries)
-    int next_flag = 0;
-    if (threadIdx.x == 0) next_flag = ld_flag(P.rebuild_flag + I.s + 1);
     const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
     float v[RED_PRE][GMD_NRED];
     load_partials(P, P.partial, nblocks, mask, v);
@@ -1731,8 +1727,6 @@ __device__ inline void step_tail(const DP &P, const StepInfo &I, double *red, co
         }
         if (I.need_save) saver_row(P, I.s, tot, vol);
         if (I.rebuild) C->nbflag[2] += 1;
-        C->rebuild_now = (I.s < I.nsteps) ? next_flag : 0;
-        C->step = I.s + 1;
     }
     __syncthreads();
 }

@@ -10,16 +10,6 @@
 // ============================================================================
 // Every step of a run inside one launch; the blocks of one system meet at a
 // software barrier after each step, and the last to arrive runs the tail.
-// a pointer that is the same in every lane, made visibly uniform (loads
-// through it become scalar loads)
-template <typename T>
-__device__ __forceinline__ T *uniform_ptr(T *p) {
-    const unsigned long long v = (unsigned long long)p;
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-    return (T *)(((unsigned long long)hi << 32) | lo);
-}
-
 template <int BASE, int CUT, int INTEG, int KIND>
 __device__ __forceinline__ void persistent_body(const DP *Pp, const BlockCtx &B) {
     extern __shared__ __align__(16) char lds[];
@@ -43,26 +33,23 @@ __device__ __forceinline__ void persistent_body(const DP *Pp, const BlockCtx &B)
     }
 }
 
-// One step.  FOLD (one system): the step is s_base + k, the rebuild decision
-// is the flag the previous step raised, and the previous step's tail runs in
-// every block here (folded_tail); the partial sums alternate between two
-// buffers.  Otherwise (replicas of a batch) the step index and the rebuild
-// decision come from the control block that the previous step's k_batch_tail
-// wrote.
-template <int BASE, int CUT, int INTEG, int KIND, bool FOLD>
+// One step, s_base + k: the rebuild decision is the flag the previous step
+// raised, and the previous step's tail runs in every block of the system here
+// (folded_tail); the partial sums alternate between two buffers.
+template <int BASE, int CUT, int INTEG, int KIND>
 __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k) {
     extern __shared__ __align__(16) char lds[];
-    const int s = FOLD ? P.ctrl->s_base + k : P.ctrl->step;
+    const int s = P.ctrl->s_base + k;
     if (s > P.ctrl->nsteps) return;
-    const bool rebuild = FOLD ? ld_flag(P.rebuild_flag + s) != 0 : P.ctrl->rebuild_now != 0;
+    const bool rebuild = ld_flag(P.rebuild_flag + s) != 0;
     PairP *pp = (PairP *)(lds + P.lds_pp);
     double *red = (double *)(lds + P.lds_red);
     char *build = lds + P.lds_build;
-    StepInfo I = step_info(P, s, INTEG, rebuild, FOLD);
+    StepInfo I = step_info(P, s, INTEG, rebuild, true);
     // the previous step's sums (only the components its tail needs) and the
     // pair table, then the step itself
-    const unsigned qmask = FOLD ? folded_tail_mask<INTEG>(P, I) : 0u;
-    if (INTEG == 2 && FOLD && !rebuild && !I.scal && qmask == (1u << RED_K) &&
+    const unsigned qmask = folded_tail_mask<INTEG>(P, I);
+    if (INTEG == 2 && !rebuild && !I.scal && qmask == (1u << RED_K) &&
         P.step_grid <= RED_PRE * (int)blockDim.x) {
         // a Nose-Hoover list step whose tail needs only the kinetic sum: the
         // partials go to LDS by DMA now and are summed after the first
@@ -122,14 +109,14 @@ __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k)
         return;
     }
     float pv[RED_PRE][GMD_NRED];
-    if (FOLD && (qmask & ~(1u << RED_K)) == 0u) {
+    if ((qmask & ~(1u << RED_K)) == 0u) {
         folded_tail_load<INTEG, 1u << RED_K>(P, I, qmask, pv);
         load_pair_table(P, pp);
         folded_tail<INTEG, 1u << RED_K>(P, B, I, red, qmask, pv);
     } else {
-        if (FOLD) folded_tail_load<INTEG, RED_ALL>(P, I, qmask, pv);
+        folded_tail_load<INTEG, RED_ALL>(P, I, qmask, pv);
         load_pair_table(P, pp);
-        if (FOLD) folded_tail<INTEG, RED_ALL>(P, B, I, red, qmask, pv);
+        folded_tail<INTEG, RED_ALL>(P, B, I, red, qmask, pv);
     }
     __syncthreads();
     float acc[GMD_NRED];
@@ -137,8 +124,8 @@ __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k)
     for (int c = 0; c < GMD_NRED; ++c) acc[c] = 0.f;
     step_body<BASE, CUT, INTEG, KIND>(P, B, I, pp, build, acc);
     const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
-    if (mask) block_partials(P, B, acc, red, FOLD ? P.partial + (size_t)(s & 1) * GMD_NRED * P.pstride : P.partial, mask);
-    if (FOLD && rebuild && B.bid == 0 && threadIdx.x == 0) P.ctrl->nbflag[2] += 1;
+    if (mask) block_partials(P, B, acc, red, P.partial + (size_t)(s & 1) * GMD_NRED * P.pstride, mask);
+    if (rebuild && B.bid == 0 && threadIdx.x == 0) P.ctrl->nbflag[2] += 1;
 }
 
 // The blocks of a launch go to the 8 XCDs in turn (block b to XCD b % 8).
@@ -163,7 +150,7 @@ __global__ void __launch_bounds__(256) k_persistent(const DP *__restrict__ Pp) {
 // blocks still running).
 template <int BASE, int CUT, int INTEG, int KIND>
 __global__ void __launch_bounds__(256, 4) k_step(const DP *__restrict__ Pp, int k) {
-    step_once<BASE, CUT, INTEG, KIND, true>(*Pp, xcd_block((int)blockIdx.x, (int)gridDim.x), k);
+    step_once<BASE, CUT, INTEG, KIND>(*Pp, xcd_block((int)blockIdx.x, (int)gridDim.x), k);
 }
 
 // Batched replicas: block b of the grid works for replica blk[b].rep as its
@@ -174,22 +161,27 @@ struct BatchBlk {
 };
 
 template <int BASE, int CUT, int INTEG>
-__global__ void __launch_bounds__(256) k_batch_persistent(const DP *const *Ps, const BatchBlk *blks) {
+__global__ void __launch_bounds__(256) k_batch_persistent(const DP *__restrict__ Ps, const BatchBlk *blks) {
     const BatchBlk a = blks[blockIdx.x];
     const int rep = __builtin_amdgcn_readfirstlane(a.rep);
     if (rep < 0) return;
     const BlockCtx B = {__builtin_amdgcn_readfirstlane(a.bid), __builtin_amdgcn_readfirstlane(a.nb)};
-    persistent_body<BASE, CUT, INTEG, 2>(uniform_ptr(Ps[rep]), B);
+    persistent_body<BASE, CUT, INTEG, 2>(Ps + rep, B);
 }
 
-// (at most 168 VGPRs: three wavefronts per SIMD)
+// One step of every replica, with the previous step's tails folded in as in
+// k_step.  The replicas' descriptors lie one after another behind one
+// restrict pointer, as k_step's does: read through a table of pointers they
+// took vector loads and the kernel 168 VGPRs; now scalar loads and 128, four
+// wavefronts per SIMD instead of three (64 KA replicas of 1000 to 8000, with
+// the tails no longer a launch of their own: 290 -> 236 us a step).
 template <int BASE, int CUT, int INTEG>
-__global__ void __launch_bounds__(256, 3) k_batch_step(const DP *const *Ps, const BatchBlk *blks) {
+__global__ void __launch_bounds__(256, 4) k_batch_step(const DP *__restrict__ Ps, const BatchBlk *blks, int k) {
     const BatchBlk a = blks[blockIdx.x];
     const int rep = __builtin_amdgcn_readfirstlane(a.rep);
     if (rep < 0) return;
     const BlockCtx B = {__builtin_amdgcn_readfirstlane(a.bid), __builtin_amdgcn_readfirstlane(a.nb)};
-    step_once<BASE, CUT, INTEG, 2, false>(*uniform_ptr(Ps[rep]), B, 0);
+    step_once<BASE, CUT, INTEG, 2>(Ps[rep], B, k);
 }
 
 
@@ -200,8 +192,8 @@ __global__ void __launch_bounds__(256, 3) k_batch_step(const DP *const *Ps, cons
     EXT template __global__ void k_persistent<B, C, I, 1>(const DP *);                           \
     EXT template __global__ void k_step<B, C, I, 0>(const DP *, int);                            \
     EXT template __global__ void k_step<B, C, I, 1>(const DP *, int);                            \
-    EXT template __global__ void k_batch_persistent<B, C, I>(const DP *const *, const BatchBlk *); \
-    EXT template __global__ void k_batch_step<B, C, I>(const DP *const *, const BatchBlk *);
+    EXT template __global__ void k_batch_persistent<B, C, I>(const DP *, const BatchBlk *); \
+    EXT template __global__ void k_batch_step<B, C, I>(const DP *, const BatchBlk *, int);
 #define GMD_STEP_KERNELS_CUT(EXT, B, C) \
     GMD_STEP_KERNELS(EXT, B, C, 0)      \
     GMD_STEP_KERNELS(EXT, B, C, 1)      \

@@ -123,3 +123,33 @@ def test_autotune_runs_and_keeps_state():
         assert np.array_equal(r.configuration['r'], x)
     for _ in b.run_timeblocks():
         pass
+
+
+@pytest.mark.parametrize("steps", [17, 40])
+def test_batched_graph_tail(steps):
+    """The graph driver folds a step's sums (thermostat, momentum reset, saver
+    row) into the next step's launch: runs that end inside and on a captured
+    group of steps, against the same replicas one by one.  The sums agree to
+    float32 rounding (1e-7 of a position of up to 15), which 40 steps at these
+    temperatures grow by less than ten and add less than 40 times."""
+    actions = lambda: [gp.ScalarSaver(8), gp.MomentumReset(10)]  # noqa: E731
+    nvt = lambda T: gp.NVT(temperature=T, tau=0.2, dt=0.004)  # noqa: E731
+    reps, singles = _replicas(nvt), _replicas(nvt)
+    for r in reps:
+        r.runtime_actions = actions()
+    batch = gp.BatchedSimulation(reps, num_timeblocks=2, steps_per_timeblock=steps, tp=4, driver='graph')
+    for _ in batch.run_timeblocks():
+        pass
+    for (_, _, T), r, s, out in zip(SYSTEMS, reps, singles, batch.outputs):
+        conf = s.configuration
+        plan = dict(gp.batch.replica_plan(s, 4, 0.5), graph=True)
+        sim = gp.Simulation(conf, _pp(), nvt(T), actions(), num_timeblocks=2, steps_per_timeblock=steps,
+                            compute_plan=plan, storage='memory', steps_in_kernel_test=0)
+        sim.ctx.force_rebuild()
+        for _ in sim.run_timeblocks():
+            pass
+        d = conf['r'] - r.configuration['r']
+        L = conf.simbox.lengths
+        assert np.max(np.abs(d - L * np.round(d / L))) < 1e-4
+        assert np.max(np.abs(conf['v'] - r.configuration['v'])) < 1e-3
+        np.testing.assert_allclose(out["scalars"][:], sim.output["scalars"][:], rtol=1e-4, atol=1e-2)
