@@ -143,6 +143,7 @@ _SIGNATURES = {
                                        c_float_p]),
     "gmd_adj_backward": (ctypes.c_int, [ctypes.c_void_p, c_double_p, c_double_p, c_float_p, c_float_p]),
     "gmd_adj_last_ms": (ctypes.c_int, [ctypes.c_void_p, c_float_p, c_float_p]),
+    "gmd_adj_use_checkpoints": (ctypes.c_int, [ctypes.c_void_p]),
 }
 
 BATCH_DRIVER = {"persistent": 0, "graph": 1}

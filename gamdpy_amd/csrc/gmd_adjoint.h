@@ -633,6 +633,9 @@ struct gmd_adj {
     float4 *pos = nullptr, *pos2 = nullptr, *vel = nullptr, *rpart = nullptr, *rref = nullptr;
     int *nbl = nullptr, *nbc = nullptr, *flag = nullptr;
     int *rnbl = nullptr, *rnbc = nullptr;   // list of one frame (radius rmax + 5 w)
+    // the positions of every step (traj), or the checkpoints and one segment
+    // recomputed from its checkpoint (adj_storage)
+    float4 *traj = nullptr;
     float4 *ck_r = nullptr, *ck_v = nullptr, *seg = nullptr;
     float4 *lr = nullptr, *lv = nullptr, *w = nullptr, *w2 = nullptr;
     double *pgl = nullptr, *pgrad_tot = nullptr, *H = nullptr, *hacc = nullptr;
@@ -642,7 +645,7 @@ struct gmd_adj {
 static int adj_free(gmd_adj *a) {
     if (!a) return 0;
     void *ptrs[] = {a->pos, a->pos2, a->vel, a->rpart, a->rref, a->nbl, a->nbc, a->flag, a->rnbl, a->rnbc,
-                    a->ck_r, a->ck_v, a->seg, a->lr, a->lv, a->w, a->w2, a->pgl, a->pgrad_tot, a->H, a->hacc, a->G};
+                    a->traj, a->ck_r, a->ck_v, a->seg, a->lr, a->lv, a->w, a->w2, a->pgl, a->pgrad_tot, a->H, a->hacc, a->G};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (a->e0) hipEventDestroy(a->e0);
@@ -704,6 +707,34 @@ static int adj_set_params(gmd_adj *a, const float *params) {
     }
     a->K.maxnb = maxnb;
     return 0;
+}
+
+// The storage the backward pass reads the positions from.  A trajectory of up
+// to ADJ_TRAJ_BYTES stays in memory as the forward pass writes it: one buffer
+// of step after step, nothing copied and no step computed twice (N = 4096, 200
+// steps: 13 MB, and the backward pass 200 forward steps and ten list builds
+// shorter).  A longer one, or one the device has no room for, keeps a
+// checkpoint of positions and velocities every ckpt_every steps and recomputes
+// a segment at a time.
+#define ADJ_TRAJ_BYTES ((size_t)4 << 30)
+static hipError_t adj_storage(gmd_adj *a, bool whole) {
+    for (float4 **p : {&a->traj, &a->pos, &a->pos2, &a->ck_r, &a->ck_v, &a->seg}) {
+        if (*p) hipFree(*p);
+        *p = nullptr;
+    }
+    a->have_forward = false;
+    const size_t N = a->d.N, F = sizeof(float4);
+    if (whole) {
+        if (hipMalloc((void **)&a->traj, ((size_t)a->d.nsteps + 1) * N * F) == hipSuccess) return hipSuccess;
+        a->traj = nullptr;
+        (void)hipGetLastError();
+    }
+    hipError_t e = hipMalloc((void **)&a->pos, N * F);
+    if (e == hipSuccess) e = hipMalloc((void **)&a->pos2, N * F);
+    if (e == hipSuccess) e = hipMalloc((void **)&a->ck_r, (size_t)a->nck * N * F);
+    if (e == hipSuccess) e = hipMalloc((void **)&a->ck_v, (size_t)a->nck * N * F);
+    if (e == hipSuccess) e = hipMalloc((void **)&a->seg, (size_t)(a->d.ckpt_every + 1) * N * F);
+    return e;
 }
 
 extern "C" {
@@ -784,18 +815,14 @@ int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass
     ATRY(hipStreamCreateWithFlags(&a->stream, hipStreamNonBlocking));
     ATRY(hipEventCreate(&a->e0));
     ATRY(hipEventCreate(&a->e1));
-    ATRY(hipMalloc((void **)&a->pos, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->vel, N * sizeof(float4)));
-    ATRY(hipMalloc((void **)&a->pos2, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->rpart, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->rnbl, N * (size_t)a->rmaxnb * sizeof(int)));
     ATRY(hipMalloc((void **)&a->rnbc, N * sizeof(int)));
     ATRY(hipMalloc((void **)&a->rref, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->nbc, N * sizeof(int)));
     ATRY(hipMalloc((void **)&a->flag, 5 * sizeof(int)));   // skin flags of three steps, list overflows
-    ATRY(hipMalloc((void **)&a->ck_r, (size_t)a->nck * N * sizeof(float4)));
-    ATRY(hipMalloc((void **)&a->ck_v, (size_t)a->nck * N * sizeof(float4)));
-    ATRY(hipMalloc((void **)&a->seg, (size_t)(d.ckpt_every + 1) * N * sizeof(float4)));
+    ATRY(adj_storage(a, ((size_t)d.nsteps + 1) * N * sizeof(float4) <= ADJ_TRAJ_BYTES));
     ATRY(hipMalloc((void **)&a->lr, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->lv, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->w, N * sizeof(float4)));
@@ -811,6 +838,13 @@ int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass
 }
 
 int gmd_adj_destroy(gmd_adj *a) { return adj_free(a); }
+
+int gmd_adj_use_checkpoints(gmd_adj *a) {
+    if (!a) return fail("gmd_adj_use_checkpoints: null handle");
+    HIPCHECK(hipStreamSynchronize(a->stream));
+    HIPCHECK(adj_storage(a, false));
+    return 0;
+}
 
 // blocks of a list build: ADJ_BT / 64 particles each
 static dim3 adj_build_grid(const gmd_adj *a) { return dim3((a->K.N + ADJ_BT / 64 - 1) / (ADJ_BT / 64)); }
@@ -877,15 +911,15 @@ int gmd_adj_forward(gmd_adj *a, const float *params, const float *r0, const floa
         hv[i] = make_float4(v0[3 * i], v0[3 * i + 1], v0[3 * i + 2], a->mass[i]);
     }
     hipStream_t st = a->stream;
-    HIPCHECK(hipMemcpyAsync(a->pos, hr.data(), N * sizeof(float4), hipMemcpyHostToDevice, st));
+    float4 *cur = a->traj ? a->traj : a->pos, *nxt = a->traj ? a->traj + N : a->pos2;
+    HIPCHECK(hipMemcpyAsync(cur, hr.data(), N * sizeof(float4), hipMemcpyHostToDevice, st));
     HIPCHECK(hipMemcpyAsync(a->vel, hv.data(), N * sizeof(float4), hipMemcpyHostToDevice, st));
     const int nh = a->K.ncls * a->K.bins;
     HIPCHECK(hipMemsetAsync(a->hacc, 0, (size_t)a->gl * nh * sizeof(double), st));
     if (adj_reset_lists(a)) return -1;
-    float4 *cur = a->pos, *nxt = a->pos2;
     HIPCHECK(hipEventRecord(a->e0, st));
     for (int n = 0; n < S; ++n) {
-        if (n % C == 0) {
+        if (!a->traj && n % C == 0) {
             HIPCHECK(hipMemcpyAsync(a->ck_r + (size_t)(n / C) * N, cur, N * sizeof(float4),
                                     hipMemcpyDeviceToDevice, st));
             HIPCHECK(hipMemcpyAsync(a->ck_v + (size_t)(n / C) * N, a->vel, N * sizeof(float4),
@@ -893,7 +927,12 @@ int gmd_adj_forward(gmd_adj *a, const float *params, const float *r0, const floa
         }
         if (n % E == 0) adj_rdf_frame(a, cur);
         adj_step(a, cur, nxt, n % C == 0);
-        std::swap(cur, nxt);
+        if (a->traj) {
+            cur = nxt;
+            nxt += N;
+        } else {
+            std::swap(cur, nxt);
+        }
     }
     if (S % E == 0) adj_rdf_frame(a, cur);
     hipLaunchKernelGGL(k_adj_sum, dim3(nh), dim3(256), 0, st, (const double *)a->hacc, a->gl, nh, a->H);
@@ -936,26 +975,31 @@ int gmd_adj_backward(gmd_adj *a, const double *dLdH, double *grad_params, float 
     if (adj_reset_lists(a)) return -1;
     HIPCHECK(hipEventRecord(a->e0, st));
     const dim3 gu((N + 255) / 256);
-    // lambda_r(S) = dL/dr_S, then lambda_v, w of step S-1; recompute r_S from the last checkpoint first
+    // lambda_r(S) = dL/dr_S, then lambda_v, w of step S-1; the last segment also provides r_S
     const int last = a->nck - 1;
-    // recompute the last segment (it also provides r_S)
     float4 *w = a->w, *wn = a->w2;
     for (int sgm = last; sgm >= 0; --sgm) {
         const int n0 = sgm * C, n1 = std::min(S, n0 + C);
-        HIPCHECK(hipMemcpyAsync(a->vel, a->ck_v + (size_t)sgm * N, N * sizeof(float4), hipMemcpyDeviceToDevice, st));
-        HIPCHECK(hipMemcpyAsync(a->seg, a->ck_r + (size_t)sgm * N, N * sizeof(float4), hipMemcpyDeviceToDevice, st));
-        // the segment's steps repeat the forward's: the list is rebuilt at the
-        // checkpoint as it was there
-        for (int k = 0; k < n1 - n0; ++k) adj_step(a, a->seg + (size_t)k * N, a->seg + (size_t)(k + 1) * N, k == 0);
+        const float4 *seg = a->traj ? a->traj + (size_t)n0 * N : a->seg;   // r_n0 .. r_n1
+        if (!a->traj) {
+            HIPCHECK(hipMemcpyAsync(a->vel, a->ck_v + (size_t)sgm * N, N * sizeof(float4), hipMemcpyDeviceToDevice,
+                                    st));
+            HIPCHECK(hipMemcpyAsync(a->seg, a->ck_r + (size_t)sgm * N, N * sizeof(float4), hipMemcpyDeviceToDevice,
+                                    st));
+            // the segment's steps repeat the forward's: the list is rebuilt at
+            // the checkpoint as it was there
+            for (int k = 0; k < n1 - n0; ++k)
+                adj_step(a, a->seg + (size_t)k * N, a->seg + (size_t)(k + 1) * N, k == 0);
+        }
         if (sgm == last) {
             // start of the adjoint: frame gradient at r_S, then lambda_v and w of step S-1
-            const float4 *rS = a->seg + (size_t)(n1 - n0) * N;
+            const float4 *rS = seg + (size_t)(n1 - n0) * N;
             if (S % E == 0) adj_rdf_grad(a, rS);
             hipLaunchKernelGGL(k_adj_start, gu, dim3(256), 0, st, a->K, (const float4 *)a->vel, a->lr, a->lv, w,
                                (const float4 *)(S % E == 0 ? a->rpart : nullptr));
         }
         for (int n = n1 - 1; n >= n0; --n) {
-            const float4 *rn = a->seg + (size_t)(n - n0) * N;
+            const float4 *rn = seg + (size_t)(n - n0) * N;
             const AdjLists A = adj_lists(a, rn, n == n1 - 1);
             if (n % E == 0) adj_rdf_grad(a, rn);
             // the positions of step n-1 (same segment) take their skin check here

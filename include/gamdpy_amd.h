@@ -318,6 +318,10 @@ int gmd_adj_forward(gmd_adj *adj, const float *params, const float *r0, const fl
  * class); grad_r0, grad_v0 (N,3) (grad_v0 may be NULL) */
 int gmd_adj_backward(gmd_adj *adj, const double *dLdH, double *grad_params, float *grad_r0, float *grad_v0);
 int gmd_adj_last_ms(gmd_adj *adj, float *fwd_ms, float *bwd_ms);
+/* keep checkpoints only, as a trajectory too long for device memory does, and
+ * recompute between them in the backward pass (same results; a forward pass
+ * before the call is dropped) */
+int gmd_adj_use_checkpoints(gmd_adj *adj);
 
 #ifdef __cplusplus
 }

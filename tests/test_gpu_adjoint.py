@@ -173,3 +173,26 @@ def test_forward_histogram_at_list_tile_edges(N, shuffled):
     Hc = _c_hist(conf, np.array(KA_SIG), np.array(KA_EPS), cut, traj)
     print(N, np.abs(H - Hc).max(), Hc.max())
     assert np.abs(H - Hc).max() <= 1e-3 * Hc.max()
+
+
+@pytest.mark.parametrize("nsteps,ckpt", [(23, 5), (20, 20), (7, 40), (1, 1)])
+def test_checkpoints_and_whole_trajectory_agree(nsteps, ckpt):
+    """The gradient from the stored positions of every step and from segments
+    recomputed between checkpoints: the same steps on the same lists, the same
+    bits, also of a second backward pass."""
+    conf = _ka([5, 5, 5], 1.2, 2.0, seed=2)
+    traj = dict(dt=0.004, nsteps=nsteps, ckpt_every=ckpt, rdf_every=5, bins=60, rmax=2.4, width=0.03)
+    got = []
+    for whole in (True, False):
+        m, _ = _model(conf, traj)
+        if not whole:
+            gp._native.check(m.engine.lib.gmd_adj_use_checkpoints(m.engine.h), "gmd_adj_use_checkpoints")
+        r0 = torch.tensor(conf['r'], requires_grad=True)
+        sig, eps = (torch.tensor(x, dtype=torch.float32, requires_grad=True) for x in (KA_SIG, KA_EPS))
+        H = m.histogram(r0, sig, eps)
+        for _ in range(2):
+            g = torch.autograd.grad((H * H).sum(), (r0, sig, eps), retain_graph=True)
+            got.append([H.detach().numpy()] + [x.numpy() for x in g])
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            np.testing.assert_array_equal(a, b)
