@@ -753,27 +753,61 @@ __global__ void __launch_bounds__(256) k_sort_count(const DP *__restrict__ Pp, i
     }
 }
 
-// exclusive prefix sum of a[0, n) in place (one block of 1024 threads)
-__global__ void __launch_bounds__(1024) k_scan(int *a, int n) {
-    __shared__ int part[1024];
-    const int t = threadIdx.x;
-    const int per = (n + 1023) / 1024;
-    const int b = min(n, t * per), e = min(n, b + per);
-    int sum = 0;
-    for (int k = b; k < e; ++k) sum += a[k];
-    part[t] = sum;
+// Exclusive prefix sum of the key counts in place: the sums of chunks of
+// SCAN_CHUNK counts, then each block scans its chunk on top of the sums before
+// it.  (One block over all counts read each thread's run of counts alone, one
+// load after another: LJ N = 1048576, 2097152 keys, 3650 us a renumbering.)
+#define SCAN_CHUNK 4096
+__device__ __forceinline__ int scan_block_sum(int v, int *red) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const int v = (t >= o) ? part[t - o] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+    v = red[0] + red[1] + red[2] + red[3];
+    __syncthreads();
+    return v;
+}
+
+__global__ void __launch_bounds__(256) k_scan_sums(const int *a, int n, int *sums) {
+    __shared__ int red[4];
+    const int b = blockIdx.x * SCAN_CHUNK;
+    int s = 0;
+#pragma unroll
+    for (int u = 0; u < SCAN_CHUNK / 256; ++u) {
+        const int k = b + u * 256 + (int)threadIdx.x;
+        if (k < n) s += a[k];
     }
-    int run = part[t] - sum;
-    for (int k = b; k < e; ++k) {
-        const int v = a[k];
-        a[k] = run;
-        run += v;
+    s = scan_block_sum(s, red);
+    if (threadIdx.x == 0) sums[blockIdx.x] = s;
+}
+
+__global__ void __launch_bounds__(256) k_scan(int *a, int n, const int *sums) {
+    __shared__ int red[4];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    int before = 0;
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += 256) before += sums[k];
+    before = scan_block_sum(before, red);
+    // a thread's run of counts
+    constexpr int R = SCAN_CHUNK / 256;
+    const int k0 = blockIdx.x * SCAN_CHUNK + (int)threadIdx.x * R;
+    int v[R], s = 0;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+        v[u] = k0 + u < n ? a[k0 + u] : 0;
+        s += v[u];
+    }
+    int inc = s;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    if (lane == 63) red[wid] = inc;
+    __syncthreads();
+    int base = before + inc - s;
+    for (int x = 0; x < wid; ++x) base += red[x];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+        if (k0 + u < n) a[k0 + u] = base;
+        base += v[u];
     }
 }
 
@@ -1031,7 +1065,7 @@ struct gmd_ctx {
     size_t nbl_len = 0;          // words of the neighbour list
     bool nb16 = false;           // 16-bit list entries
     // renumbering in cell order
-    int *perm = nullptr, *skey = nullptr, *sorder = nullptr, *scnt = nullptr, *scur = nullptr;
+    int *perm = nullptr, *skey = nullptr, *sorder = nullptr, *scnt = nullptr, *scur = nullptr, *ssum = nullptr;
     PermBufs tb = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     int nkeys = 0;                // Morton key space of the renumbering
     int reorder_every = 0;        // steps between renumberings (0: never)
@@ -1347,6 +1381,7 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
         c->nkeys = side * side * side;
         A.add(&c->scnt, (size_t)c->nkeys);
         A.add(&c->scur, (size_t)c->nkeys);
+        A.add(&c->ssum, (size_t)(c->nkeys + SCAN_CHUNK - 1) / SCAN_CHUNK);   // key counts of each chunk
         A.add(&c->tb.vel, N);
         A.add(&c->tb.frc, N);
         A.add(&c->tb.rref, N);
@@ -1752,7 +1787,9 @@ static int reorder(gmd_ctx *c) {
     const int gridc = std::max(1, std::min((nc + 255) / 256, c->cus * 8));
     HIPCHECK(hipMemsetAsync(c->scnt, 0, (size_t)nc * sizeof(int), st));
     hipLaunchKernelGGL(k_sort_count, dim3(grid), dim3(256), 0, st, (const DP *)c->d_P, c->buf0, c->skey, c->scnt);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, c->scnt, nc);
+    const int chunks = (nc + SCAN_CHUNK - 1) / SCAN_CHUNK;
+    hipLaunchKernelGGL(k_scan_sums, dim3(chunks), dim3(256), 0, st, (const int *)c->scnt, nc, c->ssum);
+    hipLaunchKernelGGL(k_scan, dim3(chunks), dim3(256), 0, st, c->scnt, nc, (const int *)c->ssum);
     HIPCHECK(hipMemcpyAsync(c->scur, c->scnt, (size_t)nc * sizeof(int), hipMemcpyDeviceToDevice, st));
     hipLaunchKernelGGL(k_sort_scatter, dim3(grid), dim3(256), 0, st, N, (const int *)c->skey, c->scur, c->sorder);
     hipLaunchKernelGGL(k_sort_cells, dim3(gridc), dim3(256), 0, st, (const int *)c->scnt, nc, N, c->sorder);
