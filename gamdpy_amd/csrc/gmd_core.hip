@@ -38,6 +38,47 @@ __global__ void __launch_bounds__(256) k_batch_advance(const DP *__restrict__ Ps
     if (r < nrep) Ps[r].ctrl->s_base += n;
 }
 
+// The kinetic sums of the replicas whose step was a split rebuild (step_once),
+// in the grouping of an unsplit one, bit for bit: block b's wavefront w adds up
+// cell after cell (particle after particle) of those it would have taken.
+__global__ void __launch_bounds__(256) k_batch_ksum(const DP *__restrict__ Ps, int k) {
+    const DP &P = Ps[blockIdx.y];
+    const int s = P.ctrl->s_base + k;
+    if (P.rebuild_grid <= P.step_grid || s >= P.ctrl->nsteps || ld_flag(P.rebuild_flag + s) == 0) return;
+    const StepInfo I = step_info(P, s, GMD_NVT, true, true);
+    if (red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum) != (1u << RED_K)) return;
+    __shared__ double red[4 * GMD_NRED];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, wpb = blockDim.x >> 6;
+    const int nb = P.step_grid, stride = nb * wpb;
+    for (int b = blockIdx.x; b < nb; b += gridDim.x) {
+        float acc[GMD_NRED];
+#pragma unroll
+        for (int c = 0; c < GMD_NRED; ++c) acc[c] = 0.f;
+        constexpr int U = 8;   // loads in flight
+        if (P.nblist_kind == 1) {
+            for (int c = b * wpb + wid; c < P.ncells; c += U * stride) {
+                float v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    v[u] = c + u * stride < P.ncells && lane < P.ccap ? P.kcell[(size_t)(c + u * stride) * P.ccap + lane]
+                                                                      : 0.f;
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc[RED_K] += v[u];
+            }
+        } else {
+            // 64 rounds at a time, added up in lane 0
+            for (int i0 = b * wpb + wid; i0 < P.N; i0 += 64 * stride) {
+                const float v = i0 + lane * stride < P.N ? P.kcell[i0 + lane * stride] : 0.f;
+                for (int u = 0; u < 64; ++u) {
+                    const float x = lane_f(v, u);
+                    if (lane == 0) acc[RED_K] += x;
+                }
+            }
+        }
+        block_partials(P, BlockCtx{b, nb}, acc, red, P.partial + (size_t)(s & 1) * GMD_NRED * P.pstride, 1u << RED_K);
+    }
+}
+
 // ---- run set-up: cell grid of the starting positions and the skin test ----
 // Kernel parameters are generic pointers (an address-space qualifier would
 // change the kernel's mangled name between the host and device passes).
@@ -1555,7 +1596,7 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     P.lds_pp = (int)lds_pp;
     P.lds_red = (int)lds_red;
     P.lds_build = (int)lds_b;
-    P.step_grid = c->grid_step;
+    P.step_grid = P.rebuild_grid = c->grid_step;
     P.perm = (const GMEM int *)c->perm;
     P.xdev = (GMEM int *)c->xdev;
     P.xhost = c->xhost;
@@ -2569,6 +2610,8 @@ struct gmd_batch {
     RunStart *h_start = nullptr;   // pinned: what each replica's run starts from (read by the kernels)
     BatchBlk *d_blk = nullptr;
     DP *d_Ps = nullptr;            // the replicas' DP, one after another (each context's d_P points here)
+    float *d_kcell = nullptr;      // the replicas' DP::kcell
+    int gk = 1;                    // blocks a replica of k_batch_ksum
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     float last_ms = 0.f;
@@ -2583,6 +2626,7 @@ static int batch_free(gmd_batch *b) {
     if (b->h_start) hipHostFree(b->h_start);
     if (b->d_blk) hipFree(b->d_blk);
     if (b->d_Ps) hipFree(b->d_Ps);
+    if (b->d_kcell) hipFree(b->d_kcell);
     if (b->ev0) hipEventDestroy(b->ev0);
     if (b->ev1) hipEventDestroy(b->ev1);
     if (b->stream) hipStreamDestroy(b->stream);
@@ -2596,7 +2640,10 @@ static int batch_free(gmd_batch *b) {
 // each into the fullest bin that still holds it whole (its positions and
 // lists then live in one XCD's L2); a replica that fits no bin whole is
 // spread over the emptiest bins.  At most 7 slots stay idle (rep = -1).
-static void batch_layout(const std::vector<int> &nb, std::vector<BatchBlk> &out) {
+// Within a bin the blocks past a replica's list steps (nlist) come first: they
+// work on rebuild steps only, the longest a block has, and start with the
+// launch.
+static void batch_layout(const std::vector<int> &nb, const std::vector<int> &nlist, std::vector<BatchBlk> &out) {
     const int NX = 8;
     long long total = 0;
     for (int n : nb) total += n;
@@ -2623,9 +2670,24 @@ static void batch_layout(const std::vector<int> &nb, std::vector<BatchBlk> &out)
             while (k < nb[r] && (long long)bins[x].size() < T) bins[x].push_back(BatchBlk{r, k++, nb[r], 0});
         }
     }
+    for (std::vector<BatchBlk> &bin : bins)
+        std::stable_partition(bin.begin(), bin.end(), [&](const BatchBlk &a) { return a.bid >= nlist[a.rep]; });
     out.assign((size_t)T * NX, BatchBlk{-1, 0, 0, 0});
     for (int x = 0; x < NX; ++x)
         for (size_t k = 0; k < bins[x].size(); ++k) out[k * NX + x] = bins[x][k];
+}
+
+// Blocks of a replica's split rebuild steps: a wavefront for every cell (or
+// NSQ_PP particles of an N-squared list) where the batch leaves the device that
+// room, else for every two.  Before and after the split: 64 KA replicas of 1000
+// to 8000 particles, tp = 2 (8 to 63 blocks a list step), 20.8 -> 18.0 ms for
+// 64 steps; a batch of few replicas 8.9 -> 4.3 ms.  (The steps alone, with a
+// wavefront for every cell of the 64 12.9 ms, for two 12.6, for three 13.0.)
+static int rebuild_blocks(const gmd_ctx *c, int nrep) {
+    const int wpb = c->block / 64;
+    const int units = c->d.nblist_kind == GMD_NBLIST_LINKED_LISTS ? c->P.ncells : (c->d.N + NSQ_PP - 1) / NSQ_PP;
+    const int every = (units + wpb - 1) / wpb;
+    return std::min(std::min(every, std::max((every + 1) / 2, c->cus * 4 / nrep)), c->cus * 4);
 }
 
 int gmd_batch_create(const gmd_desc *descs, int nrep, const int *blocks, int driver, gmd_batch **out) {
@@ -2676,15 +2738,43 @@ int gmd_batch_create(const gmd_desc *descs, int nrep, const int *blocks, int dri
             batch_free(b);
             return fail("gmd_batch_create: replica %d: %d blocks requested, allowed 1..%d", r, nb[r], cap);
         }
-        c->P.step_grid = nb[r];
+        c->P.step_grid = c->P.rebuild_grid = nb[r];
         c->d_P = b->d_Ps + r;
-        BTRY(hipMemcpy(c->d_P, &c->P, sizeof(DP), hipMemcpyHostToDevice));
         b->lds = std::max(b->lds, c->lds_step);
         b->block = c->block;
         b->cus = c->cus;
     }
     b->kern = b->reps[0]->kern;
-    batch_layout(nb, b->h_blk);
+    // Rebuild steps are split where the list steps of all replicas fill the
+    // device at most three times over (16 wavefronts a CU): a step then waits
+    // for its rebuilding replicas.  In more rounds than that their time is
+    // hidden behind the others' and the extra blocks only cost (gains and
+    // losses of the steps' time, tp = 2: 2200 list blocks 18 %, 2800 29 %;
+    // 5000 -4 %, 18000 -6 %).
+    long long blocks_all = 0;
+    for (int n : nb) blocks_all += n;
+    const std::vector<int> nlist = nb;
+    if (driver == GMD_BATCH_GRAPH && blocks_all <= 3LL * 4 * b->cus) {
+        std::vector<size_t> kat(nrep, 0);
+        size_t kn = 0;
+        for (int r = 0; r < nrep; ++r) {
+            DP &P = b->reps[r]->P;
+            P.rebuild_grid = std::max(nb[r], rebuild_blocks(b->reps[r], nrep));
+            b->gk = std::max(b->gk, std::min(P.step_grid, 16));
+            kat[r] = kn;
+            kn += P.nblist_kind == 1 ? (size_t)P.ncells * P.ccap : (size_t)P.N;
+        }
+        if (b->integrator == GMD_NVT) {
+            BTRY(hipMalloc((void **)&b->d_kcell, kn * sizeof(float)));
+            for (int r = 0; r < nrep; ++r) b->reps[r]->P.kcell = (GMEM float *)(b->d_kcell + kat[r]);
+        }
+    }
+    for (int r = 0; r < nrep; ++r) {
+        gmd_ctx *c = b->reps[r];
+        nb[r] = c->P.rebuild_grid;
+        BTRY(hipMemcpy(c->d_P, &c->P, sizeof(DP), hipMemcpyHostToDevice));
+    }
+    batch_layout(nb, nlist, b->h_blk);
     b->grid = (int)b->h_blk.size();
     if (driver == GMD_BATCH_PERSISTENT) {
         int per_cu = 0;
@@ -2749,10 +2839,13 @@ int gmd_batch_run(gmd_batch *b, float time_zero, int steps) {
         HIPCHECK(hipLaunchCooperativeKernel((const void *)b->kern.bpers, dim3(b->grid), dim3(b->block), args,
                                             (unsigned)b->lds, st));
     } else {
+        auto step = [&](int k) {
+            hipLaunchKernelGGL(b->kern.bstep, dim3(b->grid), dim3(b->block), b->lds, st, Ps, blk, k);
+            if (b->d_kcell) hipLaunchKernelGGL(k_batch_ksum, dim3(b->gk, nrep), dim3(b->block), 0, st, Ps, k);
+        };
         if (!b->gexec) {
             HIPCHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            for (int k = 0; k < GRAPH_STEPS; ++k)
-                hipLaunchKernelGGL(b->kern.bstep, dim3(b->grid), dim3(b->block), b->lds, st, Ps, blk, k);
+            for (int k = 0; k < GRAPH_STEPS; ++k) step(k);
             hipLaunchKernelGGL(k_batch_advance, dim3((nrep + 255) / 256), dim3(256), 0, st, Ps, (int)nrep, GRAPH_STEPS);
             HIPCHECK(hipStreamEndCapture(st, &b->graph));
             HIPCHECK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
@@ -2760,8 +2853,7 @@ int gmd_batch_run(gmd_batch *b, float time_zero, int steps) {
         // as in run_impl: whole groups of steps, then the rest
         const int groups = (steps + 1) / GRAPH_STEPS, rest = (steps + 1) % GRAPH_STEPS;
         for (int g = 0; g < groups; ++g) HIPCHECK(hipGraphLaunch(b->gexec, st));
-        for (int k = 0; k < rest; ++k)
-            hipLaunchKernelGGL(b->kern.bstep, dim3(b->grid), dim3(b->block), b->lds, st, Ps, blk, k);
+        for (int k = 0; k < rest; ++k) step(k);
         HIPCHECK(hipGetLastError());
     }
     HIPCHECK(hipEventRecord(b->ev1, st));

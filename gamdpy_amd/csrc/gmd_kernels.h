@@ -19,9 +19,7 @@
 // barrier.  The step's tail finishes the deterministic reductions
 // (thermostat, momentum reset, scalar saver): in the persistent kernel one
 // block runs it after the grid barrier; in the kernel-per-step path every
-// block of the next step runs it (folded_tail); for batched replicas the
-// one-block-per-replica k_batch_tail runs it and publishes the rebuild
-// decision of the next step.
+// block of the next step (of its replica, in a batch) runs it (folded_tail).
 #pragma once
 #include "gmd_device.h"
 #include <type_traits>
@@ -196,6 +194,7 @@ struct StepInfo {
     bool need_wsum;
     bool scal;                 // U, W, lapU of this evaluation are wanted (saver step or no integration)
     int conf_idx;              // ConfigurationSaver save index of this step (-1: none)
+    bool ksplit;               // each particle's kinetic energy goes to P.kcell (a split rebuild step)
     bool wrapped;              // every position of the run lies in [-L/2, L/2] (else: minimum image always)
     bool apply_shift;
     float sh0, sh1, sh2;
@@ -311,6 +310,7 @@ __device__ __forceinline__ StepInfo step_info(const DP &P, int s, int integrator
     // last evaluation of a run (which does not integrate), by the host
     I.scal = I.need_save || !I.integrate || I.npt;   // NPT_Atomic: W every step
     // configuration_saver.py:118-127: block-local step 0 -> save 0, step 2^b -> save b + 1
+    I.ksplit = false;
     I.conf_idx = -1;
     if (P.conf_saves > 0) {
         if (s == 0)
@@ -1212,7 +1212,10 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
         const int na = min(cur.na, P.ccap);
         const int nb = (sb < 125) ? min(cur.nb, P.ccap) : 0;
         const int np = lane_i(na, 62);
-        if (np == 0) continue;
+        if (np == 0) {
+            if (I.ksplit && lane < P.ccap) P.kcell[(size_t)c * P.ccap + lane] = 0.f;
+            continue;
+        }
         // the cell's own particles in index order: lane q takes the q-th
         int rank = 0;
         for (int q = 0; q < np; ++q) rank += (lane_i(ownm, q) < ownm) ? 1 : 0;
@@ -1283,6 +1286,7 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
                                                    micm);
             done = pe;
         }
+        if (I.ksplit) acc[RED_K] = 0.f;
         if (myi >= 0) {
             P.nbc[myi] = mycount;
             P.rref[myi] = myr;
@@ -1293,6 +1297,7 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
             particle_finish<INTEG>(P, I, myi, myr, myv, myr, q6[0], q6[1], q6[2], q6[3] * 0.5f,
                                    q6[4] * (0.5f / 3.0f), q6[5], true, acc);
         }
+        if (I.ksplit && lane < P.ccap) P.kcell[(size_t)c * P.ccap + lane] = acc[RED_K];
     }
 }
 
@@ -1523,6 +1528,7 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
             if (P.boff) bond_terms(P, pos, iq, rq, L0, L1, L2, sx, sy, sz, su, sw, sl);
             particle_finish<INTEG>(P, I, iq, rq, vq, rq, sx, sy, sz, su * 0.5f, sw * (0.5f / 3.0f), sl, l16 == 0,
                                    part);
+            if (I.ksplit && l16 == 0) P.kcell[iq] = part[RED_K];
         }
         // the step's sums in lane 0, particle after particle
 #pragma unroll

@@ -36,16 +36,42 @@ __device__ __forceinline__ void persistent_body(const DP *Pp, const BlockCtx &B)
 // One step, s_base + k: the rebuild decision is the flag the previous step
 // raised, and the previous step's tail runs in every block of the system here
 // (folded_tail); the partial sums alternate between two buffers.
-template <int BASE, int CUT, int INTEG, int KIND>
-__device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k) {
+//
+// BATCH (a replica of a batch; B.bid: the block among those of its rebuild
+// steps): a rebuild step is split over rebuild_grid blocks, a list step works
+// in the first step_grid of them and the others leave at once.  A rebuild's
+// time is the number of cells (or particles) its wavefronts take one after
+// another, and in a batch most steps have some replica rebuilding while the
+// others wait for it.  The sums of a step are grouped by the wavefronts of
+// step_grid blocks, split or not, so that they keep their bits: a split step
+// leaves each particle's kinetic energy in P.kcell, and k_batch_ksum adds them
+// up in that grouping.  A step that needs other sums (momentum reset, saver
+// row, virial) is not split.
+template <int BASE, int CUT, int INTEG, int KIND, bool BATCH>
+__device__ __forceinline__ void step_once(const DP &P, BlockCtx B, int k) {
     extern __shared__ __align__(16) char lds[];
     const int s = P.ctrl->s_base + k;
     if (s > P.ctrl->nsteps) return;
-    const bool rebuild = ld_flag(P.rebuild_flag + s) != 0;
+    bool rebuild = ld_flag(P.rebuild_flag + s) != 0;
+    if (BATCH) {
+        // (visibly uniform: the grid and the loops over it stay in scalar registers)
+        rebuild = __builtin_amdgcn_readfirstlane(rebuild ? 1 : 0) != 0;
+        B.nb = P.step_grid;
+        if (!rebuild && B.bid >= B.nb) return;
+    }
     PairP *pp = (PairP *)(lds + P.lds_pp);
     double *red = (double *)(lds + P.lds_red);
     char *build = lds + P.lds_build;
     StepInfo I = step_info(P, s, INTEG, rebuild, true);
+    unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
+    if (BATCH && rebuild) {
+        if (P.rebuild_grid > P.step_grid && (mask & ~(1u << RED_K)) == 0u) {
+            B.nb = P.rebuild_grid;
+            I.ksplit = mask != 0u;
+            mask = 0u;
+        }
+        if (B.bid >= B.nb) return;
+    }
     // the previous step's sums (only the components its tail needs) and the
     // pair table, then the step itself
     const unsigned qmask = folded_tail_mask<INTEG>(P, I);
@@ -104,7 +130,6 @@ __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k)
         else
             particle_loop_deferred<BASE, CUT, INTEG, 2>(P, B, I, pp, acc, hook);
         step_cells_clear(P, B, I);
-        const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
         if (mask) block_partials(P, B, acc, red, P.partial + (size_t)(s & 1) * GMD_NRED * P.pstride, mask);
         return;
     }
@@ -123,7 +148,6 @@ __device__ __forceinline__ void step_once(const DP &P, const BlockCtx &B, int k)
 #pragma unroll
     for (int c = 0; c < GMD_NRED; ++c) acc[c] = 0.f;
     step_body<BASE, CUT, INTEG, KIND>(P, B, I, pp, build, acc);
-    const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
     if (mask) block_partials(P, B, acc, red, P.partial + (size_t)(s & 1) * GMD_NRED * P.pstride, mask);
     if (rebuild && B.bid == 0 && threadIdx.x == 0) P.ctrl->nbflag[2] += 1;
 }
@@ -150,7 +174,7 @@ __global__ void __launch_bounds__(256) k_persistent(const DP *__restrict__ Pp) {
 // blocks still running).
 template <int BASE, int CUT, int INTEG, int KIND>
 __global__ void __launch_bounds__(256, 4) k_step(const DP *__restrict__ Pp, int k) {
-    step_once<BASE, CUT, INTEG, KIND>(*Pp, xcd_block((int)blockIdx.x, (int)gridDim.x), k);
+    step_once<BASE, CUT, INTEG, KIND, false>(*Pp, xcd_block((int)blockIdx.x, (int)gridDim.x), k);
 }
 
 // Batched replicas: block b of the grid works for replica blk[b].rep as its
@@ -180,8 +204,7 @@ __global__ void __launch_bounds__(256, 4) k_batch_step(const DP *__restrict__ Ps
     const BatchBlk a = blks[blockIdx.x];
     const int rep = __builtin_amdgcn_readfirstlane(a.rep);
     if (rep < 0) return;
-    const BlockCtx B = {__builtin_amdgcn_readfirstlane(a.bid), __builtin_amdgcn_readfirstlane(a.nb)};
-    step_once<BASE, CUT, INTEG, 2>(Ps[rep], B, k);
+    step_once<BASE, CUT, INTEG, 2, true>(Ps[rep], BlockCtx{__builtin_amdgcn_readfirstlane(a.bid), 0}, k);
 }
 
 
