@@ -55,6 +55,7 @@ class AdjointEngine:
                                               ctypes.byref(h)), "gmd_adj_create")
         self.h = h
         self.nframes = len(range(0, int(nsteps) + 1, int(rdf_every)))
+        self.passes = 0   # forward passes begun: the library keeps the last one's trajectory only
 
     def close(self):
         if getattr(self, "h", None) is not None and self.h.value:
@@ -69,6 +70,7 @@ class AdjointEngine:
 
     def forward(self, params, r0, v0):
         """params (nt, nt, 3) float32 (sigma, epsilon, cut) -> H (ncls, bins) float64."""
+        self.passes += 1
         p = np.ascontiguousarray(params, dtype=np.float32).reshape(-1)
         r = np.ascontiguousarray(r0, dtype=np.float32)
         v = np.ascontiguousarray(v0, dtype=np.float32)
@@ -106,8 +108,11 @@ def _function():
             params[:, :, 0] = sigma.detach().cpu().numpy()
             params[:, :, 1] = epsilon.detach().cpu().numpy()
             params[:, :, 2] = cut
-            H = engine.forward(params, r0.detach().cpu().numpy(), v0)
+            # copies: the caller may change the arrays before the backward pass
+            ctx.inputs = params, np.array(r0.detach().cpu().numpy(), np.float32), np.array(v0, np.float32)
+            H = engine.forward(*ctx.inputs)
             ctx.engine = engine
+            ctx.passes = engine.passes
             ctx.meta = (r0.dtype, r0.device, sigma.dtype, sigma.device)
             return torch.as_tensor(H, dtype=torch.float64, device=r0.device)
 
@@ -115,6 +120,10 @@ def _function():
         def backward(ctx, gH):
             engine = ctx.engine
             rdt, rdev, sdt, sdev = ctx.meta
+            if ctx.passes != engine.passes:
+                # another forward pass has replaced this one's trajectory
+                engine.forward(*ctx.inputs)
+                ctx.passes = engine.passes
             gp, gr, _ = engine.backward(gH.detach().cpu().numpy().astype(np.float64))
             nt = engine.ntypes
             gs = np.zeros((nt, nt))

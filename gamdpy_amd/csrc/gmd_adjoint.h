@@ -900,6 +900,9 @@ static void adj_step(gmd_adj *a, const float4 *r, float4 *rn, bool build) {
 int gmd_adj_forward(gmd_adj *a, const float *params, const float *r0, const float *v0, double *H, float *r_end,
                     float *v_end) {
     if (!a || !params || !r0 || !v0 || !H) return fail("gmd_adj_forward: null argument");
+    // the stored pair constants and positions are overwritten from here on: a
+    // pass that fails leaves nothing to differentiate
+    a->have_forward = false;
     if (adj_set_params(a, params)) return -1;
     const int N = a->d.N, S = a->d.nsteps, C = a->d.ckpt_every, E = a->d.rdf_every;
     std::vector<float4> hr(N), hv(N);
