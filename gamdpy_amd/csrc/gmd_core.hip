@@ -623,7 +623,8 @@ __global__ void __launch_bounds__(256) k_rdf(RdfP R) {
             const float gx = rdf_gap(bi.x, hi.x, bj.x, hj.x, R.L0, R.rL0);
             const float gy = rdf_gap(bi.y, hi.y, bj.y, hj.y, R.L1, R.rL1);
             const float gz = rdf_gap(bi.z, hi.z, bj.z, hj.z, R.L2, R.rL2);
-            if (hj.x >= 0.f && !(gx * gx + gy * gy + gz * gz > R.skip2))
+            // (a box around a position that is not finite is not a number: never skipped)
+            if (!(hj.x < 0.f) && !(gx * gx + gy * gy + gz * gz > R.skip2))
                 code = rdf_dim_code(li.x, ui.x, lj.x, uj.x, R.L0) | (rdf_dim_code(li.y, ui.y, lj.y, uj.y, R.L1) << 2) |
                        (rdf_dim_code(li.z, ui.z, lj.z, uj.z, R.L2) << 4);
             if (code >= 0 && g / (RDF_CHUNK / RDF_GROUP) == I) code = 0x3f;   // its own chunk: the form with 'after'
