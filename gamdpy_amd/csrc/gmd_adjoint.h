@@ -66,6 +66,7 @@ struct AdjK {
     // observable
     int bins;
     float rmax, dr, wid, inv_w2, kfloor, rcut2;   // rcut = rmax + 5 w
+    float hup;                   // fixed point of the frame histograms: units of 2^-32 / hup (adj_weight_scale)
 };
 
 __device__ __forceinline__ int adj_type(float4 r) { return __float_as_int(r.w); }
@@ -484,10 +485,12 @@ __global__ void __launch_bounds__(256) k_adj_bstep(AdjK K, const float4 *r_p, co
 
 // smoothed pair histogram of one frame over its half list (each pair once) of radius
 // rmax + 5 w, K.tp lanes per particle, one LDS histogram per block added to
-// hacc[block][ncls * bins].  The histogram is in 64-bit fixed point (2^-32):
-// float atomics on LDS run at a third of a lane a cycle and CU here, 32-bit
-// integer ones at eight, and the integer sum is exact and the same in every
-// order.  KA N = 4096, rmax 4, 200 bins: 57 -> 16 us a frame.
+// hacc[block][ncls * bins].  The histogram is in 64-bit fixed point: float
+// atomics on LDS run at a third of a lane a cycle and CU here, 32-bit integer
+// ones at eight, and the sum of whole numbers is the same in every order.
+// KA N = 4096, rmax 4, 200 bins: 57 -> 16 us a frame.  A weight is the
+// difference of two floats of at least kfloor > 2^-19, so a whole number of
+// 2^-42: at hup = 2^10 it is added with all its bits.
 __global__ void __launch_bounds__(256) k_adj_rdf_list(AdjK K, const float4 *pos_p, const int *nbl_p, const int *nbc_p,
                                                       int maxnb, double *hacc_p) {
     __shared__ unsigned long long h[ADJ_MAX_CLS * ADJ_MAX_BINS];
@@ -513,13 +516,19 @@ __global__ void __launch_bounds__(256) k_adj_rdf_list(AdjK K, const float4 *pos_
                       for (int kb = k0; kb <= k1; ++kb) {
                           const float x = d - ((float)kb + 0.5f) * K.dr;
                           const float kv = __expf(-0.5f * x * x * K.inv_w2) - K.kfloor;
-                          if (kv > 0.f) atomicAdd(&h[c * K.bins + kb], (unsigned long long)(unsigned)(kv * 0x1p32f));
+                          if (kv > 0.f) {
+                              const float a = kv * K.hup;
+                              const unsigned long long hi = (unsigned)a;
+                              const unsigned lo = (unsigned)(__builtin_amdgcn_fractf(a) * 0x1p32f);
+                              atomicAdd(&h[c * K.bins + kb], hi << 32 | lo);
+                          }
                       }
                   });
     }
     __syncthreads();
     GMEM double *dst = (GMEM double *)hacc_p + (size_t)blockIdx.x * nh;
-    for (int t = threadIdx.x; t < nh; t += blockDim.x) dst[t] += (double)h[t] * 0x1p-32;
+    const double unit = 0x1p-32 / (double)K.hup;
+    for (int t = threadIdx.x; t < nh; t += blockDim.x) dst[t] += (double)h[t] * unit;
 }
 
 // dL/dr_i of one frame given G = dL/dH over the frame's list (all j of i):
@@ -658,6 +667,15 @@ static int adj_free(gmd_adj *a) {
 static int adj_cls(int a, int b, int nt) {
     if (a > b) std::swap(a, b);
     return a * nt - a * (a - 1) / 2 + (b - a);
+}
+
+// The upper word's scale of the frame histograms: 2^10, or the largest power
+// of two at which a block's 64-bit counters hold every pair of its lists (only
+// lists of more than 65536 entries leave less)
+static float adj_weight_scale(double pairs) {
+    float up = 1024.0f;
+    while (up > 1.0f && pairs * up >= 4294967296.0) up *= 0.5f;
+    return up;
 }
 
 // pair constants from (sigma, epsilon, cut) per ordered type pair
@@ -802,6 +820,7 @@ int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass
         a->rmaxnb = (int)std::min<double>((2.0 * nbar + 64.0 + 31.0) / 32.0 * 32.0, (double)d.N + 31.0);
         a->rmaxnb = a->rmaxnb / 32 * 32;
     }
+    K.hup = adj_weight_scale((double)(256 / K.tp) * a->rmaxnb);
     a->nck = (d.nsteps + d.ckpt_every - 1) / d.ckpt_every;
     const size_t N = d.N;
 #define ATRY(x)                                                               \
