@@ -141,7 +141,9 @@ __device__ __forceinline__ bool box_near(const AdjK &K, const float4 r, const fl
 // staged in LDS, the accepted j compacted with a ballot (ascending j; HALF:
 // each pair in one of its particles' lists, evenly, as niii_owns says); rref
 // (if given) receives the positions and *over records the longest list beyond
-// maxnb.  The tests are most of the work, so a tile comes with the boxes of
+// maxnb (HALF: the longest there would be with every j, so that a system whose
+// gradient needs longer lists than there is room for is refused by the forward
+// pass already).  The tests are most of the work, so a tile comes with the boxes of
 // its chunks of 64 positions (a wavefront each) and a particle tests only the
 // chunks whose box is near it: positions numbered along a lattice stay
 // together, and a numbering without order costs the boxes and gains nothing.
@@ -159,7 +161,7 @@ __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_
     const bool valid = i < K.N;
     float4 ri = make_float4(0.f, 0.f, 0.f, 0.f);
     if (valid) ri = pos[i];
-    int cnt = 0;
+    int cnt = 0, all = 0;
     float4 nxt = pos[min((int)threadIdx.x, K.N - 1)];
     for (int t0 = 0; t0 < K.N; t0 += ADJ_BT) {
         float4 bc, bh;
@@ -182,21 +184,25 @@ __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_
             const float4 rj = tile[c0 + lane];
             float dx, dy, dz;
             const float d2 = dist_sq_mic(ri.x, ri.y, ri.z, rj.x, rj.y, rj.z, K.L0, K.L1, K.L2, dx, dy, dz);
-            unsigned long long m =
-                __ballot((d2 < r2) & (HALF ? niii_owns(i, t0 + c0 + lane, K.N) : true));
+            unsigned long long m = __ballot(d2 < r2);
             if (tn - c0 < 64) m &= (1ull << (tn - c0)) - 1ull;
             const unsigned self = (unsigned)(i - t0 - c0);   // the particle's own lane of these 64
             if (self < 64u) m &= ~(1ull << self);
+            if (HALF) {
+                all += __popcll(m);
+                m &= __ballot(niii_owns(i, t0 + c0 + lane, K.N));
+            }
             const int slot = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                              __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
             if (__builtin_amdgcn_inverse_ballot_w64(m) && slot < maxnb) nbl[(size_t)i * maxnb + slot] = t0 + c0 + lane;
             cnt += __popcll(m);
         }
     }
+    if (!HALF) all = cnt;
     if (valid && lane == 0) {
         nbc_p[i] = cnt;
         if (rref_p) rref_p[i] = ri;
-        if (cnt > maxnb) atomicMax(over, cnt);
+        if (all > maxnb) atomicMax(over, all);
     }
 }
 

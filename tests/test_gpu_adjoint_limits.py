@@ -1,0 +1,29 @@
+"""What the differentiable trajectory refuses and what it falls back to."""
+import numpy as np
+import pytest
+
+from gamdpy_amd import _native
+from gamdpy_amd.adjoint import AdjointEngine
+
+pytestmark = pytest.mark.gpu
+
+
+def _engine(N, L, nsteps=1, **kw):
+    kw = dict(dict(ckpt_every=5, rdf_every=5, bins=20, rmax=3.0, width=0.02), **kw)
+    return AdjointEngine(N, 1, [L] * 3, 0.0, nsteps, np.zeros(N, np.int32), np.ones(N, np.float32), **kw)
+
+
+LJ = np.array([[[1.0, 1.0, 1.7]]], np.float32)
+
+
+def test_frame_lists_too_long_for_the_gradient_are_refused_by_the_forward_pass():
+    """A droplet: 146 neighbours a particle, room for twice the mean of a
+    homogeneous system and 64 more (here 96).  Half of them would fit."""
+    n, L = 7, 40.0
+    r = np.stack(np.meshgrid(*[np.arange(n) * 0.95 - 0.95 * (n - 1) / 2] * 3, indexing="ij"), -1).reshape(-1, 3)
+    d = np.linalg.norm(r[:, None] - r[None], axis=-1)
+    longest = int((d < 3.0 + 5 * 0.02).sum(1).max()) - 1
+    assert 96 < longest < 192 and int((d < 2.2).sum(1).max()) - 1 <= 64   # (the step's own lists fit)
+    eng = _engine(len(r), L)
+    with pytest.raises(_native.NativeError, match=f"frame list of {longest} entries"):
+        eng.forward(LJ, r, np.zeros_like(r))
