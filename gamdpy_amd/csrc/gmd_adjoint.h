@@ -684,6 +684,42 @@ static float adj_weight_scale(double pairs) {
     return up;
 }
 
+// The storage the backward pass reads the positions from.  A trajectory of up
+// to ADJ_TRAJ_BYTES stays in memory as the forward pass writes it: one buffer
+// of step after step, nothing copied and no step computed twice (N = 4096, 200
+// steps: 13 MB, and the backward pass 200 forward steps and ten list builds
+// shorter).  A longer one, one the device has no room for beside everything
+// else, or any one where the caller asks for it, keeps a checkpoint of
+// positions and velocities every ckpt_every steps and recomputes a segment at
+// a time.
+#define ADJ_TRAJ_BYTES ((size_t)4 << 30)
+static hipError_t adj_storage(gmd_adj *a, bool whole) {
+    auto release = [a]() {
+        for (float4 **p : {&a->traj, &a->pos, &a->pos2, &a->ck_r, &a->ck_v, &a->seg}) {
+            if (*p) hipFree(*p);
+            *p = nullptr;
+        }
+    };
+    auto get = [](float4 **p, size_t n) {
+        const hipError_t e = hipMalloc((void **)p, n * sizeof(float4));
+        if (e != hipSuccess) {
+            *p = nullptr;
+            (void)hipGetLastError();
+        }
+        return e;
+    };
+    release();
+    a->have_forward = false;
+    const size_t N = a->d.N;
+    if (whole && get(&a->traj, ((size_t)a->d.nsteps + 1) * N) == hipSuccess) return hipSuccess;
+    hipError_t e = get(&a->pos, N);
+    if (e == hipSuccess) e = get(&a->pos2, N);
+    if (e == hipSuccess) e = get(&a->ck_r, (size_t)a->nck * N);
+    if (e == hipSuccess) e = get(&a->ck_v, (size_t)a->nck * N);
+    if (e == hipSuccess) e = get(&a->seg, (size_t)(a->d.ckpt_every + 1) * N);
+    return e;
+}
+
 // pair constants from (sigma, epsilon, cut) per ordered type pair
 static int adj_set_params(gmd_adj *a, const float *params) {
     const int nt = a->d.ntypes;
@@ -726,39 +762,21 @@ static int adj_set_params(gmd_adj *a, const float *params) {
         if (a->nbl) hipFree(a->nbl);
         a->nbl = nullptr;
         a->nbl_cap = 0;
-        if (hipMalloc((void **)&a->nbl, need * sizeof(int)) != hipSuccess) return fail("gmd_adj: list allocation");
+        hipError_t e = hipMalloc((void **)&a->nbl, need * sizeof(int));
+        if (e != hipSuccess && a->traj) {
+            // the lists come first: the trajectory makes room
+            (void)hipGetLastError();
+            e = adj_storage(a, false);
+            if (e == hipSuccess) e = hipMalloc((void **)&a->nbl, need * sizeof(int));
+        }
+        if (e != hipSuccess) {
+            a->nbl = nullptr;
+            return fail("gmd_adj: list allocation");
+        }
         a->nbl_cap = need;
     }
     a->K.maxnb = maxnb;
     return 0;
-}
-
-// The storage the backward pass reads the positions from.  A trajectory of up
-// to ADJ_TRAJ_BYTES stays in memory as the forward pass writes it: one buffer
-// of step after step, nothing copied and no step computed twice (N = 4096, 200
-// steps: 13 MB, and the backward pass 200 forward steps and ten list builds
-// shorter).  A longer one, or one the device has no room for, keeps a
-// checkpoint of positions and velocities every ckpt_every steps and recomputes
-// a segment at a time.
-#define ADJ_TRAJ_BYTES ((size_t)4 << 30)
-static hipError_t adj_storage(gmd_adj *a, bool whole) {
-    for (float4 **p : {&a->traj, &a->pos, &a->pos2, &a->ck_r, &a->ck_v, &a->seg}) {
-        if (*p) hipFree(*p);
-        *p = nullptr;
-    }
-    a->have_forward = false;
-    const size_t N = a->d.N, F = sizeof(float4);
-    if (whole) {
-        if (hipMalloc((void **)&a->traj, ((size_t)a->d.nsteps + 1) * N * F) == hipSuccess) return hipSuccess;
-        a->traj = nullptr;
-        (void)hipGetLastError();
-    }
-    hipError_t e = hipMalloc((void **)&a->pos, N * F);
-    if (e == hipSuccess) e = hipMalloc((void **)&a->pos2, N * F);
-    if (e == hipSuccess) e = hipMalloc((void **)&a->ck_r, (size_t)a->nck * N * F);
-    if (e == hipSuccess) e = hipMalloc((void **)&a->ck_v, (size_t)a->nck * N * F);
-    if (e == hipSuccess) e = hipMalloc((void **)&a->seg, (size_t)(a->d.ckpt_every + 1) * N * F);
-    return e;
 }
 
 extern "C" {
@@ -847,7 +865,6 @@ int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass
     ATRY(hipMalloc((void **)&a->rref, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->nbc, N * sizeof(int)));
     ATRY(hipMalloc((void **)&a->flag, 5 * sizeof(int)));   // skin flags of three steps, list overflows
-    ATRY(adj_storage(a, ((size_t)d.nsteps + 1) * N * sizeof(float4) <= ADJ_TRAJ_BYTES));
     ATRY(hipMalloc((void **)&a->lr, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->lv, N * sizeof(float4)));
     ATRY(hipMalloc((void **)&a->w, N * sizeof(float4)));
@@ -857,6 +874,7 @@ int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass
     ATRY(hipMalloc((void **)&a->H, (size_t)ncls * d.rdf_bins * sizeof(double)));
     ATRY(hipMalloc((void **)&a->hacc, (size_t)a->gl * ncls * d.rdf_bins * sizeof(double)));
     ATRY(hipMalloc((void **)&a->G, (size_t)ncls * d.rdf_bins * sizeof(float)));
+    ATRY(adj_storage(a, ((size_t)d.nsteps + 1) * N * sizeof(float4) <= ADJ_TRAJ_BYTES));   // (what is left for it)
 #undef ATRY
     *out = a;
     return 0;

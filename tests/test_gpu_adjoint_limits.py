@@ -1,6 +1,7 @@
 """What the differentiable trajectory refuses and what it falls back to."""
 import numpy as np
 import pytest
+import torch
 
 from gamdpy_amd import _native
 from gamdpy_amd.adjoint import AdjointEngine
@@ -27,3 +28,24 @@ def test_frame_lists_too_long_for_the_gradient_are_refused_by_the_forward_pass()
     eng = _engine(len(r), L)
     with pytest.raises(_native.NativeError, match=f"frame list of {longest} entries"):
         eng.forward(LJ, r, np.zeros_like(r))
+
+
+def test_a_trajectory_that_leaves_no_room_for_the_rest_is_not_kept():
+    """Device memory for everything but 50 MB of: a trajectory of 963 MB, lists
+    of 77 MB, histograms of 75 MB and 23 MB of vectors.  The checkpoints (170 MB)
+    fit."""
+    room = (963 + 175 - 50) << 20
+    held = []
+    for share in (0.9, 1.0, 1.0):
+        extra = int(share * (torch.cuda.mem_get_info()[0] - room)) >> 21 << 21
+        if extra > 0:
+            held.append(torch.empty(extra, dtype=torch.uint8, device="cuda"))
+    free = torch.cuda.mem_get_info()[0]
+    if not abs(free - room) < (20 << 20):
+        pytest.skip(f"{free >> 20} MB of device memory free instead of {room >> 20}")
+    try:
+        eng = _engine(200_000, 55.0, nsteps=300, ckpt_every=20, rmax=1.0, bins=3000)
+        eng.close()
+    finally:
+        del held
+        torch.cuda.empty_cache()
