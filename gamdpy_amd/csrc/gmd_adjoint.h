@@ -691,7 +691,7 @@ static float adj_weight_scale(double pairs) {
 // shorter).  A longer one, one the device has no room for beside everything
 // else, or any one where the caller asks for it, keeps a checkpoint of
 // positions and velocities every ckpt_every steps and recomputes a segment at
-// a time.
+// a time.  On an error the handle is left without storage.
 #define ADJ_TRAJ_BYTES ((size_t)4 << 30)
 static hipError_t adj_storage(gmd_adj *a, bool whole) {
     auto release = [a]() {
@@ -717,6 +717,7 @@ static hipError_t adj_storage(gmd_adj *a, bool whole) {
     if (e == hipSuccess) e = get(&a->ck_r, (size_t)a->nck * N);
     if (e == hipSuccess) e = get(&a->ck_v, (size_t)a->nck * N);
     if (e == hipSuccess) e = get(&a->seg, (size_t)(a->d.ckpt_every + 1) * N);
+    if (e != hipSuccess) release();
     return e;
 }
 
@@ -885,8 +886,11 @@ int gmd_adj_destroy(gmd_adj *a) { return adj_free(a); }
 int gmd_adj_use_checkpoints(gmd_adj *a) {
     if (!a) return fail("gmd_adj_use_checkpoints: null handle");
     HIPCHECK(hipStreamSynchronize(a->stream));
-    HIPCHECK(adj_storage(a, false));
-    return 0;
+    const bool whole = a->traj != nullptr;
+    const hipError_t e = adj_storage(a, false);
+    if (e == hipSuccess) return 0;
+    if (whole) (void)adj_storage(a, true);   // as it was
+    return fail("gmd_adj_use_checkpoints: %s", hipGetErrorString(e));
 }
 
 // blocks of a list build: ADJ_BT / 64 particles each
@@ -947,6 +951,7 @@ int gmd_adj_forward(gmd_adj *a, const float *params, const float *r0, const floa
     // pass that fails leaves nothing to differentiate
     a->have_forward = false;
     if (adj_set_params(a, params)) return -1;
+    if (!a->traj && !a->seg) return fail("gmd_adj_forward: no memory for the trajectory or its checkpoints");
     const int N = a->d.N, S = a->d.nsteps, C = a->d.ckpt_every, E = a->d.rdf_every;
     std::vector<float4> hr(N), hv(N);
     for (int i = 0; i < N; ++i) {

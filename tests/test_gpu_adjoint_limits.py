@@ -49,3 +49,23 @@ def test_a_trajectory_that_leaves_no_room_for_the_rest_is_not_kept():
     finally:
         del held
         torch.cuda.empty_cache()
+
+
+def test_checkpoints_without_room_leave_the_handle_as_it_was():
+    """A segment of 10^8 steps has no room: an error, and the trajectory is kept
+    on."""
+    rng = np.random.default_rng(3)
+    r = np.stack(np.meshgrid(*[np.arange(12) * 1.1 - 6.6] * 3, indexing="ij"), -1).reshape(-1, 3)
+    r = (r + rng.uniform(-0.05, 0.05, r.shape)).astype(np.float32)
+    N, far = len(r), 10 ** 8
+    eng = _engine(N, 13.2, nsteps=10, ckpt_every=far)
+    ref = _engine(N, 13.2, nsteps=10, ckpt_every=100)
+    want = ref.forward(LJ, r, 0 * r)
+    np.testing.assert_array_equal(eng.forward(LJ, r, 0 * r), want)
+    with pytest.raises(_native.NativeError, match="memory"):
+        _native.check(eng.lib.gmd_adj_use_checkpoints(eng.h), "gmd_adj_use_checkpoints")
+    with pytest.raises(_native.NativeError, match="no forward pass"):   # dropped, as the call says
+        eng.backward(want)
+    np.testing.assert_array_equal(eng.forward(LJ, r, 0 * r), want)
+    for a, b in zip(eng.backward(want), ref.backward(want)):
+        np.testing.assert_array_equal(a, b)
