@@ -4,8 +4,8 @@ respect to the LJ parameters and the initial positions.
 The forward pass is a float32 NVE trajectory (leap-frog as integrators/NVE.py)
 of an LJ_12_6_sigma_epsilon system with the shifted-force cutoff at a fixed
 cut; the backward pass is the hand-written adjoint in libgamdpy_amd.so
-(force Jacobian-vector products, parameter gradients, recomputation from
-checkpoints every ``ckpt_every`` steps).  The observable is the
+(force Jacobian-vector products and parameter gradients at the positions of
+every step, kept in memory or recomputed from checkpoints).  The observable is the
 trajectory-summed, Gaussian-smoothed pair histogram per type class; ``rdf``
 turns it into partial g(r).
 
@@ -38,7 +38,7 @@ class AdjointEngine:
     """Owns one gmd_adj: a trajectory of fixed length, types and masses."""
 
     def __init__(self, N, ntypes, box, dt, nsteps, ptype, mass, ckpt_every=20, rdf_every=10, bins=200,
-                 rmax=4.0, width=0.02):
+                 rmax=4.0, width=0.02, keep_trajectory=True):
         self.lib = _native.load()
         d = GmdAdjDesc()
         d.N, d.ntypes = int(N), int(ntypes)
@@ -54,6 +54,8 @@ class AdjointEngine:
         _native.check(self.lib.gmd_adj_create(ctypes.byref(d), _native.iptr(self.ptype), _native.fptr(self.mass),
                                               ctypes.byref(h)), "gmd_adj_create")
         self.h = h
+        if not keep_trajectory:
+            _native.check(self.lib.gmd_adj_use_checkpoints(self.h), "gmd_adj_use_checkpoints")
         self.nframes = len(range(0, int(nsteps) + 1, int(rdf_every)))
         self.passes = 0   # forward passes begun: the library keeps the last one's trajectory only
 
@@ -160,10 +162,17 @@ class DifferentiableNVE:
     sigma and epsilon are symmetric (ntypes, ntypes) torch tensors; the cut
     matrix is fixed.  ``rdf`` returns g[c, k] for the type classes
     ``type_classes(ntypes)`` at bin centres ``self.r``.
+
+    The positions of every step stay in device memory between the passes, 16
+    (nsteps + 1) N bytes, where that is at most 4 GiB and there is room for
+    it.  Otherwise, or with ``keep_trajectory=False``, a checkpoint every
+    ``ckpt_every`` steps does, and the backward pass repeats the steps between
+    them: the same results with 16 (2 nsteps / ckpt_every + ckpt_every) N
+    bytes, for the time of another forward pass.
     """
 
     def __init__(self, configuration, dt, nsteps, cut, ckpt_every=20, rdf_every=10, bins=200, rmax=4.0,
-                 width=0.02):
+                 width=0.02, keep_trajectory=True):
         conf = configuration
         self.N = conf.N
         self.ntypes = int(np.max(conf.ptype)) + 1
@@ -171,7 +180,8 @@ class DifferentiableNVE:
         self.cut = np.asarray(cut, np.float32) * np.ones((self.ntypes, self.ntypes), np.float32)
         self.v0 = np.ascontiguousarray(conf['v'], dtype=np.float32)
         self.engine = AdjointEngine(conf.N, self.ntypes, self.box, dt, nsteps, conf.ptype, conf['m'],
-                                    ckpt_every=ckpt_every, rdf_every=rdf_every, bins=bins, rmax=rmax, width=width)
+                                    ckpt_every=ckpt_every, rdf_every=rdf_every, bins=bins, rmax=rmax, width=width,
+                                    keep_trajectory=keep_trajectory)
         self.bins, self.rmax, self.width = bins, rmax, width
         self.dr = rmax / bins
         self.r = (np.arange(bins) + 0.5) * self.dr

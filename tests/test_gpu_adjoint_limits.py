@@ -51,9 +51,35 @@ def test_a_trajectory_that_leaves_no_room_for_the_rest_is_not_kept():
         torch.cuda.empty_cache()
 
 
+def test_checkpoints_by_choice():
+    """keep_trajectory=False: the checkpoints' memory, the same bits."""
+    n, nsteps = 27, 2000
+    L = n * 1.1
+    rng = np.random.default_rng(2)
+    r = np.stack(np.meshgrid(*[np.arange(n) * 1.1 - L / 2 + 0.5] * 3, indexing="ij"), -1).reshape(-1, 3)
+    r = (r + rng.uniform(-0.05, 0.05, r.shape)).astype(np.float32)
+    v = rng.normal(0.0, 0.5, r.shape).astype(np.float32)
+    used = []
+    for keep in (True, False):
+        before = torch.cuda.mem_get_info()[0]
+        eng = _engine(n ** 3, L, nsteps=nsteps, ckpt_every=50, keep_trajectory=keep)
+        used.append(before - torch.cuda.mem_get_info()[0])
+        eng.close()
+    assert used[0] - used[1] > 16 * (nsteps - 200) * n ** 3   # (checkpoints: 131 steps' worth)
+    got = []
+    for keep in (True, False):
+        eng = AdjointEngine(n ** 3, 1, [L] * 3, 0.004, 12, np.zeros(n ** 3, np.int32), np.ones(n ** 3, np.float32),
+                            ckpt_every=5, rdf_every=4, bins=20, rmax=2.0, width=0.05, keep_trajectory=keep)
+        H = eng.forward(LJ, r, v)
+        got.append((H,) + eng.backward(H))
+        eng.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_checkpoints_without_room_leave_the_handle_as_it_was():
     """A segment of 10^8 steps has no room: an error, and the trajectory is kept
-    on."""
+    on; a handle that never had room for either refuses to be made."""
     rng = np.random.default_rng(3)
     r = np.stack(np.meshgrid(*[np.arange(12) * 1.1 - 6.6] * 3, indexing="ij"), -1).reshape(-1, 3)
     r = (r + rng.uniform(-0.05, 0.05, r.shape)).astype(np.float32)
@@ -69,3 +95,5 @@ def test_checkpoints_without_room_leave_the_handle_as_it_was():
     np.testing.assert_array_equal(eng.forward(LJ, r, 0 * r), want)
     for a, b in zip(eng.backward(want), ref.backward(want)):
         np.testing.assert_array_equal(a, b)
+    with pytest.raises(_native.NativeError, match="memory"):
+        _engine(N, 13.2, nsteps=10, ckpt_every=far, keep_trajectory=False)
