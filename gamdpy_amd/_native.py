@@ -291,8 +291,7 @@ class Context:
         self.N = d.N
         self.nscalars = d.nscalars
         self.max_nbs = d.max_nbs
-        self._all_columns = sum(k >= 0 for k in (d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq,
-                                                 d.sid_m)) == d.nscalars
+        self._all_columns = {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq, d.sid_m} >= set(range(d.nscalars))
         self.saves_per_block = d.scalar_saves_per_block
         self.conf_saves_per_block = d.conf_saves_per_block
 

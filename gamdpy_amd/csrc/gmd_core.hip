@@ -1478,9 +1478,6 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
         HTRY(hipHostMalloc((void **)&c->pinned, (pub_words + c->xcap) * 4, hipHostMallocDefault));
         c->pub = (Ctrl *)c->pinned;
         c->xhost = c->pinned + pub_words;
-        int used = 0;
-        for (int sid : {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq, d.sid_m}) used += sid >= 0;
-        c->all_cols = used == d.nscalars;
     }
 
     // ---- device parameter block ----
@@ -1602,13 +1599,22 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
     P.xdev = (GMEM int *)c->xdev;
     P.xhost = c->xhost;
     P.pub = c->pinned;
-    P.nscal = d.nscalars;
-    P.sid_u = d.sid_u;
-    P.sid_w = d.sid_w;
-    P.sid_lap = d.sid_lap;
-    P.sid_k = d.sid_k;
-    P.sid_fsq = d.sid_fsq;
-    P.sid_m = d.sid_m;
+    // the scalar columns: a column outside the host's rows is absent (the
+    // packing kernels index the rows with it), and two quantities may share one
+    P.nscal = std::max(0, d.nscalars);
+    std::vector<char> covered(P.nscal, 0);
+    auto column = [&](int sid) {
+        if (sid < 0 || sid >= P.nscal) return -1;
+        covered[sid] = 1;
+        return sid;
+    };
+    P.sid_u = column(d.sid_u);
+    P.sid_w = column(d.sid_w);
+    P.sid_lap = column(d.sid_lap);
+    P.sid_k = column(d.sid_k);
+    P.sid_fsq = column(d.sid_fsq);
+    P.sid_m = column(d.sid_m);
+    c->all_cols = std::count(covered.begin(), covered.end(), (char)1) == P.nscal;
 
     HTRY(hipMemcpy(c->d_P, &P, sizeof(DP), hipMemcpyHostToDevice));
     c->kern = pick_kernels(d.pair_base, d.cutoff, d.integrator, d.nblist_kind);
@@ -1774,7 +1780,7 @@ int gmd_download(gmd_ctx *c, float *r, float *v, float *f, float *scalars, int *
         }
     }
     if (!rows.empty())
-        for (int sid : {d.sid_u, d.sid_w, d.sid_lap, d.sid_k, d.sid_fsq, d.sid_m})
+        for (int sid : {c->P.sid_u, c->P.sid_w, c->P.sid_lap, c->P.sid_k, c->P.sid_fsq, c->P.sid_m})
             if (sid >= 0)
                 for (size_t i = 0; i < N; ++i) scalars[i * ns + sid] = rows[i * ns + sid];
     return 0;
