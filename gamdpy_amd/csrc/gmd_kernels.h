@@ -146,8 +146,9 @@ __device__ __forceinline__ int cell_mod(double f, int n) {
 
 // floor(((x + L/2) n) / L) mod n without the division (three float64 divides
 // took a fifth of a rebuild's integrations, 28600 -> 22400 cycles a wavefront
-// at KA N = 65536): the quotient from the float32 inverse iL is off by at most
-// one (n < 2^20), and the sign of the remainder, one exact fma, says which way
+// at KA N = 65536): with iL the inverse of L to an ulp or two, the quotient is
+// off by at most one up to 2^21 cells, and the sign of the remainder, one exact
+// fma, says which way
 __device__ __forceinline__ int cell_dim(float x, double L, float iL, int n) {
     const double a = ((double)x + 0.5 * L) * (double)n;
     double q = floor(a * (double)iL);
@@ -489,7 +490,8 @@ __device__ __forceinline__ void particle_finish(const DP &P, const StepInfo &I, 
         if (P.nblist_kind == 1) {
             // (the context's box read here, not held from above: fewer live registers)
             if (INTEG == 4)
-                cell_insert(P, I.cbuf_next, i, rx, ry, rz, Ln0, Ln1, Ln2, I.iL0, I.iL1, I.iL2);
+                cell_insert(P, I.cbuf_next, i, rx, ry, rz, Ln0, Ln1, Ln2, __builtin_amdgcn_rcpf(Ln0),
+                            __builtin_amdgcn_rcpf(Ln1), __builtin_amdgcn_rcpf(Ln2));
             else
                 cell_insert(P, I.cbuf_next, i, rx, ry, rz, P.box0, P.box1, P.box2, P.ibox0, P.ibox1, P.ibox2);
         }
