@@ -1486,7 +1486,7 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
                 float dx, dy, dz;
                 const float d2 = dist_sq_mic(rj.x, rj.y, rj.z, rq.x, rq.y, rq.z, L0, L1, L2, dx, dy, dz);
                 const PairP &q = ppi[__float_as_int(rj.w)];
-                if (d2 >= q.cut2) return;
+                if (!(d2 < q.cut2)) return;   // (a cut that is not a number has no pairs)
                 if (niii)
                     pair_accum_w<BASE, CUT>(d2, dx, dy, dz, q, ax, ay, az, au, aw, al, lap,
                                             niii_owns(iq, t0 + e, N) ? 2.0f : 0.0f);
