@@ -62,6 +62,7 @@ struct AdjK {
     float skin2q;                // (skin / 2)^2
     int maxnb;                   // list slots per particle (row-major [i][slot])
     int tp, tpsh;                // lanes per particle of the list sums
+    int boxes;                   // the builds of those lists test chunks by their boxes first (adj_boxes)
     AdjPairC pc[ADJ_MAX_TYPES * ADJ_MAX_TYPES];
     // observable
     int bins;
@@ -145,14 +146,17 @@ __device__ __forceinline__ bool box_near(const AdjK &K, const float4 r, const fl
 // gradient needs longer lists than there is room for is refused by the forward
 // pass already).  The tests are most of the work, so a tile comes with the boxes of
 // its chunks of 64 positions (a wavefront each) and a particle tests only the
-// chunks whose box is near it: positions numbered along a lattice stay
-// together, and a numbering without order costs the boxes and gains nothing.
-// The particle itself and the slots past the last are taken out of the
-// wavefront's mask, not tested per lane.
+// chunks whose box is near it, where the numbering keeps chunks together
+// (boxes; adj_boxes).  Without, a chunk that has no neighbour is one test and
+// a branch.  The particle itself and the slots past the last are taken out of
+// the wavefront's mask, not tested per lane.  when (if given): build only if
+// that flag is set.
 #define ADJ_BT 1024   // threads of a build block, positions of its tile
 template <bool HALF>
 __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_p, float4 *rref_p, int *nbl_p,
-                                                      int *nbc_p, int maxnb, float r2, int *over) {
+                                                      int *nbc_p, int maxnb, float r2, int boxes, const int *when,
+                                                      int *over) {
+    if (when && *when == 0) return;
     __shared__ float4 tile[ADJ_BT], box_c[ADJ_BT / 64], box_h[ADJ_BT / 64];
     cpos_t pos = (cpos_t)pos_p;
     GMEM int *nbl = (GMEM int *)nbl_p;
@@ -165,10 +169,10 @@ __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_
     float4 nxt = pos[min((int)threadIdx.x, K.N - 1)];
     for (int t0 = 0; t0 < K.N; t0 += ADJ_BT) {
         float4 bc, bh;
-        wave_box(nxt, bc, bh);   // (a slot past the last holds the last position)
+        if (boxes) wave_box(nxt, bc, bh);   // (a slot past the last holds the last position)
         if (t0 > 0) __syncthreads();
         tile[threadIdx.x] = nxt;
-        if (lane == 0) {
+        if (boxes && lane == 0) {
             box_c[wid] = bc;
             box_h[wid] = bh;
         }
@@ -176,18 +180,19 @@ __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_
         if (t0 + ADJ_BT < K.N) nxt = pos[min(t0 + ADJ_BT + (int)threadIdx.x, K.N - 1)];
         if (!valid) continue;
         const int tn = min(ADJ_BT, K.N - t0);
-        unsigned long long live =
-            __ballot(lane < (tn + 63) / 64 && box_near(K, ri, box_c[lane & 15], box_h[lane & 15], r2));
-        while (live) {
-            const int c0 = 64 * __builtin_ctzll(live);
-            live &= live - 1;
+        // PLAIN: 64 positions, none of them the particle's own
+        auto chunk = [&](const int c0, auto whole) {
+            constexpr bool PLAIN = decltype(whole)::value;
             const float4 rj = tile[c0 + lane];
             float dx, dy, dz;
             const float d2 = dist_sq_mic(ri.x, ri.y, ri.z, rj.x, rj.y, rj.z, K.L0, K.L1, K.L2, dx, dy, dz);
             unsigned long long m = __ballot(d2 < r2);
-            if (tn - c0 < 64) m &= (1ull << (tn - c0)) - 1ull;
-            const unsigned self = (unsigned)(i - t0 - c0);   // the particle's own lane of these 64
-            if (self < 64u) m &= ~(1ull << self);
+            if (!PLAIN) {
+                if (tn - c0 < 64) m &= (1ull << (tn - c0)) - 1ull;
+                const unsigned self = (unsigned)(i - t0 - c0);   // the particle's own lane of these 64
+                if (self < 64u) m &= ~(1ull << self);
+            }
+            if (m == 0ull) return;
             if (HALF) {
                 all += __popcll(m);
                 m &= __ballot(niii_owns(i, t0 + c0 + lane, K.N));
@@ -196,6 +201,19 @@ __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_
                                                              __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
             if (__builtin_amdgcn_inverse_ballot_w64(m) && slot < maxnb) nbl[(size_t)i * maxnb + slot] = t0 + c0 + lane;
             cnt += __popcll(m);
+        };
+        if (boxes) {
+            unsigned long long live =
+                __ballot(lane < (tn + 63) / 64 && box_near(K, ri, box_c[lane & 15], box_h[lane & 15], r2));
+            while (live) {
+                chunk(64 * __builtin_ctzll(live), std::integral_constant<bool, false>{});
+                live &= live - 1;
+            }
+        } else if (tn == ADJ_BT && (unsigned)(i - t0) >= (unsigned)ADJ_BT) {
+#pragma unroll 4
+            for (int c0 = 0; c0 < ADJ_BT; c0 += 64) chunk(c0, std::integral_constant<bool, true>{});
+        } else {
+            for (int c0 = 0; c0 < tn; c0 += 64) chunk(c0, std::integral_constant<bool, false>{});
         }
     }
     if (!HALF) all = cnt;
@@ -207,9 +225,13 @@ __global__ void __launch_bounds__(ADJ_BT) k_adj_build(AdjK K, const float4 *pos_
 }
 
 // The same list for the particles of one block of a step kernel (256 threads,
-// 256 / tp particles), rebuilt in place when the skin check asked for it:
-// rare enough (a list lasts some ten steps) that the block's few wavefronts
-// may take longer than k_adj_build would.
+// 256 / tp particles), rebuilt in place when the skin check asked for it: rare
+// enough (a list lasts some ten steps) that the block's few wavefronts may take
+// longer than k_adj_build would, as long as the build is short.  From
+// ADJ_APART_N particles on the launch of its own before every step costs less.
+// Forward + backward, in place and apart, 40 steps: in lattice order N = 4000
+// (100 steps) 2362 and 2510 us, 8000 1604 and 1560, 16384 3406 and 3060; in no
+// order 4000 2691 and 2899, 8000 2060 and 2064, 16384 5532 and 4550.
 __device__ __forceinline__ void adj_relist(const AdjK &K, cpos_t pos, GMEM float4 *rref, GMEM int *nbl, GMEM int *nbc,
                                         GMEM int *over) {
     __shared__ float4 tile[256], own[64], box_c[4], box_h[4];
@@ -223,10 +245,10 @@ __device__ __forceinline__ void adj_relist(const AdjK &K, cpos_t pos, GMEM float
     float4 nxt = pos[min((int)threadIdx.x, K.N - 1)];
     for (int t0 = 0; t0 < K.N; t0 += 256) {
         float4 bc, bh;
-        wave_box(nxt, bc, bh);
+        if (K.boxes) wave_box(nxt, bc, bh);
         __syncthreads();
         tile[threadIdx.x] = nxt;
-        if (lane == 0) {
+        if (K.boxes && lane == 0) {
             box_c[wid] = bc;
             box_h[wid] = bh;
         }
@@ -238,11 +260,7 @@ __device__ __forceinline__ void adj_relist(const AdjK &K, cpos_t pos, GMEM float
             if (i >= K.N) break;
             const float4 ri = own[p];
             int cnt = count[p];
-            unsigned long long live =
-                __ballot(lane < (tn + 63) / 64 && box_near(K, ri, box_c[lane & 3], box_h[lane & 3], K.cps2));
-            while (live) {
-                const int c0 = 64 * __builtin_ctzll(live);
-                live &= live - 1;
+            auto chunk = [&](const int c0) {
                 const float4 rj = tile[c0 + lane];
                 float dx, dy, dz;
                 const float d2 = dist_sq_mic(ri.x, ri.y, ri.z, rj.x, rj.y, rj.z, K.L0, K.L1, K.L2, dx, dy, dz);
@@ -255,6 +273,16 @@ __device__ __forceinline__ void adj_relist(const AdjK &K, cpos_t pos, GMEM float
                 if (__builtin_amdgcn_inverse_ballot_w64(m) && slot < K.maxnb)
                     nbl[(size_t)i * K.maxnb + slot] = t0 + c0 + lane;
                 cnt += __popcll(m);
+            };
+            if (K.boxes) {
+                unsigned long long live =
+                    __ballot(lane < (tn + 63) / 64 && box_near(K, ri, box_c[lane & 3], box_h[lane & 3], K.cps2));
+                while (live) {
+                    chunk(64 * __builtin_ctzll(live));
+                    live &= live - 1;
+                }
+            } else {
+                for (int c0 = 0; c0 < tn; c0 += 64) chunk(c0);
             }
             if (lane == 0) count[p] = cnt;
         }
@@ -285,6 +313,7 @@ struct AdjLists {
     int b, built;
 };
 
+#define ADJ_APART_N 8000
 #define ADJ_UNR 4   // list entries a lane gathers at a time
 
 // The pairs of particle i (lane t of its tp) in list order: ADJ_UNR entries,
@@ -638,6 +667,8 @@ struct gmd_adj {
     int nck = 0;
     int gl = 0;                  // blocks of the list sums
     int rmaxnb = 0;              // slots per particle of the frame list
+    int fboxes = 0;              // K.boxes for the frame lists
+    bool apart = false;          // list builds between checkpoints in launches of their own (ADJ_APART_N)
     int chk = 0;                 // steps of a pass so far (the turn of the skin flags)
     size_t nbl_cap = 0;          // allocated list slots
     hipStream_t stream = nullptr;
@@ -719,6 +750,33 @@ static hipError_t adj_storage(gmd_adj *a, bool whole) {
     if (e == hipSuccess) e = get(&a->seg, (size_t)(a->d.ckpt_every + 1) * N);
     if (e != hipSuccess) release();
     return e;
+}
+
+// Whether the builds of lists of this radius test a chunk's box before its 64
+// positions: a question of the caller's numbering.  The share of chunks whose
+// box is near a particle is estimated from 16 of the start's chunks; the boxes
+// pay where it is below about 0.3.  Ordered along a lattice, rho = 1.2, 40
+// steps, forward + backward without and with boxes: N = 2000 (0.47) 814 and
+// 838 us, 4000 (0.30; 100 steps) 2340 and 2362, 8000 (0.16) 1687 and 1560,
+// 65536 (0.05) 38.7 and 25.5 ms.  In no order (1.0), where every box is tested
+// for nothing: 8000 2064 and 2523 us, 65536 42.9 and 71.1 ms.
+static int adj_boxes(const gmd_adj *a, const float *r, float radius) {
+    const int N = a->d.N, chunks = (N + 63) / 64, n = std::min(16, chunks);
+    double near = 0.0;
+    for (int k = 0; k < n; ++k) {
+        const int b = (int)((long long)k * chunks / n) * 64, e = std::min(N, b + 64);
+        double share = 1.0;
+        for (int c = 0; c < 3; ++c) {
+            float lo = r[3 * (size_t)b + c], hi = lo;
+            for (int i = b + 1; i < e; ++i) {
+                lo = std::min(lo, r[3 * (size_t)i + c]);
+                hi = std::max(hi, r[3 * (size_t)i + c]);
+            }
+            share *= std::min(1.0, (double)(hi - lo + 2.0f * radius) / a->d.box[c]);
+        }
+        near += share / n;
+    }
+    return near < 0.3 ? 1 : 0;
 }
 
 // pair constants from (sigma, epsilon, cut) per ordered type pair
@@ -847,6 +905,7 @@ int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass
     }
     K.hup = adj_weight_scale((double)(256 / K.tp) * a->rmaxnb);
     a->nck = (d.nsteps + d.ckpt_every - 1) / d.ckpt_every;
+    a->apart = d.N >= ADJ_APART_N;
     const size_t N = d.N;
 #define ATRY(x)                                                               \
     do {                                                                      \
@@ -899,7 +958,7 @@ static dim3 adj_build_grid(const gmd_adj *a) { return dim3((a->K.N + ADJ_BT / 64
 // the smoothed histogram of the frame at pos (its half list: each pair once)
 static void adj_rdf_frame(gmd_adj *a, const float4 *pos) {
     hipLaunchKernelGGL(k_adj_build<true>, adj_build_grid(a), dim3(ADJ_BT), 0, a->stream, a->K, pos,
-                       (float4 *)nullptr, a->rnbl, a->rnbc, a->rmaxnb, a->K.rcut2, a->flag + 4);
+                       (float4 *)nullptr, a->rnbl, a->rnbc, a->rmaxnb, a->K.rcut2, a->fboxes, (const int *)nullptr, a->flag + 4);
     hipLaunchKernelGGL(k_adj_rdf_list, dim3(a->gl), dim3(256), 0, a->stream, a->K, pos, (const int *)a->rnbl,
                        (const int *)a->rnbc, a->rmaxnb, a->hacc);
 }
@@ -907,7 +966,7 @@ static void adj_rdf_frame(gmd_adj *a, const float4 *pos) {
 // dL/dr of the frame at pos into a->rpart
 static void adj_rdf_grad(gmd_adj *a, const float4 *pos) {
     hipLaunchKernelGGL(k_adj_build<false>, adj_build_grid(a), dim3(ADJ_BT), 0, a->stream, a->K, pos,
-                       (float4 *)nullptr, a->rnbl, a->rnbc, a->rmaxnb, a->K.rcut2, a->flag + 4);
+                       (float4 *)nullptr, a->rnbl, a->rnbc, a->rmaxnb, a->K.rcut2, a->fboxes, (const int *)nullptr, a->flag + 4);
     hipLaunchKernelGGL(k_adj_rdf_grad_list, dim3(a->gl), dim3(256), 0, a->stream, a->K, pos, (const float *)a->G,
                        (const int *)a->rnbl, (const int *)a->rnbc, a->rmaxnb, a->rpart);
 }
@@ -916,10 +975,13 @@ static void adj_rdf_grad(gmd_adj *a, const float4 *pos) {
 // the step needs them afresh (a checkpoint), else by the step itself where
 // the last step's skin check asks for it
 static AdjLists adj_lists(gmd_adj *a, const float4 *pos, bool build) {
-    if (build)
+    const int b = a->chk++ % 3;
+    const bool apart = build || a->apart;
+    if (apart)
         hipLaunchKernelGGL(k_adj_build<false>, adj_build_grid(a), dim3(ADJ_BT), 0, a->stream, a->K, pos, a->rref,
-                           a->nbl, a->nbc, a->K.maxnb, a->K.cps2, a->flag + 3);
-    return AdjLists{a->nbl, a->nbc, a->flag, a->flag + 3, a->rref, a->chk++ % 3, build ? 1 : 0};
+                           a->nbl, a->nbc, a->K.maxnb, a->K.cps2, a->K.boxes,
+                           (const int *)(build ? nullptr : a->flag + b), a->flag + 3);
+    return AdjLists{a->nbl, a->nbc, a->flag, a->flag + 3, a->rref, b, apart ? 1 : 0};
 }
 
 static int adj_reset_lists(gmd_adj *a) {
@@ -953,6 +1015,8 @@ int gmd_adj_forward(gmd_adj *a, const float *params, const float *r0, const floa
     if (adj_set_params(a, params)) return -1;
     if (!a->traj && !a->seg) return fail("gmd_adj_forward: no memory for the trajectory or its checkpoints");
     const int N = a->d.N, S = a->d.nsteps, C = a->d.ckpt_every, E = a->d.rdf_every;
+    a->K.boxes = adj_boxes(a, r0, std::sqrt(a->K.cps2));
+    a->fboxes = adj_boxes(a, r0, std::sqrt(a->K.rcut2));
     std::vector<float4> hr(N), hv(N);
     for (int i = 0; i < N; ++i) {
         int t = a->ptype[i];
