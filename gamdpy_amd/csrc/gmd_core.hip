@@ -1627,6 +1627,11 @@ static int ctx_create(const gmd_desc *desc, gmd_ctx **out, hipStream_t shared_st
             ctx_free(c);
             return fail("gridsync: persistent kernel cannot be resident with %d threads per block", block);
         }
+        // at most eight wavefronts a CU: what the barrier after every step costs
+        // grows with its blocks, and a third block a CU hides less than that
+        // (NVE, linked lists, tp = 8, two and three blocks a CU: N = 20000 58 and
+        // 70 us a step, N = 60000 74 and 101)
+        nb = std::min(nb, std::max(1, 512 / block));
         c->grid_pers = std::max(1, std::min(c->grid_step, nb * c->cus));
     }
     *out = c;
