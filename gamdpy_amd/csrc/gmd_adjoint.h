@@ -761,22 +761,7 @@ static hipError_t adj_storage(gmd_adj *a, bool whole) {
 // 65536 (0.05) 38.7 and 25.5 ms.  In no order (1.0), where every box is tested
 // for nothing: 8000 2064 and 2523 us, 65536 42.9 and 71.1 ms.
 static int adj_boxes(const gmd_adj *a, const float *r, float radius) {
-    const int N = a->d.N, chunks = (N + 63) / 64, n = std::min(16, chunks);
-    double near = 0.0;
-    for (int k = 0; k < n; ++k) {
-        const int b = (int)((long long)k * chunks / n) * 64, e = std::min(N, b + 64);
-        double share = 1.0;
-        for (int c = 0; c < 3; ++c) {
-            float lo = r[3 * (size_t)b + c], hi = lo;
-            for (int i = b + 1; i < e; ++i) {
-                lo = std::min(lo, r[3 * (size_t)i + c]);
-                hi = std::max(hi, r[3 * (size_t)i + c]);
-            }
-            share *= std::min(1.0, (double)(hi - lo + 2.0f * radius) / a->d.box[c]);
-        }
-        near += share / n;
-    }
-    return near < 0.3 ? 1 : 0;
+    return chunk_share(r, a->d.N, a->d.box, 2.0f * radius, 16) < 0.3 ? 1 : 0;
 }
 
 // pair constants from (sigma, epsilon, cut) per ordered type pair

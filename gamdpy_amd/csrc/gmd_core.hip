@@ -2296,15 +2296,49 @@ static size_t rdf_lds_bytes(int nt, int bins) {
     return ((nh * 4 + 15) & ~(size_t)15) + (((size_t)(bins + 1) * 4 + 15) & ~(size_t)15);
 }
 
+// Mean share of the box that 64 consecutive positions and 'pad' around them
+// span, of n runs spread over the numbering
+static double chunk_share(const float *r, int N, const float box[3], float pad, int n) {
+    const int chunks = (N + 63) / 64;
+    n = std::min(n, chunks);
+    double sum = 0.0;
+    for (int k = 0; k < n; ++k) {
+        const int b = (int)((long long)k * chunks / n) * 64, e = std::min(N, b + 64);
+        float lo[3], hi[3];
+        for (int c = 0; c < 3; ++c) lo[c] = hi[c] = r[3 * (size_t)b + c];
+        for (int i = b + 1; i < e; ++i)   // six independent chains
+            for (int c = 0; c < 3; ++c) {
+                lo[c] = std::min(lo[c], r[3 * (size_t)i + c]);
+                hi[c] = std::max(hi[c], r[3 * (size_t)i + c]);
+            }
+        double share = 1.0;
+        for (int c = 0; c < 3; ++c) share *= std::min(1.0, (double)(hi[c] - lo[c] + pad) / box[c]);
+        sum += share;
+    }
+    return sum / n;
+}
+
+// Whether the numbering keeps particles together without a sort, asked where
+// rdf_cells does (in lattice order a run of 64 spans some hundredths of the
+// box, in no order 0.9 of it)
+static bool rdf_in_order(const float *r, int N, const float box[3]) {
+    return N >= 8192 && N < 65536 && chunk_share(r, N, box, 0.f, 8) < 0.25;
+}
+
 // Sorting cells per dimension: some 16 particles a cell; 1 (none) where the
-// sort's three launches (20 us with their gaps) are what it saves: N = 8000 in
-// random order 165 us a call sorted, 164 not; N = 20000 351 against 394.
-static int rdf_cells(int N) { return N < 8192 ? 1 : N < 32768 ? 8 : N < 262144 ? 16 : RDF_MAX_CELL; }
+// sort's three launches (20 us with their gaps) are what it saves or more.
+// In no order, without and with the sort: N = 8000 106 and 109 us, 12000 143
+// and 139, 16000 191 and 180, 30000 453 and 383; in lattice order 8000 101 and
+// 111, 16000 168 and 182, 30000 374 and 388, 131072 4630 and 4590.
+static int rdf_cells(int N, bool in_order) {
+    if (N < 8192 || (in_order && N < 65536)) return 1;
+    return N < 32768 ? 8 : N < 262144 ? 16 : RDF_MAX_CELL;
+}
 
 // The launches of one histogram on a stream: sort, boxes, counts, sum over
 // blocks.  S.pos (or S.r) / S.ptype: the input; out and the cell counts are
 // zero; grid: blocks of k_rdf, at most what R.part holds.
-static int rdf_kernels(RdfP R, RdfSort S, const float box[3], int grid, float4 *gbox, float4 *cbox,
+static int rdf_kernels(RdfP R, RdfSort S, const float box[3], int grid, bool in_order, float4 *gbox, float4 *cbox,
                        unsigned long long *out, hipStream_t st) {
     const int N = R.N;
     R.L0 = box[0];
@@ -2333,7 +2367,7 @@ static int rdf_kernels(RdfP R, RdfSort S, const float box[3], int grid, float4 *
     S.N = N;
     S.npad = R.nchunks * RDF_CHUNK;
     S.nt_bytes = R.bins * 4;
-    S.ncell = rdf_cells(N);
+    S.ncell = rdf_cells(N, in_order);
     const unsigned nb = (unsigned)((N + 255) / 256);
     if (S.ncell > 1) {
         hipLaunchKernelGGL(k_rdf_count, dim3(nb), dim3(256), 0, st, S);
@@ -2377,7 +2411,7 @@ int gmd_rdf_create(int N, int ntypes, int bins, gmd_rdf **out) {
     // beside the step kernels, 2 blocks per CU take fewer of their slots and
     // still finish within a block of steps
     r->grid_bg = (int)std::max(1LL, std::min(npairs, std::max((long long)cus * 2, need)));
-    const size_t ng = (size_t)r->nchunks * (RDF_CHUNK / RDF_GROUP), cells = rdf_cells(N);
+    const size_t ng = (size_t)r->nchunks * (RDF_CHUNK / RDF_GROUP), cells = rdf_cells(N, false);
     if (hipMalloc(&r->pos, (size_t)N * sizeof(float4)) != hipSuccess ||
         hipMalloc(&r->sorted, (size_t)r->nchunks * RDF_CHUNK * sizeof(float4)) != hipSuccess ||
         hipMalloc(&r->cbox, (size_t)4 * r->nchunks * sizeof(float4)) != hipSuccess ||
@@ -2421,14 +2455,15 @@ int gmd_rdf_destroy(gmd_rdf *r) {
 
 // Enqueue one histogram on the calculator's stream (pos: positions with types,
 // or null: the host's in r->pos; d_ptype: their types, with pos instead of its
-// own), ending in an asynchronous copy of the counts to pinned host memory.
-static int rdf_launch(gmd_rdf *r, const float4 *pos, const int *d_ptype, const float box[3], int grid) {
+// own; in_order: they need no sort), ending in an asynchronous copy of the
+// counts to pinned host memory.
+static int rdf_launch(gmd_rdf *r, const float4 *pos, const int *d_ptype, const float box[3], int grid, bool in_order) {
     if (box[0] != r->box[0] || box[1] != r->box[1] || box[2] != r->box[2] || r->thr.empty()) {
         rdf_thresholds(box, r->bins, r->thr);
         HIPCHECK(hipMemcpy(r->d_thr, r->thr.data(), (size_t)(r->bins + 1) * sizeof(float), hipMemcpyHostToDevice));
         memcpy(r->box, box, sizeof r->box);
     }
-    const size_t nh = rdf_hist_size(r->nt, r->bins), cells = rdf_cells(r->N);
+    const size_t nh = rdf_hist_size(r->nt, r->bins), cells = rdf_cells(r->N, false);
     RdfP R = {};
     R.N = r->N;
     R.nt = r->nt;
@@ -2445,7 +2480,7 @@ static int rdf_launch(gmd_rdf *r, const float4 *pos, const int *d_ptype, const f
     S.out = r->sorted;
     HIPCHECK(hipMemsetAsync(r->d_out, 0, nh * sizeof(unsigned long long) + cells * cells * cells * sizeof(int),
                             r->stream));
-    if (rdf_kernels(R, S, box, grid, r->gbox, r->cbox, r->d_out, r->stream)) return -1;
+    if (rdf_kernels(R, S, box, grid, in_order, r->gbox, r->cbox, r->d_out, r->stream)) return -1;
     HIPCHECK(hipMemcpyAsync(r->h_out, r->d_out, nh * sizeof(unsigned long long), hipMemcpyDeviceToHost, r->stream));
     HIPCHECK(hipEventRecord(r->done, r->stream));
     r->pending = true;
@@ -2493,7 +2528,7 @@ static int rdf_launch_ctx(gmd_rdf *r, gmd_ctx *c, const int *ptype, int grid) {
                             hipMemcpyDeviceToDevice, c->stream));
     HIPCHECK(hipEventRecord(r->snap, c->stream));
     HIPCHECK(hipStreamWaitEvent(r->stream, r->snap, 0));
-    return rdf_launch(r, r->pos, dp, c->cur_box, grid);
+    return rdf_launch(r, r->pos, dp, c->cur_box, grid, c->permuted);   // (renumbered: in cell order)
 }
 
 int gmd_rdf_launch_ctx(gmd_rdf *r, gmd_ctx *c, const int *ptype) {
@@ -2518,18 +2553,19 @@ int gmd_rdf_compute_host(gmd_rdf *r, const float *pos, const int *ptype, const f
     for (int i = 0; i < r->N; ++i)
         if (ptype[i] < 0 || ptype[i] >= r->nt) return fail("gmd_rdf_compute_host: type out of range");
     if (r->pending) return fail("gmd_rdf_compute_host: a launched update is not collected");
+    const bool in_order = rdf_in_order(pos, r->N, box);
     if (r->N <= RDF_ONE_COPY) {
         const size_t N = r->N;
         r->h_in.resize(4 * N);
         memcpy(r->h_in.data(), pos, 3 * N * sizeof(float));
         memcpy(r->h_in.data() + 3 * N, ptype, N * sizeof(int));
         HIPCHECK(hipMemcpy(r->pos, r->h_in.data(), 4 * N * sizeof(int), hipMemcpyHostToDevice));
-        if (rdf_launch(r, nullptr, (const int *)r->pos + 3 * N, box, r->grid)) return -1;
+        if (rdf_launch(r, nullptr, (const int *)r->pos + 3 * N, box, r->grid, in_order)) return -1;
         return rdf_collect(r, counts);
     }
     HIPCHECK(hipMemcpy(r->pos, pos, (size_t)r->N * 3 * sizeof(float), hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(r->ptype, ptype, (size_t)r->N * sizeof(int), hipMemcpyHostToDevice));
-    if (rdf_launch(r, nullptr, r->ptype, box, r->grid)) return -1;
+    if (rdf_launch(r, nullptr, r->ptype, box, r->grid, in_order)) return -1;
     return rdf_collect(r, counts);
 }
 
@@ -2606,10 +2642,10 @@ int gmd_rdf_compute_host_noalloc(int N, int ntypes, int bins, const float *pos, 
     const long long nc = (N + RDF_CHUNK - 1) / RDF_CHUNK;
     const int grid = (int)std::min(nc * (nc + 1) / 2, (long long)NOALLOC_RDF_GRID);
     hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, st, d_out, (int)nh);
-    const int cells = rdf_cells(N) * rdf_cells(N) * rdf_cells(N);
+    const int cells = rdf_cells(N, false) * rdf_cells(N, false) * rdf_cells(N, false);
     hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)(((cells + 1) / 2 + 255) / 256)), dim3(256), 0, st,
                        (unsigned long long *)S.count, (cells + 1) / 2);
-    if (rdf_kernels(R, S, box, grid, (float4 *)(base + NOALLOC_OFF_GBOX), (float4 *)(base + NOALLOC_OFF_CBOX), d_out,
+    if (rdf_kernels(R, S, box, grid, rdf_in_order(pos, N, box), (float4 *)(base + NOALLOC_OFF_GBOX), (float4 *)(base + NOALLOC_OFF_CBOX), d_out,
                     st))
         return -1;
     HIPCHECK(hipMemcpy(raw, d_out, nh * sizeof(unsigned long long), hipMemcpyDeviceToHost));
