@@ -1304,14 +1304,15 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
 }
 
 // ---------------------------------------------------------------------------
-// Rebuild step, N squared (nblist.py:89-143): NSQ_PP particles per wavefront
-// at a time.  The block stages tiles of blockDim.x positions in LDS (two
-// buffers, the next tile's load in flight during the current one: one block
-// barrier a tile).  A wavefront reads 64 positions of the tile once and tests
-// them against its particles, compacting each particle's accepted tile slots
-// with a ballot; then every particle's 16 lanes write its list entries
-// (ascending j) and add its pair terms, the particles side by side.  The
-// first lane of each group integrates its particle.
+// Rebuild step, N squared (nblist.py:89-143): PP particles per wavefront at a
+// time, four or one (step_nsq_rebuild).  The block stages tiles of blockDim.x
+// positions in LDS (two buffers, the next tile's load in flight during the
+// current one: one block barrier a tile).  A wavefront reads 64 positions of
+// the tile once and tests them against its particles, compacting each
+// particle's accepted tile slots with a ballot; then every particle's 64 / PP
+// lanes write its list entries (ascending j) and add its pair terms, the
+// particles side by side.  The first lane of each group integrates its
+// particle.
 //
 // The kernel is bound by the latency of each wavefront's chain (tile read,
 // test, ballot, compaction): a system that takes the N-squared list leaves a
@@ -1325,20 +1326,21 @@ __device__ __forceinline__ void step_ll_rebuild(const DP &P, const BlockCtx &B, 
 //
 // The sums keep the order of a wavefront that gives each accepted pair of a
 // tile the lane of its rank mod 64 and adds the lanes pairwise (32, 16, ...,
-// 1 apart): rank 16 k + l of a particle is added to its sum k in lane l of
-// its group, and sums 0 + 2 and 1 + 3 are those two levels.
+// 1 apart), for every PP: rank 16 k + l of one of four particles is added to
+// its sum k in lane l of its group, and sums 0 + 2 and 1 + 3 are those two
+// levels.
 // ---------------------------------------------------------------------------
-#define NSQ_PP 4                 // particles a wavefront takes at a time (16 lanes each in the pair pass)
+#define NSQ_PP 4                 // particles a wavefront takes at a time, at most
 #define NSQ_CAP 256              // accepted slots of one particle and tile (a tile holds at most 256 positions)
 
-template <int BASE, int CUT, int INTEG>
-__device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B, const StepInfo &I, const PairP *pp,
-                                                 float4 *tiles, float acc[GMD_NRED]) {
+template <int BASE, int CUT, int INTEG, int PP>
+__device__ __forceinline__ void nsq_rebuild(const DP &P, const BlockCtx &B, const StepInfo &I, const PairP *pp,
+                                            float4 *tiles, const int rounds, float acc[GMD_NRED]) {
+    static_assert(PP == 4 || PP == 1, "lanes of a group: 16 or 64");
+    constexpr int LPP = 64 / PP;   // lanes of a particle
     const int bd = blockDim.x;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, wpb = bd >> 6;
-    const int g = lane >> 4, l16 = lane & 15;
-    const int per_round = B.nb * wpb;
-    const int rounds = (P.N + per_round - 1) / per_round;
+    const int g = lane / LPP, lp = lane & (LPP - 1);
     const float L0 = INTEG == 4 ? I.L0 : P.box0, L1 = INTEG == 4 ? I.L1 : P.box1, L2 = INTEG == 4 ? I.L2 : P.box2;
     cpos_t pos = I.cur ? P.pos1 : P.pos0;
     const bool lap = P.compute_lap != 0;
@@ -1359,9 +1361,9 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
     const float hmin = 0.5f * fminf(L0, fminf(L1, L2));
     const bool near = I.wrapped && cps2 < 0.9999f * (hmin * hmin);
     // this wave's accepted tile slots, NSQ_CAP a particle
-    unsigned short *accs = (unsigned short *)(tiles + 2 * bd) + wid * (NSQ_PP * NSQ_CAP);
-    for (int rd = 0; rd < rounds; rd += NSQ_PP) {
-        // particle k of the wavefront: round rd + k, held by lanes 16k .. 16k + 15
+    unsigned short *accs = (unsigned short *)(tiles + 2 * bd) + wid * (PP * NSQ_CAP);
+    for (int rd = 0; rd < rounds; rd += PP) {
+        // particle k of the wavefront: round rd + k, held by lanes LPP k and on
         const int iq = ((rd + g) * B.nb + B.bid) * wpb + wid;
         const bool mine = iq < N && rd + g < rounds;
         float4 rq = make_float4(0.f, 0.f, 0.f, 0.f), vq = make_float4(0.f, 0.f, 0.f, 1.f);
@@ -1369,29 +1371,31 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
             rq = pos[iq];
             vq = P.vel[iq];
         }
-        int ik[NSQ_PP], cnt[NSQ_PP], nhalf[NSQ_PP];
-        float xk[NSQ_PP], yk[NSQ_PP], zk[NSQ_PP];
+        int ik[PP], cnt[PP], nhalf[PP];
+        float xk[PP], yk[PP], zk[PP];
 #pragma unroll
-        for (int k = 0; k < NSQ_PP; ++k) {
+        for (int k = 0; k < PP; ++k) {
             // a round past the last, or an index past N, takes no pair
-            ik[k] = lane_i(mine ? iq : -1, 16 * k);
-            xk[k] = lane_f(rq.x, 16 * k);
-            yk[k] = lane_f(rq.y, 16 * k);
-            zk[k] = lane_f(rq.z, 16 * k);
+            ik[k] = lane_i(mine ? iq : -1, LPP * k);
+            xk[k] = lane_f(rq.x, LPP * k);
+            yk[k] = lane_f(rq.y, LPP * k);
+            zk[k] = lane_f(rq.z, LPP * k);
             cnt[k] = 0;
             nhalf[k] = 0;
         }
         const PairP *ppi = pp + __float_as_int(rq.w) * P.ntypes;
-        float fx[4], fy[4], fz[4], uu[4], ww[4], ll[4];
+        float fx[PP], fy[PP], fz[PP], uu[PP], ww[PP], ll[PP];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) fx[u] = fy[u] = fz[u] = uu[u] = ww[u] = ll[u] = 0.f;
+        for (int u = 0; u < PP; ++u) fx[u] = fy[u] = fz[u] = uu[u] = ww[u] = ll[u] = 0.f;
         auto rotate = [&]() {
-            auto turn1 = [](float (&v)[4]) {
-                const float t = v[0];
-                v[0] = v[1];
-                v[1] = v[2];
-                v[2] = v[3];
-                v[3] = t;
+            auto turn1 = [](float (&v)[PP]) {
+                if constexpr (PP == 4) {
+                    const float t = v[0];
+                    v[0] = v[1];
+                    v[1] = v[2];
+                    v[2] = v[3];
+                    v[3] = t;
+                }
             };
             turn1(fx);
             turn1(fy);
@@ -1399,6 +1403,13 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
             turn1(uu);
             turn1(ww);
             turn1(ll);
+        };
+        // the value of the lane's own particle
+        auto own = [&](const int (&v)[PP]) {
+            if constexpr (PP == 4)
+                return g == 0 ? v[0] : g == 1 ? v[1] : g == 2 ? v[2] : v[3];
+            else
+                return v[0];
         };
         int buf = 0;
         float4 nxt = pos[min((int)threadIdx.x, N - 1)];
@@ -1413,10 +1424,10 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
             // the list test of 64 positions against each particle.  PLAIN: a
             // full tile that holds none of the particles themselves, no
             // exclusions, no half lists
-            int nacc[NSQ_PP];
+            int nacc[PP];
             bool plain = tn == bd && !has_excl && !niii;
 #pragma unroll
-            for (int k = 0; k < NSQ_PP; ++k) {
+            for (int k = 0; k < PP; ++k) {
                 nacc[k] = 0;
                 plain = plain && ik[k] >= 0 && (unsigned)(ik[k] - t0) >= (unsigned)bd;
             }
@@ -1431,9 +1442,9 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
                     const int c0 = 64 * u, left = tn - c0;
                     // the distances of all the particles before the first
                     // compaction: independent chains
-                    float d2[NSQ_PP];
+                    float d2[PP];
 #pragma unroll
-                    for (int k = 0; k < NSQ_PP; ++k) {
+                    for (int k = 0; k < PP; ++k) {
                         float dx, dy, dz;
                         d2[k] = NEAR ? dist_sq_list(cj[u].x, cj[u].y, cj[u].z, xk[k], yk[k], zk[k], L0, L1, L2, iL0,
                                                     iL1, iL2, dx, dy, dz)
@@ -1441,7 +1452,7 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
                                                    dz);
                     }
 #pragma unroll
-                    for (int k = 0; k < NSQ_PP; ++k) {
+                    for (int k = 0; k < PP; ++k) {
                         bool ok = d2[k] < cps2;
                         unsigned long long mask = __ballot(ok);
                         if (!PLAIN) {
@@ -1471,11 +1482,11 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
             else
                 filter(std::integral_constant<bool, false>{}, std::integral_constant<bool, false>{});
             wave_sync_lds();
-            // the accepted pairs of the tile, each particle on its 16 lanes:
-            // list entries (slots cnt + rank, tile order) and pair terms
-            const int na = g == 0 ? nacc[0] : g == 1 ? nacc[1] : g == 2 ? nacc[2] : nacc[3];
-            const int c_q = g == 0 ? cnt[0] : g == 1 ? cnt[1] : g == 2 ? cnt[2] : cnt[3];
-            const int amax = max(max(nacc[0], nacc[1]), max(nacc[2], nacc[3]));
+            // the accepted pairs of the tile, each particle on its lanes: list
+            // entries (slots cnt + rank, tile order) and pair terms
+            const int na = own(nacc), c_q = own(cnt);
+            int amax = nacc[0];
+            if constexpr (PP == 4) amax = max(max(nacc[0], nacc[1]), max(nacc[2], nacc[3]));
             const unsigned short *mya = accs + g * NSQ_CAP;
             auto pair = [&](const int a, float &ax, float &ay, float &az, float &au, float &aw, float &al) {
                 if (a >= na) return;
@@ -1497,18 +1508,22 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
             // once: the families of the later bases are long)
             int turn = 0;
 #pragma unroll 1
-            for (int a0 = 0; a0 < amax; a0 += 16, ++turn) {
-                pair(a0 + l16, fx[0], fy[0], fz[0], uu[0], ww[0], ll[0]);
+            for (int a0 = 0; a0 < amax; a0 += LPP, ++turn) {
+                pair(a0 + lp, fx[0], fy[0], fz[0], uu[0], ww[0], ll[0]);
                 rotate();
             }
 #pragma unroll 1
-            for (; turn & 3; ++turn) rotate();
+            for (; turn & (PP - 1); ++turn) rotate();
 #pragma unroll
-            for (int k = 0; k < NSQ_PP; ++k) cnt[k] += nacc[k];
+            for (int k = 0; k < PP; ++k) cnt[k] += nacc[k];
             wave_sync_lds();   // accs is rewritten for the next tile
         }
-        auto total = [&](const float (&v)[4]) {
-            float t = (v[0] + v[2]) + (v[1] + v[3]);
+        auto total = [&](const float (&v)[PP]) {
+            float t;
+            if constexpr (PP == 4)
+                t = (v[0] + v[2]) + (v[1] + v[3]);
+            else
+                t = xor_sum<16>(xor_sum<32>(v[0]));
             t = xor_sum<8>(t);
             t = xor_sum<4>(t);
             t = xor_sum<2>(t);
@@ -1520,27 +1535,42 @@ __device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B,
 #pragma unroll
         for (int c = 0; c < GMD_NRED; ++c) part[c] = 0.f;
         if (mine) {
-            const int n = g == 0 ? cnt[0] : g == 1 ? cnt[1] : g == 2 ? cnt[2] : cnt[3];
-            const int nh = g == 0 ? nhalf[0] : g == 1 ? nhalf[1] : g == 2 ? nhalf[2] : nhalf[3];
-            if (l16 == 0) {
+            const int n = own(cnt), nh = own(nhalf);
+            if (lp == 0) {
                 P.nbc[iq] = n;
                 P.rref[iq] = rq;
                 list_overflow(P, n, nh);
             }
             if (P.boff) bond_terms(P, pos, iq, rq, L0, L1, L2, sx, sy, sz, su, sw, sl);
-            particle_finish<INTEG>(P, I, iq, rq, vq, rq, sx, sy, sz, su * 0.5f, sw * (0.5f / 3.0f), sl, l16 == 0,
+            particle_finish<INTEG>(P, I, iq, rq, vq, rq, sx, sy, sz, su * 0.5f, sw * (0.5f / 3.0f), sl, lp == 0,
                                    part);
-            if (I.ksplit && l16 == 0) P.kcell[iq] = part[RED_K];
+            if (I.ksplit && lp == 0) P.kcell[iq] = part[RED_K];
         }
         // the step's sums in lane 0, particle after particle
 #pragma unroll
-        for (int k = 0; k < NSQ_PP; ++k)
+        for (int k = 0; k < PP; ++k)
 #pragma unroll
             for (int c = 0; c < GMD_NRED; ++c) {
-                const float v = lane_f(part[c], 16 * k);
+                const float v = lane_f(part[c], LPP * k);
                 if (lane == 0) acc[c] += v;
             }
     }
+}
+
+// One particle at a time where a wavefront has no more than two, each with all
+// lanes: the other slots of the four would be tested for nothing, and a
+// particle's pairs take a quarter of the lanes.  Rebuild steps of LJ N = 2048
+// at tp = 64, 32 and 16 (one, two and four particles): four at a time 35, 36
+// and 32 us, one at a time 13, 19 and 49.
+template <int BASE, int CUT, int INTEG>
+__device__ __forceinline__ void step_nsq_rebuild(const DP &P, const BlockCtx &B, const StepInfo &I, const PairP *pp,
+                                                 float4 *tiles, float acc[GMD_NRED]) {
+    const int per_round = B.nb * (int)(blockDim.x >> 6);
+    const int rounds = (P.N + per_round - 1) / per_round;
+    if (rounds <= 2)
+        nsq_rebuild<BASE, CUT, INTEG, 1>(P, B, I, pp, tiles, rounds, acc);
+    else
+        nsq_rebuild<BASE, CUT, INTEG, NSQ_PP>(P, B, I, pp, tiles, rounds, acc);
 }
 
 // linked lists: clear the cell buffer that step s+2 will fill
