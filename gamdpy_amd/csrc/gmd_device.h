@@ -161,7 +161,10 @@ struct DP {
     int lds_pp, lds_red, lds_build;   // byte offsets into dynamic LDS
     int step_grid;             // blocks of the step kernel (partial sums to reduce)
     int rebuild_grid;          // replicas of a batch: blocks of a split rebuild step (step_once)
-    GMEM float *kcell;         // the kinetic energies of such a step: [ncells][ccap], or [N] for N-squared lists
+    // the kinetic energies of such a step, [ncells][ccap] or [N] for N-squared
+    // lists; null: a rebuild whose kinetic sum is wanted is not split (it is set
+    // where rebuild_grid exceeds step_grid and the integrator is NVT)
+    GMEM float *kcell;
     const GMEM int *perm;      // internal index -> index in the caller's order (particles are kept in cell order)
     // the host's arrays: a packed copy of them in device memory (xdev) and in
     // pinned host memory (xhost), the words of each array one after another

@@ -65,7 +65,8 @@ __device__ __forceinline__ void step_once(const DP &P, BlockCtx B, int k) {
     StepInfo I = step_info(P, s, INTEG, rebuild, true);
     unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);
     if (BATCH && rebuild) {
-        if (P.rebuild_grid > P.step_grid && (mask & ~(1u << RED_K)) == 0u) {
+        // split: a step that needs no sums, or the kinetic sum and has room for its parts
+        if (P.rebuild_grid > P.step_grid && (mask == 0u || (mask == (1u << RED_K) && P.kcell != nullptr))) {
             B.nb = P.rebuild_grid;
             I.ksplit = mask != 0u;
             mask = 0u;
