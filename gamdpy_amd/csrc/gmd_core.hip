@@ -760,11 +760,6 @@ __global__ void k_rdf_reduce(const unsigned *part_p, int nblocks, int nh, int pe
     if (s) atomicAdd(gen_ptr(out + x), s);
 }
 
-__global__ void k_pack_pos(const float *r, const int *ptype, int N, float4 *pos) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < N) pos[i] = make_float4(r[3 * i], r[3 * i + 1], r[3 * i + 2], __int_as_float(ptype[i]));
-}
-
 // ============================================================================
 // Renumbering of the particles in cell order (gather locality for the step,
 // rebuild and histogram kernels).  Deterministic: cells in index order,
@@ -1020,18 +1015,6 @@ Kernels pick_kernels(int base, int cut, int integ, int kind) {
            : base == 1 ? pick_cut<1>(cut, integ, kind)
            : base <= 5 ? pick_cut<2>(cut, integ, kind)
                        : pick_cut<3>(cut, integ, kind);
-}
-
-float i2f(int v) {
-    float f;
-    memcpy(&f, &v, 4);
-    return f;
-}
-
-int f2i(float v) {
-    int i;
-    memcpy(&i, &v, 4);
-    return i;
 }
 
 // One host array's place in the packed buffer: words [at, at + n)
