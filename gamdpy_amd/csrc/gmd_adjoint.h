@@ -1,7 +1,8 @@
-// gmd_adjoint.h -- differentiable NVE trajectory: float32 forward with
-// checkpoints, hand-written adjoint (force Jacobian-vector products and
-// gradients with respect to the per-type LJ sigma / epsilon), and a
-// Gaussian-smoothed partial radial distribution as the observable.
+// gmd_adjoint.h -- differentiable NVE trajectory: float32 forward whose
+// positions stay in memory (or checkpoints of them), hand-written adjoint
+// (force Jacobian-vector products and gradients with respect to the per-type
+// LJ sigma / epsilon), and a Gaussian-smoothed partial radial distribution as
+// the observable.
 //
 // Included once into gmd_core.hip (shares its error channel and helpers).
 //
@@ -23,23 +24,24 @@
 // A = s(r), B = (ds/dr)/r, d_ij = r_i - r_j (minimum image).
 //
 // The force and J w sums run over neighbour lists (radius max cut + skin, N
-// squared build, rebuilt when a particle has moved more than skin/2 and at
-// every checkpoint, so a segment recomputed from its checkpoint in the
-// backward pass repeats the forward bit for bit); the observable and its
+// squared build, rebuilt when a particle has moved more than skin/2 and every
+// ckpt_every steps, so a segment recomputed from its checkpoint repeats the
+// forward bit for bit and both layouts give the same bits); the observable and its
 // gradient run over a list of radius rmax + 5 w built afresh (no skin) at
 // each frame, one frame every rdf_every steps.
 //
 // A step of either pass is ONE kernel: the rebuild of the lists of a block's
-// own particles where the last step's skin check asks for it, the sums, the
-// update of the particle and the skin check of its next positions.  The
-// systems are small (a step of N = 4096 is some microseconds of work spread
-// over the device), so a step is bound by its launches and by the latency of
-// each lane's chain of list entry, neighbour and pair term; the separate
-// check, build, sum and update kernels of a step were three to four launches,
-// most of the builds finding nothing to do.With
-// them apart the forward and backward passes of KA N = 4096, 200 steps, took
-// 11.7 ms, now 7.5 (N = 500, 40 steps: 2.1 -> 1.2 ms); a forward step is
-// 5 us, a backward step 9, an inline rebuild 32 us more.
+// own particles where the last step's skin check asks for it (in a launch of
+// its own for large systems), the sums, the update of the particle and the skin
+// check of its next positions.  The systems are small (a step of N = 4096 is
+// some microseconds of work spread over the device), so a step is bound by its
+// launches and by the latency of each lane's chain of list entry, neighbour and
+// pair term; the separate check, build, sum and update kernels of a step were
+// three to four launches, most of the builds finding nothing to do.  Forward
+// and backward pass of KA N = 4096, 200 steps: 11.7 ms with them apart, 7.5
+// with one kernel a step, 5.9 with the trajectory kept (N = 500, 40 steps: 2.1,
+// 1.2 and 0.95 ms); a forward step is 5 us, a backward step 9, a rebuild inside
+// one 32 us more.
 #pragma once
 
 #define ADJ_MAX_TYPES 3

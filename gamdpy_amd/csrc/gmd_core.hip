@@ -40,7 +40,9 @@ __global__ void __launch_bounds__(256) k_batch_advance(const DP *__restrict__ Ps
 
 // The kinetic sums of the replicas whose step was a split rebuild (step_once),
 // in the grouping of an unsplit one, bit for bit: block b's wavefront w adds up
-// cell after cell (particle after particle) of those it would have taken.
+// cell after cell (particle after particle) of those it would have taken.  It
+// follows every step of a split NVT batch, whether some replica rebuilds or
+// not, and takes 7.6 us of a step of 216 (64 replicas, 3.5 %).
 __global__ void __launch_bounds__(256) k_batch_ksum(const DP *__restrict__ Ps, int k) {
     const DP &P = Ps[blockIdx.y];
     const int s = P.ctrl->s_base + k;

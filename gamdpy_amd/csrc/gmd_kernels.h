@@ -1631,10 +1631,6 @@ __device__ __forceinline__ void block_partials(const DP &P, const BlockCtx &B, f
     __syncthreads();
 }
 
-// Executed by the last block of a step: final sums over all blocks, then the
-// one-thread updates of the reference (NVT.py:226-237 thermostat,
-// momentum_reset.py:166-186 shift, scalar_saver.py:374-408 output row), the
-// rebuild decision of the next step and the step counter.
 // A thread's first four per-block partials (blocks t, t+256, t+512, t+768)
 // of the components in 'mask', loaded together: one memory round trip for a
 // grid of up to 1024 blocks.  CM: the components the caller may ask for (a
@@ -1737,6 +1733,10 @@ __device__ __forceinline__ void npt_publish(const DP &P, const StepInfo &J, int 
         C->npt_grid_bad = 1;
 }
 
+// The tail of a step of the persistent driver, executed by its last block:
+// final sums over all blocks, then the one-thread updates of the reference
+// (NVT.py:226-237 thermostat, momentum_reset.py:166-186 shift,
+// scalar_saver.py:374-408 output row; NPT_Atomic.py:148-187).
 __device__ inline void step_tail(const DP &P, const StepInfo &I, double *red, const int nblocks) {
     GMEM Ctrl *C = P.ctrl;
     const unsigned mask = red_mask(I.need_ksum, I.need_mom, I.need_save, I.need_wsum);

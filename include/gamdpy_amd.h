@@ -293,8 +293,10 @@ int gmd_batch_last_run_ms(gmd_batch *batch, float *ms);
  * the initial positions, for fitting potentials to structural data).
  * Model: LJ_12_6_sigma_epsilon with gamdpy's shifted-force cutoff
  * (apply_shifted_force_cutoff.py:29-37, s(r) - s(rc)) at a fixed cut;
- * NVE leap-frog (NVE.py:59-105); float32 forward, checkpoints every
- * ckpt_every steps, adjoint by recomputation from the checkpoints.
+ * NVE leap-frog (NVE.py:59-105); float32 forward.  The adjoint pass reads the
+ * positions of every step, which stay in device memory up to 4 GiB (16 bytes a
+ * particle and step) where there is room for them, or recomputes them from
+ * checkpoints every ckpt_every steps.
  * Observable: H[c][k] = sum over frames (every rdf_every steps, including 0
  * and, when it is a multiple, nsteps) and unordered pairs of class c of
  * max(0, exp(-(d - r_k)^2 / (2 w^2)) - exp(-12.5)) for |d - r_k| < 5 w,
@@ -311,16 +313,18 @@ typedef struct gmd_adj_desc {
 int gmd_adj_create(const gmd_adj_desc *desc, const int *ptype, const float *mass, gmd_adj **out);
 int gmd_adj_destroy(gmd_adj *adj);
 /* params: ntypes*ntypes*3 float32 (sigma, epsilon, cut), symmetric; r0, v0 (N,3);
- * H: nclass*bins float64; r_end, v_end (N,3) or NULL */
+ * H: nclass*bins float64; r_end, v_end (N,3) or NULL.  Replaces what the last
+ * forward pass left for gmd_adj_backward, also when it fails. */
 int gmd_adj_forward(gmd_adj *adj, const float *params, const float *r0, const float *v0, double *H, float *r_end,
                     float *v_end);
 /* dLdH: nclass*bins; grad_params: nclass*2 float64 (dL/dsigma, dL/depsilon per
  * class); grad_r0, grad_v0 (N,3) (grad_v0 may be NULL) */
 int gmd_adj_backward(gmd_adj *adj, const double *dLdH, double *grad_params, float *grad_r0, float *grad_v0);
 int gmd_adj_last_ms(gmd_adj *adj, float *fwd_ms, float *bwd_ms);
-/* keep checkpoints only, as a trajectory too long for device memory does, and
- * recompute between them in the backward pass (same results; a forward pass
- * before the call is dropped) */
+/* keep checkpoints only, as a trajectory of more than 4 GiB does, and recompute
+ * between them in the backward pass (same results; a forward pass before the
+ * call is dropped).  Where they find no memory: an error, and the handle keeps
+ * the trajectory. */
 int gmd_adj_use_checkpoints(gmd_adj *adj);
 
 #ifdef __cplusplus
