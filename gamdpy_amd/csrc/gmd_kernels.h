@@ -490,8 +490,8 @@ __device__ __forceinline__ void particle_finish(const DP &P, const StepInfo &I, 
         if (P.nblist_kind == 1) {
             // (the context's box read here, not held from above: fewer live registers)
             if (INTEG == 4)
-                cell_insert(P, I.cbuf_next, i, rx, ry, rz, Ln0, Ln1, Ln2, __builtin_amdgcn_rcpf(Ln0),
-                            __builtin_amdgcn_rcpf(Ln1), __builtin_amdgcn_rcpf(Ln2));
+                cell_insert(P, I.cbuf_next, i, rx, ry, rz, Ln0, Ln1, Ln2, uniform_f(__builtin_amdgcn_rcpf(Ln0)),
+                            uniform_f(__builtin_amdgcn_rcpf(Ln1)), uniform_f(__builtin_amdgcn_rcpf(Ln2)));
             else
                 cell_insert(P, I.cbuf_next, i, rx, ry, rz, P.box0, P.box1, P.box2, P.ibox0, P.ibox1, P.ibox2);
         }
