@@ -39,9 +39,10 @@
 // pair term; the separate check, build, sum and update kernels of a step were
 // three to four launches, most of the builds finding nothing to do.  Forward
 // and backward pass of KA N = 4096, 200 steps: 11.7 ms with them apart, 7.5
-// with one kernel a step, 5.9 with the trajectory kept (N = 500, 40 steps: 2.1,
-// 1.2 and 0.95 ms); a forward step is 5 us, a backward step 9, a rebuild inside
-// one 32 us more.
+// with one kernel a step, 5.9 with the trajectory kept, 5.65 with builds that
+// test boxes only where that saves something (N = 500, 40 steps: 2.1, 1.2, 0.95
+// and 0.96 ms); a forward step is 5.3 us, a backward step 9.3, a rebuild inside
+// one 31 us more.
 #pragma once
 
 #define ADJ_MAX_TYPES 3
